@@ -264,12 +264,12 @@ __device__ __forceinline__ void finish_column(const ImParams& P, int p, int t, i
   if (insert_slot) fl |= kPosInsert;
   if ((double)total <= P.targets[t].seed_cutoff) fl |= kPosSeed;
   // an uncertain consensus call goes to the exact scorer, which makes the call itself
-  const bool cand = cons || cons_unsure || (P.screen_off && A.n > 0) ||
-                    screen_passes(A, ref_idx, P.log10_ref_length, P.polymorphism_cutoff, P.screen_margin);
+  const bool sure = cons || cons_unsure || (P.screen_off && A.n > 0);
+  const bool cand = sure || screen_passes(A, ref_idx, P.log10_ref_length, P.polymorphism_cutoff, P.screen_margin);
   if (cand) {
     fl |= kPosCandidate;
     const int slot = atomicAdd(P.n_cand, 1);
-    if (slot < P.cand_cap) P.cand[slot] = make_int2(p, 0);
+    if (slot < P.cand_cap) P.cand[slot] = make_int2(p, sure ? 0 : kCandScreened);
     else err |= kErrCapacity;
   }
   if (insert_slot) {

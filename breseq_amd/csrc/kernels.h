@@ -108,24 +108,28 @@ struct ImParams {
   double mutation_cutoff;
   double polymorphism_cutoff;
   double precision_decimal;
+  int32_t places;               // digits of printed frequencies
   double screen_margin;
   int32_t screen_off;           // 1: every covered column goes to the exact scorer
   // per-column outputs
   uint8_t* col_flags;
   int32_t* col_unique;
   int32_t* col_total;
-  // candidates
-  int2* cand;                   // (global column, insert slot)
+  // candidates of the column pass: (global column, kCandScreened or 0)
+  int2* cand;
   int32_t* n_cand;
+  // candidates of the exact scorer: (global column, insert slot)
+  int2* score;
+  int32_t* n_score;
   int32_t* score_next;   // work counter of the exact scorer: the next candidate a block takes (zeroed per pass)
-  int32_t cand_cap;
+  int32_t cand_cap;             // capacity of cand and of score
   int32_t* ins;                 // columns with insert slots
   int32_t* n_ins;
   int32_t ins_cap;
   int32_t key_cap;              // capacity of a candidate's read list (the most reads of a window)
   int32_t keys_global;          // 1: read lists in key_scratch (key_cap per block), else in LDS
   uint32_t* key_scratch;        // device scratch of the read lists of deep samples
-  int32_t rows_cap;             // reads whose table rows the scorer caches in LDS
+  int32_t rows_cap;             // distinct table keys of a candidate whose rows the scorer holds in LDS
   RaOut* ra_out;
   // columns whose predicted / consensus decision the column pass could not certify
   int32_t* fix;
@@ -171,7 +175,13 @@ __global__ void k_identify_columns_t(ImParams P);
 __global__ void k_prep_reads(const DRead* reads, int64_t n, int32_t S, int32_t Q, IdRec* out);
 template <bool kKeysGlobal>
 __global__ void k_fix_columns_t(ImParams P);
-__global__ void k_insert_slots(ImParams P);
+// A column that only the column pass's bound could not rule out: k_route_candidates tests it again
+constexpr int32_t kCandScreened = 1;
+__global__ void k_route_candidates(ImParams P);
+__host__ __device__ inline size_t route_words(int tab_keys) { return (size_t)tab_keys + (size_t)(tab_keys + 1) / 2; }
+constexpr int kRouteWaves = 4;              // wavefronts per block of k_route_candidates, a candidate each
+constexpr int kRouteGrid = 2048;            // its blocks
+constexpr int kRouteKeys = 2048;            // most table keys a wavefront's LDS histogram holds (6 bytes each)
 // BAM2COV per-column counts over a region (coverage_output.cpp:307-503): lane = column, the window's
 // reads in file order.
 struct CovTabParams {
@@ -197,10 +207,14 @@ __global__ void k_coverage_columns(CovTabParams C);
 __global__ void k_coverage_rows(CovTabParams C);
 
 constexpr int kScoreWaves = 4;               // wavefronts per candidate in the exact scorer
-constexpr int kScoreGrid = 2048;             // blocks of the exact scorer (each draws candidates from a work counter)
+// blocks of the exact scorer (each draws candidates from a work counter): four per CU are resident
+constexpr int kScoreGrid = 1024;
 constexpr int kFixGrid = 256;                // blocks of k_fix_columns (at most kScoreGrid)
-constexpr size_t kScoreStaticLds = 28 * 1024;   // bound on the scorer's static LDS
-constexpr size_t kScoreLdsBudget = 52 * 1024;   // static + dynamic LDS of a scorer block: three per CU
+constexpr size_t kScoreStaticLds = 6656;   // bound on the scorer's static LDS
+constexpr size_t kScoreLdsBudget = 39 * 1024;   // static + dynamic LDS of a scorer block: four per CU
+constexpr size_t kScoreLdsDeep = 64 * 1024;     // the same for samples whose read lists need more
+constexpr size_t kScoreRowBytes = 120;          // dynamic LDS of a distinct key of the candidate
+constexpr size_t kScoreKeyLds = 32 * 1024;      // most LDS for a candidate's read list
 template <bool kKeysGlobal>
 __global__ void k_score_candidates_t(ImParams P);
 // reference and alignment trims (extra.hip)

@@ -1,6 +1,7 @@
 // kernels.hip -- CDNA4 (gfx950) kernels of pass 2 that follow the column kernel.
 //
-//  k_insert_slots     enumerates insert slots >= 1 of columns whose unique reads carry insertions
+//  k_route_candidates the exact scorer's candidates: insert slots >= 1 of columns whose unique reads
+//                     carry insertions, and the columns of the column pass that can be emitted
 //  k_runs             MC and UN interval detection (identify_mutations.cpp:2262-2344, 2972-3007)
 #include <hip/hip_runtime.h>
 
@@ -14,47 +15,277 @@ namespace bsq {
 __device__ __forceinline__ int uniform_i(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 /* ------------------------------------------------------------------------------------------ */
-/* Insert slots >= 1                                                                           */
+/* Candidates of the exact scorer                                                              */
 
-// One wavefront per column whose unique reads carry insertions enumerates the insert slots the
-// reference visits (identify_mutations.cpp:1359-1361, 1598-1599): slot 1 always, and slot s+1 while
+// Insert slots >= 1 of column p, whose unique reads carry insertions (one wavefront): the slots the
+// reference visits (identify_mutations.cpp:1359-1361, 1598-1599), slot 1 always, and slot s+1 while
 // some unique read with a longer insertion has a base other than N at slot s.  Lanes take the
 // window's alignments.  Every visited slot goes to the exact scorer, which makes the consensus and
 // polymorphism calls itself.
-__global__ void __launch_bounds__(64) k_insert_slots(ImParams P) {
-  const int n_ins = min(*P.n_ins, P.ins_cap);
-  const int lane = threadIdx.x;
+__device__ __forceinline__ void route_insert_slots(const ImParams& P, int p, int lane, uint32_t& err) {
+  const int64_t w = p / WAVE;
+  if (p < 0 || p >= P.n_pos || w >= P.n_windows) {
+    err |= kErrIndex;
+    return;
+  }
+  const int rb = P.win_rb[w], re = P.win_re[w];
+  if (rb < 0 || re < rb || re > P.n_reads) {
+    err |= kErrIndex;
+    return;
+  }
+  for (int slot = 1; slot < 65536; slot++) {
+    if (lane == 0) {
+      const int c = atomicAdd(P.n_score, 1);
+      if (c < P.cand_cap) P.score[c] = make_int2(p, slot);
+      else err |= kErrCapacity;
+    }
+    bool next = false;
+    for (int r0 = rb; r0 < re; r0 += WAVE) {
+      const int r = r0 + lane;
+      if (r >= re) continue;
+      const DRead R = P.reads[r];
+      if (R.x1 != 1) continue;
+      int qpos, indel;
+      bool is_del;
+      if (!entry_at(R, P.cigar, p, qpos, indel, is_del, err) || is_del || indel <= slot) continue;
+      if (P.bases[R.seq_off + qpos + slot] != 15) next = true;
+    }
+    if (!__any(next)) break;
+  }
+}
+
+template <int kCtrl>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffffLL), kCtrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), kCtrl, 0xf, 0xf, true);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+__device__ __forceinline__ double lane_d(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), l);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Sum over the wavefront: within each row of 16 lanes by DPP (lane ^ 1, ^ 2, ^ 7, ^ 15), then the
+// four rows' sums.  A sixth of the latency of six shuffles, which go through the LDS crossbar.
+__device__ __forceinline__ double wave_sum_d(double v) {
+  v = dpp_add<0xB1>(v);    // quad_perm [1,0,3,2]
+  v = dpp_add<0x4E>(v);    // quad_perm [2,3,0,1]
+  v = dpp_add<0x141>(v);   // row_half_mirror
+  v = dpp_add<0x140>(v);   // row_mirror
+  return (lane_d(v, 0) + lane_d(v, 16)) + (lane_d(v, 32) + lane_d(v, 48));
+}
+
+// Orders a wavefront's own LDS accesses (its lanes read what other lanes wrote).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// One EM pass over a column's distinct keys (lane = key, 64 at a time): S[b] = Sum_i r_i(b) / s_i,
+// s_i = Sum_b f_b r_i(b), and the log10 likelihood Sum_i log10 s_i (without the lpmax sum), each key
+// weighted with its reads.  The logarithms are FP32 (each within 2e-6 for s_i above 1e-30).  False
+// when a read has no likelihood to speak of.
+__device__ __forceinline__ bool key_pass(const ImParams& P, const uint16_t* keys, const uint32_t* hist, int K, int lane,
+                                         const double f[5], double S[5], double& ll) {
+  double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, l2 = 0.0;
+  bool bad = false;
+  for (int k0 = 0; k0 < K; k0 += WAVE) {
+    const int k = k0 + lane;
+    if (k >= K) continue;
+    const uint32_t key = keys[k];
+    const double h = (double)hist[key];
+    const double* t = P.tab_r + (size_t)key * 6;
+    double r[5], s = 0.0;
+#pragma unroll
+    for (int b = 0; b < 5; b++) {
+      r[b] = t[b];
+      s = fma(f[b], r[b], s);
+    }
+    bad = bad || !(s > 1e-30 && s < 1e30);
+    double y = __builtin_amdgcn_rcp(s);
+    y = fma(fma(-s, y, 1.0), y, y);
+    y = fma(fma(-s, y, 1.0), y, y) * h;
+#pragma unroll
+    for (int b = 0; b < 5; b++) acc[b] = fma(r[b], y, acc[b]);
+    l2 = fma(h, (double)log2f((float)s), l2);
+  }
+#pragma unroll
+  for (int b = 0; b < 5; b++) S[b] = wave_sum_d(acc[b]);
+  ll = wave_sum_d(l2) * 0.30102999566398119521;
+  return !__any(bad);
+}
+
+// Whether a column that only the column pass's bound let through can reach the presence-score cutoff
+// (identify_mutations.cpp:3240-3344): false only if no allele v can, from bounds on the two
+// likelihoods of its score that follow the reference's own EM loops a few passes (one wavefront).
+//   * Full fit: the likelihood is concave in the frequencies, so its maximum is at most
+//     LL(f) + (max_b Sum_i r_i(b) / s_i - n) / ln 10 at any f.  f: the EM iterates from the
+//     reference's starting point, the least bound of the first four.
+//   * Null fit of v: EM never lowers the likelihood, and the reference reports that of its last
+//     pass's frequencies, so any earlier iterate's likelihood is at most the reported one.  The k-th
+//     iterate is used only when every step before it moved a frequency by more than 2 tol, which makes
+//     the reference take that pass too.
+// The reads' likelihoods depend on their table keys alone, so the passes run over the distinct keys
+// with their counts.  The comparison keeps the margin of the column pass's screen, plus the
+// rounding of the FP32 logarithms (2e-6 a read and likelihood).
+__device__ __forceinline__ bool may_be_emitted(const ImParams& P, const uint16_t* keys, const uint32_t* hist, int K,
+                                               const uint32_t cnt[5], int ref_idx, int lane) {
+  double n = 0.0;
+#pragma unroll
+  for (int b = 0; b < 5; b++) n += (double)cnt[b];
+  const double need = P.polymorphism_cutoff - P.screen_margin - 4e-6 * n + P.log10_ref_length;
+  double upper = INFINITY;
+  {
+    double f[5], S[5], ll, total = 0.0;
+#pragma unroll
+    for (int b = 0; b < 5; b++) {
+      f[b] = 0.5 + (double)cnt[b];
+      total += f[b];
+    }
+#pragma unroll
+    for (int b = 0; b < 5; b++) f[b] /= total;
+    for (int it = 0; it < 4; it++) {
+      if (!key_pass(P, keys, hist, K, lane, f, S, ll)) return true;
+      double g = 0.0;
+#pragma unroll
+      for (int b = 0; b < 5; b++) {
+        g = fmax(g, S[b]);
+        f[b] = f[b] * S[b] / n;
+      }
+      const double gap = (g - n) * 0.43429448190325182765;
+      upper = fmin(upper, ll + fmax(gap, 0.0));
+      if (gap < 0.02) break;
+    }
+  }
+#pragma unroll 1
+  for (int v = 0; v < 5; v++) {
+    if (v == ref_idx) continue;
+    double f[5], S[5], ll, total = 0.0;
+#pragma unroll
+    for (int b = 0; b < 5; b++) {
+      f[b] = (b == v) ? 0.0 : 0.5 + (double)cnt[b];
+      total += f[b];
+    }
+#pragma unroll
+    for (int b = 0; b < 5; b++) f[b] /= total;
+    bool clear = false;
+    for (int it = 0; it < 8; it++) {
+      if (!key_pass(P, keys, hist, K, lane, f, S, ll)) return true;
+      if (upper - ll < need) {
+        clear = true;
+        break;
+      }
+      double most = 0.0;
+#pragma unroll
+      for (int b = 0; b < 5; b++) {
+        const double fn = f[b] * S[b] / n;
+        most = fmax(most, fabs(fn - f[b]));
+        f[b] = fn;
+      }
+      if (!(most > 2.0 * P.precision_decimal)) break;
+    }
+    if (!clear) return true;
+  }
+  return false;
+}
+
+// The exact scorer's candidates (one wavefront per column): insert slots of the columns with
+// insertions, and the column pass's candidates, those that its bound alone let through tested
+// again by may_be_emitted.  At 3,000 reads a column the bound of the column pass rules out next to
+// nothing (19,743 of 20,011 columns passed it, of which some 30 are emitted) and the exact null fit of
+// each took the scorer 35.6 ms; this test takes 0.98 ms and leaves 36 (1 Mb at 300x with
+// 390 variants: 7,852 candidates, 0.17 ms, leaves 451).
+// LDS: a count per table key, and the list of the keys that occur.
+__global__ void __launch_bounds__(64 * kRouteWaves) k_route_candidates(ImParams P) {
+  extern __shared__ uint32_t route_lds[];   // per wavefront: tab_keys counts, then tab_keys 16-bit keys
+  const int lane = threadIdx.x & (WAVE - 1), wave = uniform_i((int)threadIdx.x / WAVE);
+  const int wv = blockIdx.x * kRouteWaves + wave, n_wv = gridDim.x * kRouteWaves;
+  uint32_t* route_hist = route_lds + (size_t)wave * route_words(P.tab_keys);
+  uint16_t* list = (uint16_t*)(route_hist + P.tab_keys);
   uint32_t err = 0;
-  for (int i = blockIdx.x; i < n_ins; i += gridDim.x) {
-    const int p = P.ins[i];
+  const int n_ins = min(*P.n_ins, P.ins_cap);
+  for (int i = wv; i < n_ins; i += n_wv) route_insert_slots(P, uniform_i(P.ins[i]), lane, err);
+  const bool test = P.tab_keys <= kRouteKeys;
+  if (test)
+    for (int i = lane; i < P.tab_keys; i += WAVE) route_hist[i] = 0;
+  wave_lds_sync();
+  const int n_cand = min(*P.n_cand, P.cand_cap);
+  for (int ci = wv; ci < n_cand; ci += n_wv) {
+    const int2 cd = P.cand[ci];
+    const int p = uniform_i(cd.x);
     const int64_t w = p / WAVE;
     if (p < 0 || p >= P.n_pos || w >= P.n_windows) {
       err |= kErrIndex;
       continue;
     }
-    const int rb = P.win_rb[w], re = P.win_re[w];
-    if (rb < 0 || re < rb || re > P.n_reads) {
-      err |= kErrIndex;
-      continue;
-    }
-    for (int slot = 1; slot < 65536; slot++) {
-      if (lane == 0) {
-        const int c = atomicAdd(P.n_cand, 1);
-        if (c < P.cand_cap) P.cand[c] = make_int2(p, slot);
-        else err |= kErrCapacity;
+    bool keep = true;
+    if (uniform_i(cd.y) == kCandScreened && test) {
+      const int rb = uniform_i(P.win_rb[w]), re = uniform_i(P.win_re[w]);
+      if (rb < 0 || re < rb || re > P.n_reads) {
+        err |= kErrIndex;
+        continue;
       }
-      bool next = false;
+      const uint32_t qspan = (uint32_t)max(0, P.quality_max - P.base_quality_cutoff);
+      uint32_t cnt[5] = {0, 0, 0, 0, 0};
       for (int r0 = rb; r0 < re; r0 += WAVE) {
         const int r = r0 + lane;
-        if (r >= re) continue;
-        const DRead R = P.reads[r];
-        if (R.x1 != 1) continue;
-        int qpos, indel;
-        bool is_del;
-        if (!entry_at(R, P.cigar, p, qpos, indel, is_del, err) || is_del || indel <= slot) continue;
-        if (P.bases[R.seq_off + qpos + slot] != 15) next = true;
+        bool use = false;
+        uint32_t key = 0;
+        int obs = 0;
+        bool past = true;   // starts after the column: so do all later ones
+        if (r < re) {
+          const uint4* src = (const uint4*)(P.idrec + r);
+          const uint4 ra = src[0], rc = src[1];
+          past = (int)ra.x > p;
+          const uint32_t xf = rc.z, flags = xf >> 16;
+          if ((uint32_t)p - ra.x < ra.y - ra.x && (xf & 0xFFFFu) == 1u) {
+            if (flags & kReadSimple) {
+              const uint32_t qpos = (uint32_t)p + ra.w;
+              const uint32_t b = P.bases[ra.z + qpos], q = P.quals[ra.z + qpos];
+              const int o = bam_index((uint8_t)b);
+              use = o >= 0 && o < 4 && qpos >= (rc.x & 0xFFFFu) && qpos < (rc.x >> 16) &&
+                    q - (uint32_t)P.base_quality_cutoff < qspan && rc.y != 0xffffffffu;
+              obs = o;
+              key = rc.y * 2u + q * 10u + (uint32_t)o * 2u + ((flags & kReadReversed) ? 1u : 0u);
+            } else {
+              // data errors of this read were reported by the column pass
+              int strand_idx = 0;
+              uint32_t e = 0;
+              use = pdata_key(P.reads[r], P.cigar, P.bases, P.quals, p, 0, P.read_set_max, P.quality_max,
+                              P.base_quality_cutoff, key, obs, strand_idx, e);
+            }
+          }
+        }
+        use = use && key < (uint32_t)P.tab_keys;
+        if (use) atomicAdd(&route_hist[key], 1u);
+#pragma unroll
+        for (int b = 0; b < 5; b++) cnt[b] += (uint32_t)__popcll(__ballot(use && obs == b));
+        if (__all(past)) break;
       }
-      if (!__any(next)) break;
+      wave_lds_sync();
+      int K = 0;
+      for (int k0 = 0; k0 < P.tab_keys; k0 += WAVE) {
+        const bool on = k0 + lane < P.tab_keys && route_hist[k0 + lane] != 0;
+        const unsigned long long m = __ballot(on);
+        if (on) list[K + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)(k0 + lane);
+        K += __popcll(m);
+      }
+      wave_lds_sync();
+      const int c = char_index(P.ref[p]);
+      keep = K > 0 && may_be_emitted(P, list, route_hist, K, cnt, c < 0 ? 5 : c, lane);
+      wave_lds_sync();
+      for (int k = lane; k < K; k += WAVE) route_hist[list[k]] = 0;
+      wave_lds_sync();
+    }
+    if (keep && lane == 0) {
+      const int k = atomicAdd(P.n_score, 1);
+      if (k < P.cand_cap) P.score[k] = make_int2(p, 0);
+      else err |= kErrCapacity;
     }
   }
   if (err) atomicOr(P.err, err);

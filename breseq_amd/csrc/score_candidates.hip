@@ -3,32 +3,39 @@
 // Fisher strand and KS quality tests (identify_mutations.cpp:1669-1910, 3009-3318; stats.cpp
 // 2144-2284).
 //
-// One 4-wavefront block per candidate.  Every sum the reference forms over its per-read data
-// (pdata) is accumulated in read order, so results are bit-identical to a sequential loop:
-//   * EM: a wavefront runs up to two EM loops ("tasks") in lockstep.  Per pass, each lane takes
-//     one read and computes that read's responsibilities for every running task from a
-//     per-candidate LDS cache of the reads' table rows; then lane 5t+b adds term column b of task
-//     t in read order.  The in-order additions are the pass's critical path and its largest
-//     instruction count, and one pass of them serves both tasks.  The log likelihood, which
-//     the reference reports only from the last pass of a loop, is formed once per loop from that
-//     pass's frequencies: after its last update a task makes one more pass in "likelihood" mode.
-//   * The candidate's EM work is a chain of ~1000 passes (null fit, profile likelihoods,
-//     bisections), run as phases:
-//       phase 0: full fit | pure-genotype sums
-//       phase 1: null fit + a speculative bisection midpoint | profile at the ML frequency and
-//                at 1, then Fisher and KS | profile at 0 + a midpoint | two more midpoints
-//       phase 2+: bisection rounds.  Each round evaluates the midpoints a sequential bisection
-//                 would visit along one predicted path: eight levels with one bound open, four
-//                 per bound with both open (two midpoints per wavefront).  The path follows the
-//                 crossing point of a model of the profile likelihood (below); the round then
-//                 keeps every level up to the first one where the real decision leaves the path.
-//                 A bound whose prediction goes wrong within its first two levels switches to
-//                 full trees (seven midpoints = three levels, or three = two levels).  The first
-//                 four path levels (two per bound with both open) run in phase 1.  Only
-//                 midpoints the sequential bisection visits are used, so the bounds are its own.
-//   * Fisher terms are evaluated across lanes and added in order by one lane; the exact KS lattice
-//     is filled one anti-diagonal at a time (each cell is one addition of two neighbours, so the
-//     order of the cells does not change any value).
+// One block of four wavefronts per candidate.  A candidate is a chain of EM loops (50 passes over
+// its reads at most), so the kernel is bound by the latency of a pass, not by bandwidth.
+//
+//   * The reference forms every sum in read order, and its output is decided by comparisons and by
+//     printed digits.  The EM loops run with sums in any order, over the candidate's distinct table
+//     keys weighted with their reads (em_full, em_tasks): the same iterations, whose results differ from
+//     the reference's by rounding (about 1e-15 in a frequency, 1e-11 in a log10 likelihood).  Every
+//     decision and every printed digit is then checked to lie farther from its boundary than a
+//     guard some hundred times that (kGuardLog, kGuardRel); the candidates where one does not, about one
+//     in a hundred with 8 printed digits, are done once more with the reference's sums, as are all of
+//     them when the screen is off.
+//   * em_exact makes the reference's sums: row g of a wavefront (16 lanes) holds allele g's terms of 16
+//     reads, and a chain of 16 additions whose operand is broadcast from lane k of the row
+//     (v_fmac_f64 with row_newbcast, times 1.0, which rounds like an addition) adds them in order,
+//     the fifth allele in a second chain beside the first; some 500 cycles per 16 reads.
+//   * The frequency bounds are bisections, 20 levels each.  The midpoints a round evaluates lie on
+//     one predicted path per bound: the crossing point is solved from the profile's likelihood with
+//     the other alleles' proportions held (model_root), and the path holds the midpoints a sequential
+//     bisection visits if every decision agrees with it.  The walk afterwards keeps every level up to
+//     the first one where a decision leaves the path.  From the second round on the first levels are a
+//     full tree, so a round always gains some.
+//
+// Phases: full fit (wavefront 0) | pure-genotype sums and call, in order (1); then rounds of the EM
+// tasks (0-2): the null fit, the profiles at the ML frequency, 0 and 1 and the bounds' midpoints, 24
+// tasks of eight lanes or 48 of four | KS and Fisher (3, first round).
+//
+// With 669 candidates of about 100 reads the kernel takes 0.26 ms (1.23 ms with two ordered EM tasks per
+// wavefront in LDS and three rounds of bisection); 28 candidates of 206 reads take 0.15 ms (1.40 ms),
+// 36 of 3,000 reads 0.39 ms.
+//
+// Fisher terms are evaluated across lanes and added in order by one lane; the exact KS lattice is
+// filled one anti-diagonal at a time (each cell is one addition of two neighbours, so the order of
+// the cells does not change any value).
 #include <hip/hip_runtime.h>
 
 #include "device_common.h"
@@ -40,58 +47,47 @@ namespace {
 
 constexpr int kSW = kScoreWaves;
 static_assert(kSW == 4, "phase roles are laid out for four wavefronts");
-constexpr int kTW = 2;           // EM tasks per wavefront
-constexpr int kTermCols = 64;    // reads per EM chunk (one per lane)
-constexpr int kTermRow = 65;     // LDS row stride of a term column: the summing lanes hit different banks
-constexpr int kKsDiag = 100;     // exact KS runs when m*n < 10000, so min(m, n) <= 99
-constexpr int kBisectPts = 8;    // midpoints evaluated per bound and round (one per task slot)
-
-// result slots of the phase tasks
-enum { kResFull = 0, kResNull = 1, kResPlmax = 2, kResP0 = 3, kResP1 = 4, kResBisect = 5 };   // + side*8 + node
-constexpr int kNumRes = kResBisect + 2 * kBisectPts;
-
-// EM task states
-enum { kTaskIdle = 0, kTaskIter = 1, kTaskLast = 2 };
-
-// The EM tasks of one wavefront (LDS).
-struct WaveTasks {
-  double term[kTW][5][kTermRow];   // per task: five term columns of the current chunk
-  double f[kTW][5];                // current frequencies
-  double fl[kTW][5];               // frequencies of the last pass (the likelihood pass uses them)
-  double sum[kTW][5];              // the pass's in-order sums
-  double delta[kTW][5];            // |new - old| frequency per allele of the last update
-  double x[kTW];                   // profile: pinned frequency
-  int32_t mode[kTW];               // 1 fit, 2 profile
-  uint32_t allowed[kTW];
-  int32_t v[kTW];                  // profile: pinned allele
-  int32_t state[kTW];
-  int32_t it[kTW];
-  int32_t res[kTW];                // result slot
-};
+constexpr int kTaskWaves = 3;            // wavefronts of the EM tasks; the fourth has the statistics
+constexpr int kTaskSlots = 48;           // most tasks of a round: 4 lanes each, or 24 of 8 lanes
+constexpr int kKsDiag = 100;             // exact KS runs when m*n < 10000, so min(m, n) <= 99
+constexpr double kDrop = 0.587566;       // kProfileLikelihoodLog10Drop (identify_mutations.cpp:3173)
+// How far a result of sums in any order may be from the reference's, generously: the rounding of
+// 50 EM passes leaves a frequency within about 1e-15 (relative) and a log10 likelihood within about
+// 1e-11.  A decision or a printed digit closer to its boundary than this is made on exact sums.
+constexpr double kGuardLog = 1e-8;       // log10 likelihoods and scores
+constexpr double kGuardRel = 1e-12;      // frequencies, relative
 
 struct ScoreShared {
-  WaveTasks wt[kSW];
   double full_f[5];
-  double lps[5];
-  double res[kNumRes];
-  double pts[2][kBisectPts];       // bisection midpoints of the round, per bound
+  double fit[5];                   // frequencies em_exact starts from and leaves
+  double full_ll, null_ll;
+  double gscore;                   // pure-genotype score
+  double val[kTaskSlots];          // profile values of the round's tasks (without the lpmax sum)
+  double pts[2][kTaskSlots];       // bisection midpoints of the round, per bound
   double vlo[2], vhi[2];           // profile values at the ends of each bound's interval
   double lo[2], hi[2];
-  double target, lower, upper, ks_p, fisher_p;
+  double out[2];                   // the bounds as reported so far
+  double target, ks_p, fisher_p;
+  double exact_x[2], exact_v, exact_target;
   double ks_a[kKsDiag + 1], ks_b[kKsDiag + 1];
   double fisher[64];
+  double ks_log_total;
   uint32_t ks_bnd[(10000 + 2 + 31) / 32 + 1];
   uint32_t qh[2][128];
   uint32_t cov[6][3];
   uint32_t obs[5];                 // reads per observed class (both strands)
   uint32_t wcount[kSW];
   int32_t n_keys;
+  int32_t best;                    // pure-genotype best allele
   int32_t iter[2];
   int32_t active[2];
-  int32_t depth[2];                // bisection levels evaluated this round, per bound
-  int32_t path[2];                 // this round's midpoints follow one predicted path (else: a tree)
-  int32_t tree_only[2];            // a predicted path went wrong early: trees from then on
-  int32_t spec[2];                 // first path levels per bound evaluated beside phase 1
+  int32_t depth[2];                // midpoints evaluated this round, per bound
+  int32_t slot0[2];                // first task slot of each bound's midpoints
+  int32_t n_tree;                  // the first of each bound's midpoints are a full tree's nodes
+  int32_t exact;                   // bounds: 0 a round of tasks, 1 + side: an exact comparison is needed
+  int32_t exact_have;              // exact_target is known
+  int32_t bad_r;                   // a ratio outside the fast division's range
+  int32_t unsure;                  // a result too close to a boundary: the candidate is done again exactly
   int32_t emitted;
   int32_t done;
 };
@@ -100,7 +96,6 @@ struct ScoreShared {
 // compile to LDS instructions rather than generic (flat) ones, whose waits also cover memory loads.
 typedef __attribute__((address_space(3))) double LdsDouble;
 typedef __attribute__((address_space(3))) uint32_t LdsU32;
-typedef __attribute__((address_space(3))) WaveTasks LdsTasks;
 typedef __attribute__((address_space(3))) ScoreShared LdsShared;
 
 static_assert(sizeof(ScoreShared) <= kScoreStaticLds, "scorer static LDS above its declared bound");
@@ -111,13 +106,6 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ double readfirstlane_d(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffLL));
-  const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
 __device__ __forceinline__ double readlane_d(double v, int l) {
   const long long b = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), l);
@@ -125,326 +113,631 @@ __device__ __forceinline__ double readlane_d(double v, int l) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// The candidate's reads: per read the table row r[0..4] = 10^(lp_b - lpmax), r[5] = lpmax, cached
-// in LDS when it fits, else read from the table in HBM.
+__device__ __forceinline__ double readfirstlane_d(double v) { return readlane_d(v, 0); }
+
+template <int kCtrl>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffffLL), kCtrl, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), kCtrl, 0xf, 0xf, true);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Cross-lane sum over aligned groups of kN lanes; every lane of the group gets the same value.
+template <int kN>
+__device__ __forceinline__ double sum_lanes(double v) {
+  v = dpp_add<0x4E>(dpp_add<0xB1>(v));            // quad_perm: lane ^ 1, lane ^ 2
+  if constexpr (kN >= 8) v = dpp_add<0x141>(v);   // row_half_mirror: the other quad of eight lanes
+  if constexpr (kN == 64) {
+    v = dpp_add<0x140>(v);                        // row_mirror: the other eight of a row
+    v = (readlane_d(v, 0) + readlane_d(v, 16)) + (readlane_d(v, 32) + readlane_d(v, 48));
+  }
+  return v;
+}
+
+// 1/s correctly rounded for a normal s well inside the exponent range: the hardware's reciprocal
+// estimate, two Newton steps, and the correction step of a division by s (numerator 1), each fused.
+__device__ __forceinline__ double recip_newton(double s) {
+  double y = __builtin_amdgcn_rcp(s);
+  y = fma(fma(-s, y, 1.0), y, y);
+  y = fma(fma(-s, y, 1.0), y, y);
+  return y;
+}
+
+// The candidate's reads.  A read's likelihoods depend on its table key alone, so the rows
+// r[0..4] = 10^(lp_b - lpmax), r[5] = lpmax are kept once per distinct key, with the number of its
+// reads, and the reads' list holds each read's row.  Where the rows are is a compile-time choice
+// of the loops over them:
+//   kRowsLds     in LDS (they fit)
+//   kRowsGlobal  in the table in HBM: the list holds keys, and every read is a row of its own
+enum { kRowsLds = 0, kRowsGlobal = 1 };
+
 struct Rows {
-  const double* lds;            // n x 6, or nullptr
-  const uint32_t* keys;
+  const uint32_t* list;         // per read: its row (kRowsLds) or its key (kRowsGlobal)
+  const double* lds;            // rows, six doubles each
+  const uint32_t* reads;        // per row: its reads (kRowsLds)
   const double* __restrict__ tab_r;
-  __device__ __forceinline__ void get(int i, double r[6]) const {
-    if (lds) {
-      typedef __attribute__((address_space(3))) const double LdsD;
-      const LdsD* p = (const LdsD*)lds + (size_t)i * 6;
+  template <int kKind>
+  __device__ __forceinline__ void row(int k, double r[6]) const {   // k: a row or a key
+    typedef __attribute__((address_space(3))) const double LdsD;
+    if constexpr (kKind == kRowsGlobal) {
+      const double* p = tab_r + (size_t)k * 6;
 #pragma unroll
-      for (int k = 0; k < 6; k++) r[k] = p[k];
+      for (int c = 0; c < 6; c++) r[c] = p[c];
     } else {
-      const double* p = tab_r + (size_t)keys[i] * 6;
+      const LdsD* p = (const LdsD*)lds + k * 6;
 #pragma unroll
-      for (int k = 0; k < 6; k++) r[k] = p[k];
+      for (int c = 0; c < 6; c++) r[c] = p[c];
+    }
+  }
+  // row `i` of the distinct rows, and its reads
+  template <int kKind>
+  __device__ __forceinline__ uint32_t distinct(int i, double r[6]) const {
+    if constexpr (kKind == kRowsGlobal) {
+      row<kKind>((int)list[i], r);
+      return 1u;
+    } else {
+      row<kKind>(i, r);
+      return ((const __attribute__((address_space(3))) uint32_t*)reads)[i];
     }
   }
 };
 
-// acc + t[0] + t[1] + ... + t[m-1], added left to right (one lane).  LDS latency (~120 cycles)
-// is 25 dependent FP64 additions, so the reads run three groups of eight (24 terms) ahead of
-// the additions.
-__device__ __forceinline__ double sum_in_order(double acc, const LdsDouble* t, int m) {
-  int j = 0;
-  if (m >= 32) {
-    double c0[8], c1[8], c2[8];
+// Arguments of functions that are not inlined arrive in vector registers; a wave-uniform one is
+// made scalar again, so that the branches and loops on it are scalar too.
+__device__ __forceinline__ int uniform_i(int v) { return __builtin_amdgcn_readfirstlane(v); }
+template <class T>
+__device__ __forceinline__ T* uniform_p(T* q) {
+  const uint64_t u = (uint64_t)q;
+  const uint32_t lo = (uint32_t)uniform_i((int)(uint32_t)u), hi = (uint32_t)uniform_i((int)(uint32_t)(u >> 32));
+  return (T*)(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ Rows uniform_rows(const Rows& R) {
+  return Rows{uniform_p(R.list), uniform_p(R.lds), uniform_p(R.reads), uniform_p(R.tab_r)};
+}
+
+template <bool kListGlobal>
+__device__ __forceinline__ uint32_t list_at(const uint32_t* list, int i) {
+  if constexpr (kListGlobal) return list[i];
+  else return ((const __attribute__((address_space(3))) uint32_t*)list)[i];
+}
+
+// One step of the two in-order chains: a += (lane K of this lane's row of ta), b likewise.
+// v_fmac_f64 rounds ta * 1.0 + a once, as an addition does.
+#define BSQ_CHAIN(K)                                                                                  \
+  asm("v_fmac_f64_dpp %0, %2, %4 row_newbcast:" #K " row_mask:0xf bank_mask:0xf\n\t"                  \
+      "v_fmac_f64_dpp %1, %3, %4 row_newbcast:" #K " row_mask:0xf bank_mask:0xf"                       \
+      : "+v"(a), "+v"(b)                                                                              \
+      : "v"(ta), "v"(tb), "v"(one))
+// the first step waits out the VALU-write-to-DPP-read hazard of its operands, the last one the
+// VALU-write-to-readlane hazard of its results
+#define BSQ_CHAIN_FIRST                                                                               \
+  asm("s_nop 1\n\t"                                                                                   \
+      "v_fmac_f64_dpp %0, %2, %4 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"                       \
+      "v_fmac_f64_dpp %1, %3, %4 row_newbcast:0 row_mask:0xf bank_mask:0xf"                            \
+      : "+v"(a), "+v"(b)                                                                              \
+      : "v"(ta), "v"(tb), "v"(one))
+#define BSQ_CHAIN_LAST                                                                                \
+  asm("v_fmac_f64_dpp %0, %2, %4 row_newbcast:15 row_mask:0xf bank_mask:0xf\n\t"                      \
+      "v_fmac_f64_dpp %1, %3, %4 row_newbcast:15 row_mask:0xf bank_mask:0xf\n\t"                      \
+      "s_nop 1"                                                                                       \
+      : "+v"(a), "+v"(b)                                                                              \
+      : "v"(ta), "v"(tb), "v"(one))
+
+// The terms of 16 reads (one per lane of a row, the same reads in every row): ta the row's allele
+// w_i(g), tb the fifth allele's, w_i(b) = f_b r_i(b) / s_i with s_i = Sum_b f_b r_i(b) in allele
+// order, each quotient correctly rounded (the SharedDiv step: one reciprocal per read, then an FMA
+// correction); f_b where s_i = 0; -0.0, which changes no sum, past the last read.  An allele that
+// is not allowed has f_b = 0, so its products add nothing to s_i and its terms are 0.
+struct Freq {
+  double f0, f1, f2, f3, f4;
+  double fg;      // the frequency of this lane's row
+  bool slow;      // a product f_b r_i(b) may be too small for the shared reciprocal
+};
+
+__device__ __forceinline__ double row_value(double v0, double v1, double v2, double v3, int g) {
+  return g < 2 ? (g == 0 ? v0 : v1) : (g == 2 ? v2 : v3);
+}
+
+struct Terms {
+  double ta, tb;
+  double s, xg, x4;
+};
+
+__device__ __forceinline__ Terms em_terms(const double r[6], const Freq& F, int g, bool live) {
+  Terms T;
+  const double x0 = F.f0 * r[0], x1 = F.f1 * r[1], x2 = F.f2 * r[2], x3 = F.f3 * r[3];
+  T.x4 = F.f4 * r[4];
+  T.s = (((x0 + x1) + x2) + x3) + T.x4;
+  T.xg = row_value(x0, x1, x2, x3, g);
+  const double y0 = recip_newton(T.s);
+  const double y = fma(fma(-T.s, y0, 1.0), y0, y0);
+  const double qa = T.xg * y, qb = T.x4 * y;
+  const double ta = fma(fma(-T.s, qa, T.xg), y, qa);
+  const double tb = fma(fma(-T.s, qb, T.x4), y, qb);
+  T.ta = live ? ta : -0.0;
+  T.tb = live ? tb : -0.0;
+  return T;
+}
+
+// The terms by ordinary division, f_b where s_i = 0: what the fast quotients do not cover.
+__device__ __forceinline__ void em_terms_slow(Terms& T, const Freq& F, bool live) {
+  const double ta = (T.s > 0.0) ? T.xg / T.s : F.fg;
+  const double tb = (T.s > 0.0) ? T.x4 / T.s : F.f4;
+  T.ta = live ? ta : -0.0;
+  T.tb = live ? tb : -0.0;
+}
+
+// One EM loop of the reference with its sums in read order, by one wavefront; returns the log10
+// likelihood it reports and leaves the final frequencies in fit[].
+//   mode 1: fit_allele_frequencies (identify_mutations.cpp:3240-3318) from the frequencies in fit[];
+//           allele v (if any) is held out, with frequency zero.
+//   mode 2: profile_log10_likelihood (:3094-3143): fit[v] pinned to x.
+// 50 passes at most; a loop ends when no frequency moved by tol, and the likelihood is that of the
+// last pass's frequencies: Sum_i (log10 s_i + lpmax_i) over reads with s_i > 0, in read order.
+template <int kKind, bool kListGlobal>
+__device__ __noinline__ double em_exact(const Rows Rv, int nv, int modev, int vv, double xv, LdsDouble* fit, double tolv,
+                                        int bad_rv) {
+  const Rows R = uniform_rows(Rv);
+  const int n = uniform_i(nv), mode = uniform_i(modev), v = uniform_i(vv), bad_r = uniform_i(bad_rv);
+  const double x = readfirstlane_d(xv), tol = readfirstlane_d(tolv);
+  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+  auto L = [&](int i) { return (int)list_at<kListGlobal>(R.list, i); };
+  Freq F;
+  F.f0 = readfirstlane_d(fit[0]);
+  F.f1 = readfirstlane_d(fit[1]);
+  F.f2 = readfirstlane_d(fit[2]);
+  F.f3 = readfirstlane_d(fit[3]);
+  F.f4 = readfirstlane_d(fit[4]);
+  double l0, l1, l2, l3, l4;   // frequencies of the last pass
+  const double dn = (double)n, one = 1.0;
+  const SharedDiv by_n(dn);
+  // the first two groups of 16 reads, which every pass begins with
+  double r0[6], r1[6];
+  R.row<kKind>(L(min(j, n - 1)), r0);
+  R.row<kKind>(L(min(16 + j, n - 1)), r1);
+  const int third = L(min(32 + j, n - 1));
+  F.fg = row_value(F.f0, F.f1, F.f2, F.f3, g);
+  for (int it = 0;;) {
+    // with a ratio of at least 2^-100 or 0, a frequency of at least 2^-800 or 0 keeps every product
+    // inside the range where the fast quotients are correctly rounded
+    F.slow = bad_r || __any((F.fg != 0.0 && F.fg < 0x1p-800) || (F.f4 != 0.0 && F.f4 < 0x1p-800));
+    double a = 0.0, b = 0.0;
+    double r[6];
+    Terms T = em_terms(r0, F, g, j < n);
+    if (F.slow || __any(!(T.s > 0.0))) em_terms_slow(T, F, j < n);
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-      c0[k] = t[k];
-      c1[k] = t[8 + k];
-      c2[k] = t[16 + k];
+    for (int k = 0; k < 6; k++) r[k] = r1[k];
+    int next = third;
+    for (int c0 = 0; c0 < n; c0 += 16) {
+      // the chain over these 16 reads, with the next 16 reads' terms computed between its steps
+      // (the compiler interleaves them) and the reads after those loaded
+      const double ta = T.ta, tb = T.tb;
+      const bool live = c0 + 16 + j < n;
+      BSQ_CHAIN_FIRST;
+      BSQ_CHAIN(1);
+      BSQ_CHAIN(2);
+      BSQ_CHAIN(3);
+      T = em_terms(r, F, g, live);
+      R.row<kKind>(next, r);
+      next = L(min(c0 + 48 + j, n - 1));
+      BSQ_CHAIN(4);
+      BSQ_CHAIN(5);
+      BSQ_CHAIN(6);
+      BSQ_CHAIN(7);
+      BSQ_CHAIN(8);
+      BSQ_CHAIN(9);
+      BSQ_CHAIN(10);
+      BSQ_CHAIN(11);
+      BSQ_CHAIN(12);
+      BSQ_CHAIN(13);
+      BSQ_CHAIN(14);
+      BSQ_CHAIN_LAST;
+      // the usual terms are final here, in the chain's own block; without this the compiler moves
+      // their divisions behind the branch below
+      asm volatile("" : "+v"(T.ta), "+v"(T.tb));
+      if (F.slow || __any(!(T.s > 0.0))) em_terms_slow(T, F, live);
     }
-    for (; j + 32 <= m; j += 8) {
-      double nx[8];
+    // the reference's loop body: new frequencies, and whether any moved by tol
+    double fa = F.fg, fb = F.f4;
+    if (mode == 1) {
+      if (g != v) fa = by_n(a);
+      if (4 != v) fb = by_n(b);
+    } else {
+      const double s0 = readlane_d(a, 0), s1 = readlane_d(a, 16), s2 = readlane_d(a, 32), s3 = readlane_d(a, 48), s4 = b;
+      double others = 0.0;
+      if (v != 0) others += s0;
+      if (v != 1) others += s1;
+      if (v != 2) others += s2;
+      if (v != 3) others += s3;
+      if (v != 4) others += s4;
+      const SharedDiv d(others);
+      const double rest = (1.0 - x) / 4.0;
+      if (g != v) fa = (others > 0.0) ? d((1.0 - x) * a) : rest;
+      if (4 != v) fb = (others > 0.0) ? d((1.0 - x) * b) : rest;
+    }
+    const bool moved = __any(fabs(fa - F.fg) >= tol || fabs(fb - F.f4) >= tol);
+    l0 = F.f0;
+    l1 = F.f1;
+    l2 = F.f2;
+    l3 = F.f3;
+    l4 = F.f4;
+    F.f0 = readlane_d(fa, 0);
+    F.f1 = readlane_d(fa, 16);
+    F.f2 = readlane_d(fa, 32);
+    F.f3 = readlane_d(fa, 48);
+    F.f4 = readlane_d(fb, 0);
+    F.fg = fa;
+    if (++it >= 50 || !moved) break;
+  }
+  if (lane == 0) {
+    fit[0] = F.f0;
+    fit[1] = F.f1;
+    fit[2] = F.f2;
+    fit[3] = F.f3;
+    fit[4] = F.f4;
+  }
+  // the likelihood: 64 reads' terms at a time, added row by row
+  double ll = 0.0;
+  for (int c0 = 0; c0 < n; c0 += 64) {
+    double r[6];
+    R.row<kKind>(L(min(c0 + lane, n - 1)), r);
+    const double s = (((l0 * r[0] + l1 * r[1]) + l2 * r[2]) + l3 * r[3]) + l4 * r[4];
+    double ta = (s > 0.0) ? log10(s) + r[5] : 0.0;
+    if (c0 + lane >= n) ta = -0.0;
+    const double tb = -0.0;
+    double b = 0.0;
+#pragma unroll 1
+    for (int row = 0; row < 64; row += 16) {
+      double a = ll;
+      BSQ_CHAIN_FIRST;
+      BSQ_CHAIN(1);
+      BSQ_CHAIN(2);
+      BSQ_CHAIN(3);
+      BSQ_CHAIN(4);
+      BSQ_CHAIN(5);
+      BSQ_CHAIN(6);
+      BSQ_CHAIN(7);
+      BSQ_CHAIN(8);
+      BSQ_CHAIN(9);
+      BSQ_CHAIN(10);
+      BSQ_CHAIN(11);
+      BSQ_CHAIN(12);
+      BSQ_CHAIN(13);
+      BSQ_CHAIN(14);
+      BSQ_CHAIN_LAST;
+      ll = readlane_d(a, row);
+    }
+  }
+  return ll;
+}
+
+// The in-order sums of the reads' log10 likelihoods under each hypothesis (identify_mutations.cpp:
+// 1669-1689), by one wavefront: lane g*16 + j reads hypothesis g of read j, as em_exact's rows.
+template <bool kListGlobal>
+__device__ __noinline__ void genotype_sums(const uint32_t* list, const uint32_t* key_of, const double* __restrict__ tab_lp,
+                                           int nv, double* lps) {
+  const int n = uniform_i(nv);
+  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+  const double one = 1.0;
+  double a = 0.0, b = 0.0;
+  for (int c0 = 0; c0 < n; c0 += 64) {
+    double va[4], vb[4];
 #pragma unroll
-      for (int k = 0; k < 8; k++) nx[k] = t[j + 24 + k];
+    for (int q = 0; q < 4; q++) {
+      const int i = c0 + 16 * q + j;
+      const uint32_t e = list_at<kListGlobal>(list, min(i, n - 1));
+      const double* lp = tab_lp + (size_t)(key_of ? key_of[e] : e) * 5;
+      va[q] = lp[g];
+      vb[q] = lp[4];
+      if (i >= n) va[q] = vb[q] = -0.0;
+    }
 #pragma unroll
-      for (int k = 0; k < 8; k++) acc += c0[k];
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        c0[k] = c1[k];
-        c1[k] = c2[k];
-        c2[k] = nx[k];
+    for (int q = 0; q < 4; q++) {
+      const double ta = va[q], tb = vb[q];
+      BSQ_CHAIN_FIRST;
+      BSQ_CHAIN(1);
+      BSQ_CHAIN(2);
+      BSQ_CHAIN(3);
+      BSQ_CHAIN(4);
+      BSQ_CHAIN(5);
+      BSQ_CHAIN(6);
+      BSQ_CHAIN(7);
+      BSQ_CHAIN(8);
+      BSQ_CHAIN(9);
+      BSQ_CHAIN(10);
+      BSQ_CHAIN(11);
+      BSQ_CHAIN(12);
+      BSQ_CHAIN(13);
+      BSQ_CHAIN(14);
+      BSQ_CHAIN_LAST;
+    }
+  }
+  lps[0] = readlane_d(a, 0);
+  lps[1] = readlane_d(a, 16);
+  lps[2] = readlane_d(a, 32);
+  lps[3] = readlane_d(a, 48);
+  lps[4] = readlane_d(b, 0);
+}
+
+// Sum_i log10 s_i over distinct rows with their reads, s_i > 2^-100: the products of the powers,
+// exponents kept apart, one logarithm at the end.
+struct LogSum {
+  double p = 1.0;
+  int e = 0;
+  __device__ __forceinline__ void add(double s, uint32_t h) {
+    double q = s;
+    int eq = 0;
+    for (;;) {
+      if (h & 1u) {
+        p *= q;
+        e += __builtin_amdgcn_frexp_exp(p) + eq;
+        p = __builtin_amdgcn_frexp_mant(p);
       }
+      h >>= 1;
+      if (!h) break;
+      q *= q;
+      const int x = __builtin_amdgcn_frexp_exp(q);
+      q = __builtin_amdgcn_frexp_mant(q);
+      eq = 2 * eq + x;
     }
-#pragma unroll
-    for (int k = 0; k < 8; k++) acc += c0[k];
-#pragma unroll
-    for (int k = 0; k < 8; k++) acc += c1[k];
-#pragma unroll
-    for (int k = 0; k < 8; k++) acc += c2[k];
-    j += 24;
   }
-  for (; j < m; j++) acc += t[j];
-  return acc;
-}
+  __device__ __forceinline__ double value() const { return log10(p) + (double)e * 0.30102999566398119521; }
+};
 
-// The same for exactly K terms (K a multiple of 8), unrolled in groups of eight, each group's LDS
-// reads issued two groups before it is added.
-template <int K>
-__device__ __forceinline__ double sum_in_order_k(double acc, const LdsDouble* t) {
-  static_assert(K % 8 == 0, "groups of eight");
-  constexpr int G = K / 8;
-  double g0[8], g1[8], g2[8];
+// fit_allele_frequencies (identify_mutations.cpp:3240-3318) over all alleles with sums in any order,
+// by one wavefront: 64 lanes share the distinct rows.  Leaves the frequencies in f and returns the
+// log10 likelihood without the sum of the reads' lpmax; NaN where the loop cannot stand for the
+// reference's (a read with s_i = 0, or a last step too close to tol).
+template <int kKind>
+__device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble* fit, double tol) {
+  const Rows R = uniform_rows(Rv);
+  const int K = uniform_i(Kv), lane = threadIdx.x & 63;
+  const double per_n = 1.0 / (double)uniform_i(nv);
+  double f[5], fl[5];
 #pragma unroll
-  for (int k = 0; k < 8; k++) g0[k] = t[k];
-  if (G > 1) {
+  for (int b = 0; b < 5; b++) f[b] = fl[b] = fit[b];
+  bool bad = false;
+  for (int it = 1;; it++) {
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int i = lane; i < K; i += 64) {
+      double r[6];
+      const uint32_t h = R.distinct<kKind>(i, r);
+      double s = f[0] * r[0];
 #pragma unroll
-    for (int k = 0; k < 8; k++) g1[k] = t[8 + k];
-  }
+      for (int b = 1; b < 5; b++) s = fma(f[b], r[b], s);
+      const double y = recip_newton(s) * (double)h;
 #pragma unroll
-  for (int grp = 0; grp < G; grp++) {
-    double* cur = (grp % 3 == 0) ? g0 : (grp % 3 == 1) ? g1 : g2;
-    double* nxt = (grp % 3 == 0) ? g2 : (grp % 3 == 1) ? g0 : g1;
-    if (grp + 2 < G) {
-#pragma unroll
-      for (int k = 0; k < 8; k++) nxt[k] = t[(grp + 2) * 8 + k];
+      for (int b = 0; b < 5; b++) acc[b] = fma(r[b], y, acc[b]);
     }
-#pragma unroll
-    for (int k = 0; k < 8; k++) acc += cur[k];
-  }
-  return acc;
-}
-
-// A chunk's column of m terms, padded in LDS with -0.0 up to the next multiple of 16: adding -0.0
-// leaves every double unchanged (+0.0 included), so the result is the in-order sum of the m terms.
-__device__ __forceinline__ double sum_chunk(double acc, const LdsDouble* t, int m) {
-  switch ((m + 15) >> 4) {
-    case 1: return sum_in_order_k<16>(acc, t);
-    case 2: return sum_in_order_k<32>(acc, t);
-    case 3: return sum_in_order_k<48>(acc, t);
-    default: return sum_in_order_k<64>(acc, t);
-  }
-}
-
-// Starts EM task slot t of a wavefront (one lane): the starting point of the reference's loops.
-//   mode 1: fit_allele_frequencies (identify_mutations.cpp:3240-3318) over the alleles in
-//           `allowed`, from the Laplace-smoothed counts obs_of.
-//   mode 2: profile_log10_likelihood (:3094-3143): f[v] pinned to x, the other alleles started
-//           from full_f rescaled.
-// A fit with no reads or no allowed allele has likelihood 0 and frequencies 0 without a pass.
-__device__ __noinline__ void task_start(LdsTasks* W, int t, int mode, uint32_t allowed, int v, double x, int res,
-                           const LdsU32* obs_of, const LdsDouble* full_f, int n, LdsDouble* res_out) {
-  double f[5];
-  W->mode[t] = mode;
-  W->v[t] = v;
-  W->x[t] = x;
-  W->res[t] = res;
-  W->it[t] = 0;
-  if (mode == 1) {
-#pragma unroll
-    for (int b = 0; b < 5; b++) f[b] = 0.0;
-    if (n == 0 || allowed == 0) {
-#pragma unroll
-      for (int b = 0; b < 5; b++) W->f[t][b] = 0.0;
-      W->state[t] = kTaskIdle;
-      res_out[res] = 0.0;
-      return;
-    }
-#pragma unroll
-    for (int b = 0; b < 5; b++)
-      if (allowed & (1u << b)) f[b] = 0.5 + (double)obs_of[b];   // 0.5 + one per observing read
-    double init_total = 0.0;
-#pragma unroll
-    for (int b = 0; b < 5; b++) init_total += f[b];
-#pragma unroll
-    for (int b = 0; b < 5; b++) f[b] /= init_total;
-  } else {
-    double other = 0.0;
-#pragma unroll
-    for (int b = 0; b < 5; b++)
-      if (b != v) other += full_f[b];
+    double most = 0.0, sum = 0.0;
 #pragma unroll
     for (int b = 0; b < 5; b++) {
-      if (b == v) f[b] = x;
-      else f[b] = (other > 0.0) ? (1.0 - x) * full_f[b] / other : (1.0 - x) / 4.0;
+      fl[b] = f[b];
+      f[b] = f[b] * sum_lanes<64>(acc[b]) * per_n;
+      sum += f[b];
+      most = fmax(most, fabs(f[b] - fl[b]));
     }
-    allowed = 31u;
+    bad = bad || !(sum > 0.5 && sum < 2.0) || (it < 50 && fabs(most - tol) < 1e-6 * tol);
+    if (!(most >= tol) || it >= 50) break;
   }
-  W->allowed[t] = allowed;
+  LogSum L;
+  for (int i = lane; i < K; i += 64) {
+    double r[6];
+    const uint32_t h = R.distinct<kKind>(i, r);
+    double s = fl[0] * r[0];
 #pragma unroll
-  for (int b = 0; b < 5; b++) W->f[t][b] = f[b];
-  W->state[t] = kTaskIter;
+    for (int b = 1; b < 5; b++) s = fma(fl[b], r[b], s);
+    bad = bad || !(s > 0x1p-100);
+    L.add(s, h);
+  }
+  const double ll = sum_lanes<64>(L.value());
+  if (lane == 0) {
+#pragma unroll
+    for (int b = 0; b < 5; b++) fit[b] = f[b];
+  }
+  return __any(bad) ? __longlong_as_double(0x7ff8000000000000LL) : ll;
 }
 
-// The likelihood pass of task t for one chunk of reads: term column 0 gets log10 s_i + lpmax_i
-// (0 for s_i = 0), s_i = Sum_{allowed b} f_b r_i(b) in allele order.  Kept out of line: the
-// inlined log10 would set the register budget of every EM pass, and runs once per EM loop.
-__device__ __noinline__ void likelihood_terms(const Rows R, int n, int c0, LdsTasks* W, int t, double f0, double f1,
-                                              double f2, double f3, double f4, uint32_t al) {
-  const int lane = threadIdx.x & 63;
-  const int i = c0 + lane;
-  if (i >= n) return;
-  double r[6];
-  R.get(i, r);
-  const double f[5] = {f0, f1, f2, f3, f4};
-  double s = 0.0;
+// The EM tasks of one wavefront, kSub lanes each: the null fit (the variant held out, from the counts
+// of the reads' observations) or profile_log10_likelihood (identify_mutations.cpp:3094-3143: the
+// variant pinned to x, the others from the full fit rescaled), the same iterations as em_exact's with
+// sums in any order over the candidate's distinct rows.  prow: per row the ratio of the variant, those
+// of the other four alleles in order, and the row's reads.  Returns log10 of the likelihood without
+// the sum of the reads' lpmax, which every such value of a candidate shares; NaN where the value cannot
+// stand for the reference's (a read with s_i = 0, or a last step too close to tol).
+//   start[4]: the other alleles' starting frequencies; scale: 1 / n in the null fit, else 0
+template <int kSub>
+__device__ __noinline__ double em_tasks(const LdsDouble* prow, int Kv, double x, double start0, double start1, double start2,
+                                        double start3, double scale_null, bool active, double tol) {
+  const int K = uniform_i(Kv), sub = threadIdx.x & (kSub - 1);
+  double f1 = start0, f2 = start1, f3 = start2, f4 = start3;
+  const double rest = (1.0 - x) / 4.0;
+  const bool null_fit = scale_null != 0.0;
+  bool run = active, bad = false;
+  for (int it = 1; __any(run); it++) {
+    double a1 = 0.0, a2 = 0.0, a3 = 0.0, a4 = 0.0;
+    // Four rows of a lane at a time, step by step: a row's chain (five products, a reciprocal, four
+    // sums) is some 250 cycles of latency and 16 instructions, so four in flight fill each other's
+    // waits.  The barriers keep the steps apart: left to itself the compiler runs the rows one after
+    // the other.
+    for (int i0 = sub; i0 < K; i0 += 4 * kSub) {
+      double r[4][5], h[4], s[4], y[4];
 #pragma unroll
-  for (int b = 0; b < 5; b++) {
-    const double x = f[b] * r[b];
-    if (al & (1u << b)) s += x;
+      for (int u = 0; u < 4; u++) {
+        const int i = i0 + u * kSub;
+        const LdsDouble* p = prow + min(i, K - 1) * 6;
+#pragma unroll
+        for (int b = 0; b < 5; b++) r[u][b] = p[b];
+        h[u] = (i < K) ? p[5] : 0.0;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; u++) s[u] = x * r[u][0];
+#pragma unroll
+      for (int u = 0; u < 4; u++) s[u] = fma(f1, r[u][1], s[u]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; u++) s[u] = fma(f2, r[u][2], s[u]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; u++) s[u] = fma(f3, r[u][3], s[u]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; u++) s[u] = fma(f4, r[u][4], s[u]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; u++) y[u] = __builtin_amdgcn_rcp(s[u]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int step = 0; step < 2; step++) {   // recip_newton
+        double e[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) e[u] = fma(-s[u], y[u], 1.0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 4; u++) y[u] = fma(e[u], y[u], y[u]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) y[u] *= h[u];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        a1 = fma(r[u][1], y[u], a1);
+        a2 = fma(r[u][2], y[u], a2);
+        a3 = fma(r[u][3], y[u], a3);
+        a4 = fma(r[u][4], y[u], a4);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    a1 = f1 * sum_lanes<kSub>(a1);
+    a2 = f2 * sum_lanes<kSub>(a2);
+    a3 = f3 * sum_lanes<kSub>(a3);
+    a4 = f4 * sum_lanes<kSub>(a4);
+    const double others = (a1 + a2) + (a3 + a4);
+    const double scale = null_fit ? scale_null : (1.0 - x) * recip_newton(others);
+    const bool some = others > 0.0;
+    const double g1 = some ? scale * a1 : rest, g2 = some ? scale * a2 : rest;
+    const double g3 = some ? scale * a3 : rest, g4 = some ? scale * a4 : rest;
+    const double most = fmax(fmax(fabs(g1 - f1), fabs(g2 - f2)), fmax(fabs(g3 - f3), fabs(g4 - f4)));
+    // (not-a-number sums fail the first test)
+    bad |= run & (!(others >= 0.0) | ((others > 0.0) & (others < 0x1p-500)) | ((it < 50) & (fabs(most - tol) < 1e-6 * tol)));
+    run &= (most >= tol) & (it < 50);
+    // a task that ends keeps this pass's frequencies: the likelihood is theirs
+    f1 = run ? g1 : f1;
+    f2 = run ? g2 : f2;
+    f3 = run ? g3 : f3;
+    f4 = run ? g4 : f4;
   }
-  W->term[t][0][lane] = (s > 0.0) ? log10(s) + r[5] : 0.0;
+  LogSum L;
+  for (int i = sub; i < K; i += kSub) {
+    const LdsDouble* p = prow + i * 6;
+    const double s = fma(f4, p[4], fma(f3, p[3], fma(f2, p[2], fma(f1, p[1], x * p[0]))));
+    bad = bad || !(s > 0x1p-100);
+    L.add(s, (uint32_t)p[5]);
+  }
+  const double ll = sum_lanes<kSub>(L.value());
+  // one lane that saw a read it cannot stand for spoils its task
+  const unsigned long long m = __ballot(bad);
+  const int base = (threadIdx.x & 63) & ~(kSub - 1);
+  return ((m >> base) & ((1ull << kSub) - 1ull)) ? __longlong_as_double(0x7ff8000000000000LL) : ll;
 }
 
-// Runs the started tasks of a wavefront to completion; each task's log10 likelihood goes to
-// res_out[its slot] and its final frequencies stay in W->f.  Per pass, for every running task:
-//   kTaskIter: sums[b] = Sum_i w_i(b), w_i(b) = f_b r_i(b) / s_i, s_i = Sum_{allowed b} f_b r_i(b)
-//   kTaskLast: sums[0] = Sum_i (log10 s_i + lpmax_i) over reads with s_i > 0
-// every sum in read order (identify_mutations.cpp:3268-3300); then the reference's loop body
-// (:3268-3318, 3094-3143) updates the frequencies: 50 passes at most, stop when the largest change
-// is below tol, then one likelihood pass from that last pass's frequencies.
-__device__ __noinline__ void run_tasks(const Rows R, int n, LdsTasks* W, double tol, LdsDouble* res_out) {
-  const int lane = threadIdx.x & 63;
-  const int my_t = min(lane / 5, kTW - 1), my_b = lane % 5;
-  const bool sum_lane = lane < 5 * kTW;
-  const LdsDouble* my_col = &W->term[my_t][my_b][0];
-  for (;;) {
-    // the pass's task states and frequencies, read once (wave-uniform)
-    int st[kTW];
-    uint32_t al[kTW];
-    double f[kTW][5];
-    bool any = false;
-#pragma unroll
-    for (int t = 0; t < kTW; t++) {
-      st[t] = __builtin_amdgcn_readfirstlane(W->state[t]);
-      al[t] = (uint32_t)__builtin_amdgcn_readfirstlane((int)W->allowed[t]);
-      const LdsDouble* src = (st[t] == kTaskLast) ? W->fl[t] : W->f[t];
-#pragma unroll
-      for (int b = 0; b < 5; b++) f[t][b] = readfirstlane_d(src[b]);
-      any = any || (st[t] != kTaskIdle);
-    }
-    if (!any) break;
-    double acc = 0.0;
-    for (int c0 = 0; c0 < n; c0 += kTermCols) {
-      const int i = c0 + lane;
-#pragma unroll
-      for (int t = 0; t < kTW; t++)
-        if (st[t] == kTaskLast) likelihood_terms(R, n, c0, W, t, f[t][0], f[t][1], f[t][2], f[t][3], f[t][4], al[t]);
-      if (i >= n) {
-        // padding of the chunk's last partial group of 16
-#pragma unroll
-        for (int t = 0; t < kTW; t++) {
-          LdsDouble* tm = &W->term[t][0][0];
-#pragma unroll
-          for (int b = 0; b < 5; b++) tm[b * kTermRow + lane] = -0.0;
-        }
+// Where the profile likelihood is predicted to cross the target inside the interval of bound
+// `side` (lanes 0-31: the lower bound, lanes 32-63: the upper one), used only to choose which
+// midpoints to evaluate.  Model: m(x) = Sum_i log10(t_i + x d_i), the likelihood with the other
+// alleles' proportions held at the full fit's (t_i their mixture, d_i = r_i(v) - t_i), with FP32
+// logarithms, whose rounding moves the prediction by about 1e-7.  It is evaluated at 32 points per
+// interval, the one bracketing the crossing is divided again, three times over, and the last
+// bracket's ends are joined by a line.  Once profile values are known at the interval's ends, the model
+// is corrected by the line through its errors there.  On 669 candidates of a 100x sample the path it
+// gives is right to the last of some 20 levels for 96% of the bounds.
+//   pre: per row d_i, t_i; prow: per row, its reads at [5]
+//   known: the values vlo / vhi hold (else the target is m at the ML frequency, minus the drop)
+__device__ __noinline__ double model_root(const LdsDouble* prow, const LdsDouble* pre, int Kv, double lo, double hi, bool known,
+                                          double vlo, double vhi, double target) {
+  const int K = uniform_i(Kv);
+  const int lane = threadIdx.x & 63, side = lane >> 5, k = lane & 31;
+  double a = lo, b = hi, d0 = 0.0, d1 = 0.0, va = 0.0, vb = 0.0;
+#pragma unroll 1
+  for (int round = 0; round < 3; round++) {
+    const double x = a + (b - a) * ((double)k * (1.0 / 31.0));
+    double l2 = 0.0;
+#pragma unroll 4
+    for (int i = 0; i < K; i++)
+      l2 = fma(prow[6 * i + 5], (double)__builtin_amdgcn_logf((float)fma(x, pre[2 * i], pre[2 * i + 1])), l2);
+    const double m = l2 * 0.30102999566398119521;
+    if (round == 0) {
+      const double m_lo = __shfl(m, 32 * side, 64), m_hi = __shfl(m, 32 * side + 31, 64);
+      if (known) {
+        d0 = vlo - m_lo;
+        d1 = vhi - m_hi;
+        if (!isfinite(d0)) d0 = isfinite(d1) ? d1 : 0.0;
+        if (!isfinite(d1)) d1 = d0;
       } else {
-        double r[6];
-        R.get(i, r);
-#pragma unroll
-        for (int t = 0; t < kTW; t++) {
-          if (st[t] != kTaskIter) continue;
-          double x[5];
-          double s = 0.0;
-#pragma unroll
-          for (int b = 0; b < 5; b++) {
-            x[b] = f[t][b] * r[b];
-            if (al[t] & (1u << b)) s += x[b];
-          }
-          LdsDouble* tm = &W->term[t][0][0];
-          double q[5];
-          if (s > 0.0) {
-            // f_b r_b / s correctly rounded from one reciprocal (the SharedDiv step, with the
-            // out-of-range fallback taken per lane only when needed)
-            const double y = 1.0 / s;
-            bool slow = !(s >= 0x1p-500 && s <= 0x1p500);
-#pragma unroll
-            for (int b = 0; b < 5; b++) {
-              const double q0 = x[b] * y;
-              q[b] = fma(fma(-s, q0, x[b]), y, q0);
-              slow = slow || !(x[b] == 0.0 || (x[b] >= 0x1p-500 && x[b] <= 0x1p500));
-            }
-            if (slow) {
-#pragma unroll
-              for (int b = 0; b < 5; b++) q[b] = x[b] / s;
-            }
-          } else {
-#pragma unroll
-            for (int b = 0; b < 5; b++) q[b] = f[t][b];
-          }
-#pragma unroll
-          for (int b = 0; b < 5; b++) tm[b * kTermRow + lane] = (al[t] & (1u << b)) ? q[b] : 0.0;
-        }
-      }
-      wave_sync();
-      // lanes of idle tasks add stale columns; their sums are not used
-      if (sum_lane) acc = sum_chunk(acc, my_col, min(kTermCols, n - c0));
-      wave_sync();
-    }
-    if (sum_lane) W->sum[my_t][my_b] = acc;
-    wave_sync();
-    // update, lane 5t+b for allele b of task t
-    if (sum_lane) {
-      const int mst = W->state[my_t];
-      if (mst == kTaskLast) {
-        if (my_b == 0) {
-          res_out[W->res[my_t]] = acc;
-          W->state[my_t] = kTaskIdle;
-        }
-      } else if (mst == kTaskIter) {
-        const double fo = W->f[my_t][my_b];
-        const double mine = W->sum[my_t][my_b];
-        double fn = fo;
-        bool upd = false;
-        if (W->mode[my_t] == 1) {
-          upd = (W->allowed[my_t] >> my_b) & 1u;
-          // one correctly rounded division: a reciprocal hoisted out of the pass loop would be
-          // spilled to scratch under this function's register budget
-          if (upd) fn = mine / (double)n;
-        } else {
-          const int v = W->v[my_t];
-          const double x = W->x[my_t];
-          double others = 0.0;
-#pragma unroll
-          for (int b = 0; b < 5; b++)
-            if (b != v) others += W->sum[my_t][b];
-          upd = my_b != v;
-          if (upd) fn = (others > 0.0) ? SharedDiv(others)((1.0 - x) * mine) : (1.0 - x) / 4.0;
-        }
-        W->fl[my_t][my_b] = fo;
-        W->f[my_t][my_b] = fn;
-        W->delta[my_t][my_b] = upd ? fabs(fn - fo) : 0.0;
+        target = ((side == 0) ? m_hi : m_lo) - kDrop;   // the ML frequency is the inner end
       }
     }
-    wave_sync();
-    if (lane < kTW && W->state[lane] == kTaskIter) {
-      double max_delta = 0.0;
-#pragma unroll
-      for (int b = 0; b < 5; b++) max_delta = fmax(max_delta, W->delta[lane][b]);
-      const int it = W->it[lane] + 1;
-      W->it[lane] = it;
-      if (max_delta < tol || it >= 50) W->state[lane] = kTaskLast;
-    }
-    wave_sync();
+    const double y = m + d0 + (hi > lo ? (d1 - d0) * ((x - lo) / (hi - lo)) : 0.0);
+    // lower bound: the profile rises towards the ML frequency; upper bound: it falls away from it
+    const bool before = (side == 0) ? (y < target) : (y >= target);
+    const uint32_t half = (uint32_t)(__ballot(before) >> (32 * side));
+    int c = __popc(half);
+    c = min(max(c, 1), 31);
+    va = __shfl(y, 32 * side + c - 1, 64);
+    vb = __shfl(y, 32 * side + c, 64);
+    const double na = a + (b - a) * ((double)(c - 1) * (1.0 / 31.0)), nb = a + (b - a) * ((double)c * (1.0 / 31.0));
+    a = na;
+    b = nb;
   }
+  const double t = (target - va) / (vb - va);
+  return a + (b - a) * ((t >= 0.0 && t <= 1.0) ? t : 0.5);
 }
 
-__device__ __noinline__ double log_choose(double n, double k) { return lgamma(n + 1) - lgamma(k + 1) - lgamma(n - k + 1); }
+__device__ __noinline__ double lgamma_w(double x) { return lgamma(x); }
 
-// fisher_exact_test_2x2 (stats.cpp:2144-2169): terms across lanes, summed in order by lane 0.
-__device__ __noinline__ double fisher_2x2_w(uint32_t a, uint32_t b, uint32_t c, uint32_t d, LdsDouble* buf) {
+// fisher_exact_test_2x2 (stats.cpp:2144-2169) and the logarithm of KS's lattice count: terms across
+// lanes, summed in order by lane 0.  The nine logarithms of factorials that every lane needs (and
+// three for KS) are one lgamma evaluated on twelve lanes, and the four that a term needs of its own
+// one each: an lgamma is some thousand cycles, and the chain of eighteen was the longest part of
+// the statistics.  log C(n, k) is lgamma(n + 1) - lgamma(k + 1) - lgamma(n - k + 1), as the reference
+// forms it.
+//   choose_ks: returns log C(ks_n, ks_k) too
+__device__ __noinline__ double fisher_2x2_w(uint32_t a, uint32_t b, uint32_t c, uint32_t d, LdsDouble* buf, uint32_t ks_n,
+                                            uint32_t ks_k, LdsDouble* choose_ks) {
   const int lane = threadIdx.x & 63;
   const uint32_t row1 = a + b, row2 = c + d, col1 = a + c, col2 = b + d;
   const uint32_t n = row1 + row2;
   const uint32_t a_min = (row1 > col2) ? (row1 - col2) : 0;
   const uint32_t a_max = min(row1, col1);
-  const double log_denom = log_choose(n, row1);
-  const double lpo = log_choose(col1, a) + log_choose(col2, row1 - a) - log_denom;
+  // arguments as the reference's doubles: whole numbers, exact
+  double arg = 1.0;
+  if (lane == 0) arg = (double)n + 1;
+  if (lane == 1) arg = (double)row1 + 1;
+  if (lane == 2) arg = (double)n - (double)row1 + 1;
+  if (lane == 3) arg = (double)col1 + 1;
+  if (lane == 4) arg = (double)a + 1;
+  if (lane == 5) arg = (double)col1 - (double)a + 1;
+  if (lane == 6) arg = (double)col2 + 1;
+  if (lane == 7) arg = (double)(row1 - a) + 1;
+  if (lane == 8) arg = (double)col2 - (double)(row1 - a) + 1;
+  if (lane == 9) arg = (double)ks_n + 1;
+  if (lane == 10) arg = (double)ks_k + 1;
+  if (lane == 11) arg = (double)ks_n - (double)ks_k + 1;
+  const double lg = lgamma_w(arg);
+  if (lane == 0) *choose_ks = readlane_d(lg, 9) - readlane_d(lg, 10) - readlane_d(lg, 11);
+  const double g_col1 = readlane_d(lg, 3), g_col2 = readlane_d(lg, 6);
+  const double log_denom = readlane_d(lg, 0) - readlane_d(lg, 1) - readlane_d(lg, 2);
+  const double lpo = (g_col1 - readlane_d(lg, 4) - readlane_d(lg, 5)) + (g_col2 - readlane_d(lg, 7) - readlane_d(lg, 8)) - log_denom;
   const double lre = log(1.0 + 1e-7);
   double total = 0.0;
   for (uint32_t base = a_min; base <= a_max; base += 64) {
-    const uint32_t ai = base + (uint32_t)lane;
-    double t = 0.0;
-    if (ai <= a_max) {
-      const double lp = log_choose(col1, ai) + log_choose(col2, row1 - ai) - log_denom;
-      if (lp <= lpo + lre) t = exp(lp);
-    }
-    buf[lane] = t;
+    const uint32_t ai = min(base + (uint32_t)lane, a_max);
+    const double l1 = g_col1 - lgamma_w((double)ai + 1) - lgamma_w((double)col1 - (double)ai + 1);
+    const double l2 = g_col2 - lgamma_w((double)(row1 - ai) + 1) - lgamma_w((double)col2 - (double)(row1 - ai) + 1);
+    const double lp = l1 + l2 - log_denom;
+    buf[lane] = (lp <= lpo + lre) ? exp(lp) : 0.0;
     wave_sync();
     if (lane == 0) {
       const uint32_t m = min<uint32_t>(64u, a_max - base + 1u);
@@ -456,28 +749,35 @@ __device__ __noinline__ double fisher_2x2_w(uint32_t a, uint32_t b, uint32_t c, 
 }
 
 // ks_test_two_sample_less (stats.cpp:2190-2284) from per-quality histograms of x (minor allele) and
-// y (major allele); pooled ties are whole quality values.
-__device__ __noinline__ double ks_less_w(LdsShared* SS, uint32_t nx, uint32_t ny) {
+// y (major allele); pooled ties are whole quality values.  log_total: log C(nx + ny, ny).
+__device__ __noinline__ double ks_less_w(LdsShared* SS, uint32_t nxv, uint32_t nyv, double log_total) {
   const int lane = threadIdx.x & 63;
-  const LdsU32* hx = SS->qh[0];
-  const LdsU32* hy = SS->qh[1];
-  // statistic and the counts at its minimum (lane-redundant: 128 steps)
-  uint32_t cx = 0, cy = 0, bx = 0, by = 0;
-  double min_z = 0.0;
-  bool have = false;
-#pragma unroll 1
-  for (int v = 0; v < 128; v++) {
-    if (hx[v] == 0 && hy[v] == 0) continue;
-    cx += hx[v];
-    cy += hy[v];
-    const double z = (double)cx / nx - (double)cy / ny;
-    if (!have || z < min_z) {
-      min_z = z;
-      have = true;
-      bx = cx;
-      by = cy;
+  const uint32_t nx = (uint32_t)uniform_i((int)nxv), ny = (uint32_t)uniform_i((int)nyv);
+  // the counts up to qualities 2 * lane and 2 * lane + 1
+  const uint32_t hx0 = SS->qh[0][2 * lane], hx1 = SS->qh[0][2 * lane + 1];
+  const uint32_t hy0 = SS->qh[1][2 * lane], hy1 = SS->qh[1][2 * lane + 1];
+  uint32_t cx1 = hx0 + hx1, cy1 = hy0 + hy1;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t ux = __shfl_up(cx1, o, 64), uy = __shfl_up(cy1, o, 64);
+    if (lane >= o) {
+      cx1 += ux;
+      cy1 += uy;
     }
   }
+  const uint32_t cx0 = cx1 - hx1, cy0 = cy1 - hy1;
+  // the statistic: the least z over the qualities that occur, the first of equal ones
+  const bool on0 = hx0 + hy0 != 0, on1 = hx1 + hy1 != 0;
+  const double z0 = on0 ? (double)cx0 / nx - (double)cy0 / ny : INFINITY;
+  const double z1 = on1 ? (double)cx1 / nx - (double)cy1 / ny : INFINITY;
+  const double z = (z1 < z0) ? z1 : z0;
+  const uint32_t zx = (z1 < z0) ? cx1 : cx0, zy = (z1 < z0) ? cy1 : cy0;
+  double min_z = z;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) min_z = fmin(min_z, __shfl_xor(min_z, o, 64));
+  const int at = __builtin_ctzll(__ballot(z == min_z) | (1ull << 63));
+  const uint32_t bx = (uint32_t)__builtin_amdgcn_readlane((int)zx, at), by = (uint32_t)__builtin_amdgcn_readlane((int)zy, at);
+  min_z = readlane_d(min_z, 0);
   const double stat = -min_z;
   if ((double)nx * ny >= 10000) {
     const double neff = ((double)nx * ny) / (nx + ny);
@@ -490,52 +790,67 @@ __device__ __noinline__ double ks_less_w(LdsShared* SS, uint32_t nx, uint32_t ny
   if (min(m, n) > (uint32_t)kKsDiag || D > 10000u) return __longlong_as_double(0x7ff8000000000000LL);
   // boundary(d): d is 0 or the pooled count at the end of a tie group
   const uint32_t nw = D / 32 + 1;
-  for (uint32_t k = lane; k < nw; k += 64) SS->ks_bnd[k] = 0;
+  for (uint32_t k = lane; k < nw; k += 64) SS->ks_bnd[k] = (k == 0) ? 1u : 0u;
   wave_sync();
-  if (lane == 0) {
-    SS->ks_bnd[0] |= 1u;
-    uint32_t cum = 0;
-#pragma unroll 1
-    for (int v = 0; v < 128; v++) {
-      const uint32_t g = hx[v] + hy[v];
-      if (!g) continue;
-      cum += g;
-      SS->ks_bnd[cum >> 5] |= 1u << (cum & 31);
-    }
-  }
+  if (on0) __hip_atomic_fetch_or(&SS->ks_bnd[(cx0 + cy0) >> 5], 1u << ((cx0 + cy0) & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (on1) __hip_atomic_fetch_or(&SS->ks_bnd[(cx1 + cy1) >> 5], 1u << ((cx1 + cy1) & 31), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   wave_sync();
   // the diagonal index runs over the smaller dimension
   const bool by_i = (m <= n);
   const uint32_t small = by_i ? m : n, large = by_i ? n : m;
-  LdsDouble* A = SS->ks_a;   // diagonal d-1
-  LdsDouble* B = SS->ks_b;   // diagonal d
-  for (uint32_t d = 0; d <= D; d++) {
-    const bool bnd = (SS->ks_bnd[d >> 5] >> (d & 31)) & 1u;
-    const uint32_t s_lo = (d > large) ? d - large : 0u;
-    const uint32_t s_hi = min(small, d);
-    for (uint32_t s = s_lo + lane; s <= s_hi; s += 64) {
-      const uint32_t i = by_i ? s : d - s;
-      const uint32_t j = by_i ? d - s : s;
-      double val;
-      if (d == 0) {
-        val = 1.0;
-      } else {
-        // u[i-1][j] + u[i][j-1], both on diagonal d-1
-        const double up = (i > 0) ? A[by_i ? s - 1 : s] : 0.0;
-        const double left = (j > 0) ? A[by_i ? s : s - 1] : 0.0;
-        val = up + left;
+  double umn;
+  if (small < 64u) {
+    // A diagonal in registers, cell s on lane s: a cell is its own and the lane before's value on the
+    // diagonal before.  A cell that does not exist yet is 0; one that has left the lattice is not
+    // read again by a cell inside it.
+    const int32_t ti = (int32_t)thr;
+    double u = (lane == 0) ? 1.0 : 0.0;
+    int32_t lvl = by_i ? lane * (int32_t)(n + m) : -lane * (int32_t)(n + m);   // i*n - j*m on diagonal 0
+    const int32_t step = by_i ? -(int32_t)m : (int32_t)n;
+    uint32_t word = 0;
+    for (uint32_t d = 0; d <= D; d++) {
+      if ((d & 31u) == 0) word = (uint32_t)uniform_i((int)SS->ks_bnd[d >> 5]);
+      if (d > 0) {
+        const long long bits = __double_as_longlong(u);
+        const int lo = __builtin_amdgcn_mov_dpp((int)(bits & 0xffffffffLL), 0x138, 0xf, 0xf, true);   // wave_shr:1
+        const int hi = __builtin_amdgcn_mov_dpp((int)(bits >> 32), 0x138, 0xf, 0xf, true);
+        u = __longlong_as_double(((long long)hi << 32) | (unsigned int)lo) + u;
       }
-      const int64_t lvl = (int64_t)i * n - (int64_t)j * m;
-      if (lvl >= thr && bnd) val = 0.0;
-      B[s] = val;
+      if (((word >> (d & 31u)) & 1u) && lvl >= ti) u = 0.0;
+      lvl += step;
     }
-    wave_sync();
-    LdsDouble* t = A;
-    A = B;
-    B = t;
+    umn = readlane_d(u, (int)small);
+  } else {
+    LdsDouble* A = SS->ks_a;   // diagonal d-1
+    LdsDouble* B = SS->ks_b;   // diagonal d
+    for (uint32_t d = 0; d <= D; d++) {
+      const bool bnd = (SS->ks_bnd[d >> 5] >> (d & 31)) & 1u;
+      const uint32_t s_lo = (d > large) ? d - large : 0u;
+      const uint32_t s_hi = min(small, d);
+      for (uint32_t s = s_lo + lane; s <= s_hi; s += 64) {
+        const uint32_t i = by_i ? s : d - s;
+        const uint32_t j = by_i ? d - s : s;
+        double val;
+        if (d == 0) {
+          val = 1.0;
+        } else {
+          // u[i-1][j] + u[i][j-1], both on diagonal d-1
+          const double up = (i > 0) ? A[by_i ? s - 1 : s] : 0.0;
+          const double left = (j > 0) ? A[by_i ? s : s - 1] : 0.0;
+          val = up + left;
+        }
+        const int64_t lvl = (int64_t)i * n - (int64_t)j * m;
+        if (lvl >= thr && bnd) val = 0.0;
+        B[s] = val;
+      }
+      wave_sync();
+      LdsDouble* t = A;
+      A = B;
+      B = t;
+    }
+    umn = A[small];
   }
-  const double umn = A[by_i ? m : n];
-  const double total = exp(log_choose(m + n, m));
+  const double total = exp(log_total);
   const double pv = 1.0 - umn / total;
   return fmin(fmax(pv, 0.0), 1.0);
 }
@@ -546,56 +861,6 @@ __device__ __noinline__ void pure_genotype_call(const double* lps, uint32_t n, i
   double l[5];
   for (int b = 0; b < 5; b++) l[b] = lps[b];
   pure_genotype(l, n, *best, *score);
-}
-
-// Relative entropy KL(fh || f) of two-allele frequencies: the drop of a binomial log likelihood
-// from its maximum at fh, per read and in natural-log units.
-__device__ double kl_two(double fh, double f) {
-  double t = 0.0;
-  if (fh > 0.0) t += fh * (log(fh) - log(f));
-  if (fh < 1.0) t += (1.0 - fh) * (log1p(-fh) - log1p(-f));
-  return t;
-}
-
-// Predicted crossing point of the profile likelihood with the target inside [lo, hi] (bound
-// `side`: 0 lower, 1 upper), used only to choose which midpoints to evaluate.  Model:
-// profile(f) = vmax - A * KL(fh || f) + c, fitted to the interval ends whose values are known and
-// interior (two ends: A and c; one end: A; none: A = n / ln 10, the binomial curvature of n reads).
-__device__ __noinline__ double predict_crossing(int side, double lo, double hi, double vlo, double vhi, double fh,
-                                                double vmax, double target, int n) {
-  double xs[2], vs[2];
-  int k = 0;
-  if (lo != fh && lo > 0.0 && lo < 1.0 && isfinite(vlo)) {
-    xs[k] = lo;
-    vs[k++] = vlo;
-  }
-  if (hi != fh && hi > 0.0 && hi < 1.0 && isfinite(vhi)) {
-    xs[k] = hi;
-    vs[k++] = vhi;
-  }
-  double A = (double)n / 2.302585092994046, c = 0.0;
-  if (k == 2) {
-    const double d0 = kl_two(fh, xs[0]), d1 = kl_two(fh, xs[1]);
-    if (d1 != d0) {
-      A = (vs[0] - vs[1]) / (d1 - d0);
-      c = vs[0] + A * d0 - vmax;
-    }
-  } else if (k == 1) {
-    const double d = kl_two(fh, xs[0]);
-    if (d > 0.0) A = (vmax - vs[0]) / d;
-  }
-  const double want = (vmax - target + c) / A;
-  if (!(A > 0.0) || !isfinite(want)) return 0.5 * (lo + hi);
-  // KL grows away from fh: falls across the lower interval, rises across the upper one.  20 halvings
-  // place the crossing within 2^-20 of the interval, far finer than the eight levels a round uses.
-  double a = lo, b = hi;
-  for (int it = 0; it < 20; it++) {
-    const double m = 0.5 * (a + b);
-    const bool beyond = kl_two(fh, m) > want;   // m lies outside the crossing (farther from fh)
-    if ((side == 0) == beyond) a = m;
-    else b = m;
-  }
-  return 0.5 * (a + b);
 }
 
 // allele_model::major_index / next_index (identify_mutations.cpp:3061-3086)
@@ -619,45 +884,145 @@ __device__ __forceinline__ int next_index(const double f[5], uint32_t n, int exc
   return best;
 }
 
+// KS quality and Fisher strand p values of the entry (annotate_polymorphism_statistics,
+// identify_mutations.cpp:3009-3033), by one wavefront.
+// key_of, reads: the distinct keys and their reads, or (null) every one of the K list entries a key.
+__device__ __noinline__ void stats_w(LdsShared* SS, const uint32_t* list, const uint32_t* key_of, const uint32_t* reads, int K,
+                                     int Q, int major, int minor) {
+  const int lane = threadIdx.x & 63;
+  for (int i = lane; i < 256; i += 64) (&SS->qh[0][0])[i] = 0;
+  wave_sync();
+  uint32_t nx = 0, ny = 0;
+  for (int i = lane; i < K; i += 64) {
+    const uint32_t k = key_of ? key_of[i] : list[i];
+    const uint32_t h = key_of ? reads[i] : 1u;
+    const int ob = (int)((k % 10u) / 2u);
+    const int q = (int)((k / 10u) % (uint32_t)Q);
+    if (ob == major && q < 128) {
+      __hip_atomic_fetch_add(&SS->qh[1][q], h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      ny += h;
+    }
+    if (ob == minor && q < 128) {
+      __hip_atomic_fetch_add(&SS->qh[0][q], h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      nx += h;
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    nx += __shfl_xor(nx, o, 64);
+    ny += __shfl_xor(ny, o, 64);
+  }
+  wave_sync();
+  const uint32_t mjt = (major < 5) ? SS->cov[major][2] : 0, mjb = (major < 5) ? SS->cov[major][0] : 0;
+  const uint32_t mnt = (minor < 5) ? SS->cov[minor][2] : 0, mnb = (minor < 5) ? SS->cov[minor][0] : 0;
+  const double fs = fisher_2x2_w(mnt, mnb, mjt, mjb, SS->fisher, nx + ny, ny, &SS->ks_log_total);
+  wave_sync();
+  const double ks = (nx > 0 && ny > 0) ? ks_less_w(SS, nx, ny, SS->ks_log_total) : 1.0;
+  if (lane == 0) {
+    SS->ks_p = ks;
+    SS->fisher_p = fs;
+  }
+}
+
+// Whether a value known to kGuardRel prints as the reference's: %.*e with `places` digits, whose
+// rounding boundary must not lie within the error.  A decade's end is no boundary: both sides of it
+// print alike.
+__device__ __noinline__ bool prints_surely_e(double v, int places) {
+  if (v == 0.0) return true;
+  if (!(v > 1e-280) || places > 12) return false;
+  const double e = floor(log10(v));
+  const double scaled = v * pow(10.0, (double)places - e);
+  return fabs(scaled - floor(scaled) - 0.5) > 2.0 * kGuardRel * scaled;
+}
+
+// The same of a score known to kGuardLog, printed with one decimal.
+__device__ __forceinline__ bool prints_surely_f1(double v) {
+  const double scaled = 10.0 * fabs(v);
+  return fabs(scaled - floor(scaled) - 0.5) > 10.0 * kGuardLog;
+}
+
+// Whether the full fit's decisions (which alleles count, and their order) hold for any frequencies
+// within kGuardRel of these, and the frequencies that are printed print alike.
+__device__ __noinline__ bool fit_is_sure(const LdsDouble* f, uint32_t n, int places) {
+  const double thr = 0.5 / (double)n;
+  for (int a = 0; a < 5; a++) {
+    if (f[a] < fmin(0.5 * thr, 0.01)) continue;
+    if (fabs(f[a] - thr) <= 4.0 * kGuardRel * thr) return false;
+    for (int b = 0; b < a; b++)
+      if (fabs(f[a] - f[b]) <= 4.0 * kGuardRel * f[a]) return false;
+    if (f[a] >= thr && !prints_surely_e(f[a], places)) return false;
+  }
+  return true;
+}
+
+// The search of one bound (write_RA_frequency_bounds, identify_mutations.cpp:3175-3217), in
+// registers of the lane that walks it.
+struct Bound {
+  double lo, hi, vlo, vhi;
+  double out;       // the bound as reported so far
+  int active;       // 0 ended, 1 between midpoints, 2 its end of the range is still to be compared
+  int iter;
+  // One comparison with the target: at the end of the range, which opens the search when the profile
+  // there is below the target, or at the midpoint m of the interval.
+  __device__ __forceinline__ void step(int side, bool ge, double m, double v, double tol, double fh) {
+    if (active == 2) {
+      active = (!ge && (hi - lo) > tol) ? 1 : 0;
+      if (!ge) out = fh;
+      return;
+    }
+    // lower bound: a profile >= target moves hi down; upper bound: it moves lo up
+    const bool left = (side == 0) ? ge : !ge;   // the interval kept is [lo, m]
+    if (left) {
+      hi = m;
+      vhi = v;
+    } else {
+      lo = m;
+      vlo = v;
+    }
+    iter++;
+    active = (iter < 40 && (hi - lo) > tol) ? 1 : 0;
+    out = (side == 0) ? hi : lo;
+  }
+};
+
 }  // namespace
 
 // kKeysGlobal: the candidate's read list is this block's slice of a device scratch list (columns
-// too deep for LDS; the table-row cache then takes all of the dynamic LDS), else it is in LDS.  The
-// location is a compile-time choice, so that each instantiation's accesses to the list keep their
-// address space (LDS instructions in the usual case); one pointer that may be either would make
-// them all generic (flat) accesses.
+// too deep for LDS), else it is in LDS.  The location is a compile-time choice, so that each
+// instantiation's accesses to the list keep their address space (LDS instructions in the usual
+// case); one pointer that may be either would make them all generic (flat) accesses.
 template <bool kKeysGlobal>
-__global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(3))) k_score_candidates_t(ImParams P) {
+__global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4))) k_score_candidates_t(ImParams P) {
   extern __shared__ __align__(16) unsigned char dyn[];
-  uint32_t* keys;
+  uint32_t* list;   // the candidate's reads, in order: table keys, then rows
   size_t key_lds;
   if constexpr (kKeysGlobal) {
-    keys = P.key_scratch + (size_t)blockIdx.x * (size_t)P.key_cap;
+    list = P.key_scratch + (size_t)blockIdx.x * (size_t)P.key_cap;
     key_lds = 0;
   } else {
-    keys = (uint32_t*)dyn;
+    list = (uint32_t*)dyn;
     key_lds = ((size_t)P.key_cap * sizeof(uint32_t) + 15) & ~(size_t)15;
   }
+  // P.rows_cap rows (six doubles each), the same with the variant first (em_tasks), their two model
+  // values, their keys and reads; before the rows are filled, a count and then a row number per table
+  // key lie in their place
   double* rows = (double*)(dyn + key_lds);
+  double* prow = rows + (size_t)P.rows_cap * 6;
+  double* pre = prow + (size_t)P.rows_cap * 6;
+  uint32_t* key_of = (uint32_t*)(pre + (size_t)P.rows_cap * 2);
+  uint32_t* row_reads = key_of + P.rows_cap;
+  uint32_t* row_of = (uint32_t*)rows;
+  const bool direct = (size_t)P.tab_keys * sizeof(uint32_t) <= (size_t)P.rows_cap * 96;
+  constexpr bool kLG = kKeysGlobal;
   __shared__ ScoreShared SS;
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  LdsTasks* W = (LdsTasks*)&SS.wt[wave];
-  LdsDouble* term = &W->term[0][0][0];
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int S = P.read_set_max, Q = P.quality_max;
   const double tol = P.precision_decimal;
-  const double kDrop = 0.587566;   // kProfileLikelihoodLog10Drop (identify_mutations.cpp:3173)
-  const int n_cand = min(*P.n_cand, P.cand_cap);
-  // With many more candidates than resident blocks the pass is bound by total work, not by one
-  // candidate's chain: the null fit then runs alone first, and only candidates that are emitted go on
-  // to the profile likelihoods and bisections (one phase more on their chain).  With few, all of
-  // phase 1 runs together.
-  const bool two_stage = n_cand > 2 * (int)gridDim.x;
-  const int prof_ph = two_stage ? 2 : 1;   // the phase of the profile likelihoods and first path levels
+  const int n_cand = min(*P.n_score, P.cand_cap);
   uint32_t err = 0;
   // Blocks take candidates from the pass's work counter, one at a time: a candidate's cost varies
-  // several-fold (emitted ones go on to the profiles and bisections), so a fixed stride over the
-  // grid would leave blocks idle while others work through a run of costly candidates.
+  // several-fold, so a fixed stride over the grid would leave blocks idle while others work through a
+  // run of costly candidates.
   __shared__ int s_next;
   for (;;) {
     if (tid == 0) s_next = atomicAdd(P.score_next, 1);
@@ -670,7 +1035,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(3
     // as wave-uniform scalars, so the checks are uniform branches: a skip decided on per-lane
     // copies of the same value is a divergent branch to the compiler, and around the block's
     // barriers that has paired barriers across wavefronts wrongly (results read stale LDS).
-    const int2 cd0 = P.cand[ci];
+    const int2 cd0 = P.score[ci];
     const int2 cd = make_int2(__builtin_amdgcn_readfirstlane(cd0.x), __builtin_amdgcn_readfirstlane(cd0.y));
     if (cd.x < 0 || cd.x >= P.n_pos || cd.y < 0) {
       err |= kErrIndex;
@@ -688,7 +1053,14 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(3
       continue;
     }
     if (tid < 18) SS.cov[tid / 3][tid % 3] = 0;
-    if (tid == 0) SS.n_keys = 0;
+    if (tid == 0) {
+      SS.n_keys = 0;
+      SS.bad_r = 0;
+      SS.unsure = 0;
+      SS.best = -1;    // not computed yet
+      SS.ks_p = 2.0;   // not computed yet
+      SS.fisher_p = 1.0;
+    }
     __syncthreads();
     // ---- pdata in file order (identify_mutations.cpp:1561-1657): order-preserving compaction
     for (int r0 = rb; r0 < re; r0 += kSW * 64) {
@@ -711,7 +1083,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(3
       }
       if (use) {
         const int idx = base + __popcll(mask & ((1ull << lane) - 1ull));
-        if (idx < P.key_cap) keys[idx] = key;
+        if (idx < P.key_cap) list[idx] = key;
         else err |= kErrCapacity;
         atomicAdd(&SS.cov[obs][strand_idx], 1u);
       }
@@ -723,305 +1095,393 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(3
       }
       __syncthreads();
     }
-    const int n = min(SS.n_keys, P.key_cap);
+    const int n = __builtin_amdgcn_readfirstlane(min(SS.n_keys, P.key_cap));
     if (tid < 5) SS.obs[tid] = SS.cov[tid][0] + SS.cov[tid][2];
-    // ---- table rows of the reads, cached in LDS
-    const bool cached = n <= P.rows_cap;
-    if (cached)
-      for (int i = tid; i < n * 6; i += kSW * 64) rows[i] = P.tab_r[(size_t)keys[i / 6] * 6 + i % 6];
-    if (tid == 0) {
-      SS.done = 0;
-      SS.emitted = 0;
-      SS.active[0] = SS.active[1] = 0;
-      SS.depth[0] = SS.depth[1] = 0;
-      SS.path[0] = SS.path[1] = 0;
-      SS.tree_only[0] = SS.tree_only[1] = 0;
-      SS.lower = 0.0;
-      SS.upper = 1.0;
-      SS.ks_p = 1.0;
-      SS.fisher_p = 1.0;
+    // ---- the distinct keys: counted per table key, numbered in key order by a block scan.  A
+    // table too large for that keeps a row per read.
+    int K = n;
+    bool dedup = false;
+    if (direct) {
+      for (int i = tid; i < P.tab_keys; i += kSW * 64) row_of[i] = 0;
+      __syncthreads();
+      for (int i = tid; i < n; i += kSW * 64) atomicAdd(&row_of[list[i]], 1u);
+      __syncthreads();
+      const int per = (P.tab_keys + kSW * 64 - 1) / (kSW * 64);
+      const int k0 = min(tid * per, P.tab_keys), k1 = min(k0 + per, P.tab_keys);
+      int mine = 0;
+      for (int k = k0; k < k1; k++) mine += row_of[k] ? 1 : 0;
+      int incl = mine;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += u;
+      }
+      if (lane == 63) SS.wcount[wave] = (uint32_t)incl;
+      __syncthreads();
+      int at = incl - mine;
+      K = 0;
+      for (int k = 0; k < kSW; k++) {
+        if (k < wave) at += (int)SS.wcount[k];
+        K += (int)SS.wcount[k];
+      }
+      K = uniform_i(K);
+      dedup = K <= P.rows_cap;
+      if (dedup) {
+        for (int k = k0; k < k1; k++)
+          if (row_of[k]) {
+            key_of[at] = (uint32_t)k;
+            row_reads[at] = row_of[k];
+            row_of[k] = (uint32_t)at++;
+          }
+        __syncthreads();
+        for (int i = tid; i < n; i += kSW * 64) list[i] = row_of[list[i]];
+      }
+    }
+    const int kind = (dedup || n <= P.rows_cap) ? kRowsLds : kRowsGlobal;
+    if (!dedup) {
+      K = n;
+      if (kind == kRowsLds)
+        for (int i = tid; i < n; i += kSW * 64) {
+          key_of[i] = list[i];
+          row_reads[i] = 1u;
+          list[i] = (uint32_t)i;
+        }
     }
     __syncthreads();
-    Rows RR;
-    RR.lds = cached ? rows : nullptr;
-    RR.keys = keys;
-    RR.tab_r = P.tab_r;
+    bool bad_r = false;
+    const int n_check = (kind == kRowsLds) ? K * 6 : P.tab_keys * 6;
+    for (int i = tid; i < n_check; i += kSW * 64) {
+      const double r = P.tab_r[kind == kRowsLds ? (size_t)key_of[i / 6] * 6 + i % 6 : (size_t)i];
+      if (kind == kRowsLds) rows[i] = r;
+      bad_r = bad_r || (i % 6 != 5 && r != 0.0 && !(r >= 0x1p-100 && r <= 2.0));
+    }
+    if (bad_r) SS.bad_r = 1;
+    const Rows RR{list, rows, row_reads, P.tab_r};
+    const uint32_t* keys = (kind == kRowsLds) ? key_of : nullptr;
+    auto fit_exact = [&](int mode, int v, double x) {
+      return kind == kRowsLds ? em_exact<kRowsLds, kLG>(RR, n, mode, v, x, (LdsDouble*)SS.fit, tol, SS.bad_r)
+                              : em_exact<kRowsGlobal, kLG>(RR, n, mode, v, x, (LdsDouble*)SS.fit, tol, SS.bad_r);
+    };
     const char refc = (slot == 0) ? P.ref[p] : '.';
     const int ref_idx = char_index(refc) < 0 ? 5 : char_index(refc);
+    __syncthreads();
+    // ---- the candidate, with sums in any order; then, when a decision or a printed digit lies too
+    // close to its boundary (or every candidate is to be exact), once more with the reference's sums
     int major = 5, minor = 5, variant = 5;
-    bool cons = false;
-    // ---- phases: each wavefront starts its tasks of the phase, then runs them to completion
-    for (int ph = 0;; ph++) {
-      {
-        // task slots of this wavefront for this phase, set up by every lane with the same values
-        // (identical LDS stores).  Kept out of a lane-0 branch on purpose: at the join of such a
-        // branch, ahead of the run_tasks call, the compiler has placed a register spill before the
-        // exec-mask restore, so the lanes outside the branch reloaded another value's slot; the
-        // build rejects that spill placement (build.py, spill_before_exec_restore).
-        int k = 0;
-        auto start = [&](int mode, uint32_t allowed, int v, double x, int res) {
-          task_start(W, k++, mode, allowed, v, x, res, (const LdsU32*)SS.obs, (const LdsDouble*)SS.full_f, n,
-                     (LdsDouble*)SS.res);
-        };
-        if (ph == 0) {
-          if (wave == 0) start(1, 31u, -1, 0.0, kResFull);
-        } else if (ph == 1 && two_stage) {
-          if (variant != 5 && n > 0 && wave == 0) start(1, 31u & ~(1u << variant), -1, 0.0, kResNull);
-        } else if (ph == prof_ph) {
-          if (variant != 5 && n > 0) {
-            // the first path levels of the bounds (lower bound's first) fill the slots that the
-            // four phase-1 tasks leave idle; plmax and p1 end after a pass or two and share a wave
-            auto spec_start = [&](int j) {
-              const int side = j < SS.spec[0] ? 0 : 1, level = side ? j - SS.spec[0] : j;
-              if (level < SS.spec[side]) start(2, 31u, variant, SS.pts[side][level], kResBisect + side * kBisectPts + level);
-            };
-            if (wave == 0) {
-              if (!two_stage) start(1, 31u & ~(1u << variant), -1, 0.0, kResNull);
-              spec_start(0);
-            } else if (wave == 1) {
-              start(2, 31u, variant, SS.full_f[variant], kResPlmax);
-              start(2, 31u, variant, 1.0, kResP1);
-            } else if (wave == 2) {
-              start(2, 31u, variant, 0.0, kResP0);
-              spec_start(1);
-            } else {
-              spec_start(2);
-              spec_start(3);
-            }
-          }
-        } else {
-          // one bound open: its midpoints on nodes 2w, 2w+1; both open: the lower bound's on
-          // wavefronts 0-1 and the upper bound's on wavefronts 2-3, nodes 2(w%2), 2(w%2)+1
-          const bool a0 = SS.active[0] != 0, a1 = SS.active[1] != 0;
-          if (a0 || a1) {
-            const int side = (a0 && a1) ? wave / 2 : (a0 ? 0 : 1);
-            const int n0 = (a0 && a1) ? 2 * (wave % 2) : 2 * wave;
-            const int npts = SS.path[side] ? SS.depth[side] : (1 << SS.depth[side]) - 1;
-            for (int node = n0; node < min(n0 + 2, npts); node++)
-              start(2, 31u, variant, SS.pts[side][node], kResBisect + side * kBisectPts + node);
-          }
-        }
-        for (; k < kTW; k++) W->state[k] = kTaskIdle;
-      }
-      wave_sync();
-      run_tasks(RR, n, W, tol, (LdsDouble*)SS.res);
-      if (ph == 0 && wave == 0 && lane < 5) SS.full_f[lane] = W->f[0][lane];
-      if (ph == 0 && wave == 1) {
-        // pure_genotype_call on the summed likelihoods of the same reads, in read order
-        // (identify_mutations.cpp:1669-1689, 3398-3433)
-        double acc = 0.0;
-        for (int c0 = 0; c0 < n; c0 += kTermCols) {
-          if (c0 + lane < n) {
-            const double* lp = P.tab_lp + (size_t)keys[c0 + lane] * 5;
+    bool have_v = false;
+    // level 0: sums in any order; 1: the full fit and close comparisons with the reference's sums; 2: the
+    // score's likelihoods too
+    for (int level = (P.screen_off || kind != kRowsLds) ? 2 : 0;;) {
+      const bool in_order = level > 0;
+      if (wave == 0) {
+        // full fit, from 0.5 + one per observing read, normalized (identical values from every lane)
+        double f[5], total = 0.0;
 #pragma unroll
-            for (int b = 0; b < 5; b++) term[b * kTermRow + lane] = lp[b];
-          }
-          wave_sync();
-          if (lane < 5) acc = sum_in_order(acc, term + lane * kTermRow, min(kTermCols, n - c0));
-          wave_sync();
-        }
-        if (lane < 5) SS.lps[lane] = acc;
-      }
-      if (ph == prof_ph && wave == 1) {
-        // annotate_polymorphism_statistics (identify_mutations.cpp:3009-3033); used if emitted
-        for (int i = lane; i < 256; i += 64) (&SS.qh[0][0])[i] = 0;
-        wave_sync();
-        uint32_t nx = 0, ny = 0;
-        for (int i = lane; i < n; i += 64) {
-          const uint32_t k = keys[i];
-          const int ob = (int)((k % 10u) / 2u);
-          const int q = (int)((k / 10u) % (uint32_t)Q);
-          if (ob == major && q < 128) {
-            atomicAdd(&SS.qh[1][q], 1u);
-            ny++;
-          }
-          if (ob == minor && q < 128) {
-            atomicAdd(&SS.qh[0][q], 1u);
-            nx++;
-          }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-          nx += __shfl_xor(nx, o, 64);
-          ny += __shfl_xor(ny, o, 64);
-        }
-        wave_sync();
-        const double ks = (nx > 0 && ny > 0) ? ks_less_w((LdsShared*)&SS, nx, ny) : 1.0;
-        const uint32_t mjt = (major < 5) ? SS.cov[major][2] : 0, mjb = (major < 5) ? SS.cov[major][0] : 0;
-        const uint32_t mnt = (minor < 5) ? SS.cov[minor][2] : 0, mnb = (minor < 5) ? SS.cov[minor][0] : 0;
-        const double fs = fisher_2x2_w(mnt, mnb, mjt, mjb, (LdsDouble*)SS.fisher);
-        if (lane == 0) {
-          SS.ks_p = ks;
-          SS.fisher_p = fs;
-        }
-      }
-      __syncthreads();
-      if (ph == 0) {
-        // every thread derives the same calls from the shared sums
-        double full_f[5], lps[5];
         for (int b = 0; b < 5; b++) {
-          full_f[b] = SS.full_f[b];
-          lps[b] = SS.lps[b];
+          f[b] = 0.5 + (double)SS.obs[b];
+          total += f[b];
         }
+#pragma unroll
+        for (int b = 0; b < 5; b++) SS.fit[b] = (n > 0) ? f[b] / total : 0.0;
+        wave_sync();
+        double ll = 0.0;
+        bool unsure = false;
+        if (n > 0) {
+          if (in_order) {
+            ll = fit_exact(1, -1, 0.0);
+          } else {
+            ll = em_full<kRowsLds>(RR, K, n, (LdsDouble*)SS.fit, tol);
+            unsure = !(fabs(ll) < 1e300);
+          }
+        }
+        wave_sync();
+        if (lane < 5) SS.full_f[lane] = SS.fit[lane];
+        if (lane == 0) {
+          if (level != 1) SS.full_ll = ll;   // level 1 keeps the value that goes with the null task's
+          SS.unsure = unsure ? 2 : 0;
+        }
+      } else if (wave == 1 && (level == 0 || SS.best < 0)) {
+        double lps[5];
+        genotype_sums<kLG>(list, keys, P.tab_lp, n, lps);
         int best;
         double gscore;
         pure_genotype_call(lps, (uint32_t)n, &best, &gscore);
-        const double cbs = gscore - P.log10_ref_length;
-        cons = (best != ref_idx) && !isnan(cbs) && (cbs > 0.0);
-        major = major_index(full_f, (uint32_t)n);
-        minor = next_index(full_f, (uint32_t)n, major);
-        variant = next_index(full_f, (uint32_t)n, ref_idx);
-        if (tid == 0) {
-          // the first levels of each bound's predicted path, evaluated speculatively in phase 1:
-          // four for a bound whose interval alone is wide enough to be searched, else two each
-          // (the model needs only the ML frequency and n until profile values are known)
-          SS.spec[0] = SS.spec[1] = 0;
-          if (variant != 5 && n > 0) {
-            const double fh = SS.full_f[variant];
-            const bool open0 = fh > tol, open1 = (1.0 - fh) > tol;
-            SS.spec[0] = open0 ? (open1 ? 2 : 4) : 0;
-            SS.spec[1] = open1 ? (open0 ? 2 : 4) : 0;
-            for (int side = 0; side < 2; side++) {
-              const double lo = side ? fh : 0.0, hi = side ? 1.0 : fh;
-              const double fs = predict_crossing(side, lo, hi, 0.0, 0.0, fh, kDrop, 0.0, n);
-              double a = lo, b = hi;
-              for (int d = 0; d < SS.spec[side]; d++) {
-                const double m = 0.5 * (a + b);
-                SS.pts[side][d] = m;
-                const bool left = (side == 0) ? (fs <= m) : (fs < m);
-                if (left) b = m;
-                else a = m;
+        if (lane == 0) {
+          SS.best = best;
+          SS.gscore = gscore;
+        }
+      }
+      __syncthreads();
+      // every thread derives the same calls from the shared results
+      bool cons;
+      {
+        double full_f[5];
+        for (int b = 0; b < 5; b++) full_f[b] = SS.full_f[b];
+        const double cbs = SS.gscore - P.log10_ref_length;
+        cons = (SS.best != ref_idx) && !isnan(cbs) && (cbs > 0.0);
+        major = uniform_i(major_index(full_f, (uint32_t)n));
+        minor = uniform_i(next_index(full_f, (uint32_t)n, major));
+        variant = uniform_i(next_index(full_f, (uint32_t)n, ref_idx));
+      }
+      have_v = variant != 5 && n > 0;
+      const double fh = have_v ? SS.full_f[variant] : 0.0;
+      double other = 0.0;   // the other alleles' share of the full fit
+#pragma unroll
+      for (int b = 0; b < 5; b++)
+        if (b != variant) other += SS.full_f[b];
+      if (have_v && kind == kRowsLds) {
+        for (int i = tid; i < K; i += kSW * 64) {
+          double r[6], t = 0.0;
+          RR.row<kRowsLds>(i, r);
+          int at = 1;
+#pragma unroll
+          for (int b = 0; b < 5; b++) {
+            const bool mine = b == variant;
+            prow[6 * i + (mine ? 0 : at)] = r[b];
+            if (!mine) {
+              t = fma((other > 0.0) ? SS.full_f[b] / other : 0.25, r[b], t);
+              at++;
+            }
+          }
+          prow[6 * i + 5] = (double)row_reads[i];
+          pre[2 * i] = rows[6 * i + variant] - t;
+          pre[2 * i + 1] = t;
+        }
+      }
+      if (tid == 0) {
+        SS.done = 0;
+        SS.emitted = 0;
+        SS.exact = SS.exact_have = 0;
+        SS.active[0] = SS.active[1] = 0;
+        SS.depth[0] = SS.depth[1] = 0;
+        SS.out[0] = 0.0;
+        SS.out[1] = 1.0;
+        if (!in_order && n > 0 && SS.unsure == 0 && !fit_is_sure((LdsDouble*)SS.full_f, (uint32_t)n, P.places)) SS.unsure = 1;
+      }
+      __syncthreads();
+      // ---- rounds: the null fit, the profiles at the ML frequency, 0 and 1 and the bounds' midpoints |
+      // KS and Fisher; then more midpoints.  Nothing of an unsure fit is worth going on with.
+      const bool go = uniform_i(SS.unsure) == 0;
+      for (int round = 0; go; round++) {
+        const int exact = uniform_i(SS.exact);
+        const bool search = round == 0 || SS.active[0] || SS.active[1];
+        if (have_v && wave == kTaskWaves && (exact || (level == 2 && round == 0))) {
+          // the null fit, or both sides of a comparison too close for the tasks' values
+          if (exact) {
+            for (int part = SS.exact_have ? 1 : 0; part < 2; part++) {
+              const double x = part ? SS.exact_x[exact - 1] : fh;
+#pragma unroll
+              for (int b = 0; b < 5; b++)
+                SS.fit[b] = (b == variant) ? x : (other > 0.0) ? (1.0 - x) * SS.full_f[b] / other : (1.0 - x) / 4.0;
+              wave_sync();
+              const double ll = fit_exact(2, variant, x);
+              wave_sync();
+              if (lane == 0) {
+                if (part) SS.exact_v = ll;
+                else SS.exact_target = ll - kDrop;
+              }
+            }
+          } else {
+            double f[5], total = 0.0;
+#pragma unroll
+            for (int b = 0; b < 5; b++) {
+              f[b] = (b == variant) ? 0.0 : 0.5 + (double)SS.obs[b];
+              total += f[b];
+            }
+#pragma unroll
+            for (int b = 0; b < 5; b++) SS.fit[b] = f[b] / total;
+            wave_sync();
+            const double ll = fit_exact(1, variant, 0.0);
+            if (lane == 0) SS.null_ll = ll;
+          }
+        }
+        if (!exact) {
+          if (wave == kTaskWaves) {
+            // annotate_polymorphism_statistics (identify_mutations.cpp:3009-3033); used if emitted
+            if (round == 0 && n > 0 && !(in_order && SS.ks_p != 2.0))
+              stats_w((LdsShared*)&SS, list, keys, row_reads, K, Q, major, minor);
+          } else if (have_v && search && kind == kRowsLds) {
+            // task slots of the round.  Round 0: the profiles at the ML frequency, 0 and 1 and the null
+            // fit, then the first path of each bound that may be searched.  Later: per open bound
+            // the first levels of the full tree, whatever the prediction, then a path.  A bound needs
+            // 20 levels at most for its 1e-6; with one open, 24 tasks of eight lanes hold them.
+            const int s0 = (round == 0) ? 4 : 0;
+            const bool open0 = (round == 0) ? fh > tol : SS.active[0] != 0;
+            const bool open1 = (round == 0) ? (1.0 - fh) > tol : SS.active[1] != 0;
+            const bool both = open0 && open1;
+            const int shift = both ? 2 : 3;   // lanes per task: 4 or 8
+            const int share = both ? (kTaskSlots - s0) / 2 : kTaskSlots / 2 - s0;
+            const int n_tree = (round == 0) ? 0 : 7;
+            const int side_l = lane >> 5;
+            const double lo_l = (round == 0) ? (side_l ? fh : 0.0) : SS.lo[side_l];
+            const double hi_l = (round == 0) ? (side_l ? 1.0 : fh) : SS.hi[side_l];
+            const LdsDouble *pr = (const LdsDouble*)prow, *pm = (const LdsDouble*)pre;
+            const double root = model_root(pr, pm, K, lo_l, hi_l, round > 0, SS.vlo[side_l], SS.vhi[side_l], SS.target);
+            const double root0 = readlane_d(root, 0), root1 = readlane_d(root, 32);
+            const int slot_i = (wave * 64 + lane) >> shift;
+            const bool first = (lane & ((1 << shift) - 1)) == 0;
+            double x = 0.0;
+            bool active = false;
+            const bool null_task = round == 0 && slot_i == 3;
+            if (slot_i < s0) {
+              x = (slot_i == 0) ? fh : (slot_i == 2) ? 1.0 : 0.0;
+              active = !(null_task && level == 2);
+            } else {
+              const int side = (open0 && slot_i - s0 < share) ? 0 : 1;
+              const int rel = slot_i - s0 - ((open0 && side == 1) ? share : 0);
+              if (rel < share && (side ? open1 : open0)) {
+                double a = (round == 0) ? (side ? fh : 0.0) : SS.lo[side], b = (round == 0) ? (side ? 1.0 : fh) : SS.hi[side];
+                const int it0 = (round == 0) ? 0 : SS.iter[side];
+                const double fs = side ? root1 : root0;
+                // a tree node's turns are the bits of its breadth-first number below the leading one,
+                // a path's those of the prediction
+                const bool tree = rel < n_tree;
+                const int node = rel + 1;
+                const int deep = tree ? 31 - __clz(node) : rel - n_tree;
+                double m = 0.5 * (a + b);
+                active = true;
+                for (int d = 0; d < deep; d++) {
+                  const bool left = tree ? !((node >> (deep - 1 - d)) & 1) : (side == 0) ? (fs <= m) : (fs < m);
+                  if (left) b = m;
+                  else a = m;
+                  if (!(it0 + d + 1 < 40 && (b - a) > tol)) active = false;
+                  m = 0.5 * (a + b);
+                }
+                x = m;
+                if (first) SS.pts[side][rel] = active ? m : -1.0;
+              }
+            }
+            if (tid == 0) {
+              SS.n_tree = n_tree;
+              for (int side = 0; side < 2; side++) {
+                SS.depth[side] = (side ? open1 : open0) ? share : 0;
+                SS.slot0[side] = s0 + ((side == 1 && open0) ? share : 0);
+              }
+            }
+            if (__any(active)) {
+              // the other alleles' starting frequencies, in order
+              double st[4], total = 0.0;
+              int at = 0;
+#pragma unroll
+              for (int b = 0; b < 5; b++) total += (b == variant) ? 0.0 : 0.5 + (double)SS.obs[b];
+#pragma unroll
+              for (int q = 0; q < 4; q++) {
+                at = q + (q >= variant ? 1 : 0);
+                st[q] = null_task ? (0.5 + (double)SS.obs[at]) / total
+                                  : (other > 0.0) ? (1.0 - x) * SS.full_f[at] / other : (1.0 - x) / 4.0;
+              }
+              const double sc = null_task ? 1.0 / (double)n : 0.0;
+              const double val = both ? em_tasks<4>(pr, K, x, st[0], st[1], st[2], st[3], sc, active, tol)
+                                      : em_tasks<8>(pr, K, x, st[0], st[1], st[2], st[3], sc, active, tol);
+              if (first && active) {
+                if (null_task) SS.null_ll = val;
+                else SS.val[slot_i] = val;
               }
             }
           }
         }
         __syncthreads();
-        continue;   // phase 1 reads the derived calls and the speculative midpoints
-      }
-      if (tid == 0) {
-        if (ph == 1) {
-          bool poly = false;
-          if (variant != 5 && n > 0) poly = ((SS.res[kResFull] - SS.res[kResNull]) - P.log10_ref_length) >= P.polymorphism_cutoff;
-          SS.emitted = (cons || poly) ? 1 : 0;
-        }
-        if (ph == 1 && two_stage) {
-          // the profile phase runs only for an emitted entry with a variant allele
-          SS.done = (SS.emitted && variant < 5 && n > 0) ? 0 : 1;
-        } else if (ph == prof_ph) {
-          // write_RA_frequency_bounds (identify_mutations.cpp:3175-3217)
-          if (SS.emitted && variant < 5 && n > 0) {
-            const double fh = SS.full_f[variant];
-            const double target = SS.res[kResPlmax] - kDrop;
+        if (wave == 0) {
+          // lanes 0 and 32 walk the lower and the upper bound side by side
+          const int side = lane >> 5;
+          const bool walker = (lane & 31) == 0;
+          bool close = false;   // a comparison the tasks' values do not decide
+          const bool tasks = kind == kRowsLds;
+          const double guard = P.screen_off ? INFINITY : kGuardLog;
+          Bound B;
+          if (round == 0) {
+            // (used if emitted)
+            B.lo = side ? fh : 0.0;
+            B.hi = side ? 1.0 : fh;
+            B.vlo = side ? SS.val[0] : SS.val[1];
+            B.vhi = side ? SS.val[2] : SS.val[0];
+            B.out = side ? 1.0 : 0.0;
+            B.iter = 0;
+            B.active = have_v ? 2 : 0;
+          } else {
+            B.lo = SS.lo[side];
+            B.hi = SS.hi[side];
+            B.vlo = SS.vlo[side];
+            B.vhi = SS.vhi[side];
+            B.out = SS.out[side];
+            B.iter = SS.iter[side];
+            B.active = SS.active[side];
+          }
+          const double target = (round == 0) ? SS.val[0] - kDrop : SS.target;
+          const int n_tree = SS.n_tree, slot0 = SS.slot0[side];
+          if (exact == 1 + side) {
+            // the exact comparison decides this side's end of the range, or its midpoint.  (The values
+            // are within the guard of the target; the exact ones hold the lpmax sum.)
+            B.step(side, SS.exact_v >= SS.exact_target, SS.exact_x[side], target, tol, fh);
+          }
+          if (walker && (!exact || !tasks || P.screen_off) && B.active) {
+            const int depth = (exact || !tasks) ? 0 : SS.depth[side];
+            if (B.active == 2) {
+              const double v = side ? B.vhi : B.vlo;
+              close = !tasks || !(fabs(v - target) > guard);
+              if (!close) B.step(side, v >= target, 0.0, v, tol, fh);
+            }
+            // down the evaluated levels: every level is one sequential bisection step (the interval
+            // halved at 0.5 * (lo + hi), 40 steps at most, until it is no wider than tol)
+            int node = 0;
+            for (int level = 0; B.active == 1 && !close; level++) {
+              // a tree's node is the sequential midpoint by construction; a path's only while every
+              // earlier decision followed the path (off it, the interval and so its midpoint differ)
+              const int k = node < n_tree ? node : n_tree + level;
+              if (k >= depth) break;
+              const double m = 0.5 * (B.lo + B.hi), at = SS.pts[side][k], v = SS.val[slot0 + k];
+              if (m != at) break;
+              close = !(fabs(v - target) > guard);
+              if (close) break;
+              const bool ge = v >= target;
+              B.step(side, ge, m, v, tol, fh);
+              node = 2 * node + (((side == 0) ? ge : !ge) ? 1 : 2);
+            }
+            if (B.active == 1 && (!tasks || P.screen_off)) close = true;   // every step exactly
+          }
+          // neither end of the search may hang on the last bits of the ML frequency
+          const double width = B.hi - B.lo;
+          if (!in_order && (fabs(width - tol) < 1e-11 || fabs(2.0 * width - tol) < 1e-11)) close = true;
+          if (walker) {
+            SS.lo[side] = B.lo;
+            SS.hi[side] = B.hi;
+            SS.vlo[side] = B.vlo;
+            SS.vhi[side] = B.vhi;
+            SS.out[side] = B.out;
+            SS.iter[side] = B.iter;
+            SS.active[side] = B.active;
+            SS.exact_x[side] = (B.active == 2) ? (side ? 1.0 : 0.0) : 0.5 * (B.lo + B.hi);
+          }
+          const unsigned long long u = __ballot(walker && close), open = __ballot(walker && B.active != 0);
+          const double out0 = readlane_d(B.out, 0), out1 = readlane_d(B.out, 32);
+          if (lane == 0) {
             SS.target = target;
-            if (SS.res[kResP0] < target) {
-              SS.lo[0] = 0.0;
-              SS.hi[0] = fh;
-              SS.vlo[0] = SS.res[kResP0];
-              SS.vhi[0] = SS.res[kResPlmax];
-              SS.iter[0] = 0;
-              SS.active[0] = (fh - 0.0) > tol ? 1 : 0;
-              SS.lower = fh;
+            if (exact) SS.exact_have = 1;
+            SS.exact = (in_order && u) ? ((u & 1ull) ? 1 : 2) : 0;
+            // emitted: a consensus call, or a presence score at the cutoff
+            const double score = (SS.full_ll - SS.null_ll) - P.log10_ref_length;
+            const bool emitted = cons || (have_v && score >= P.polymorphism_cutoff);
+            SS.emitted = emitted ? 1 : 0;
+            SS.done = (!emitted || !have_v || !open) ? 1 : 0;
+            int unsure = 0;
+            if (level < 2 && have_v) {
+              if (!(fabs(score - P.polymorphism_cutoff) > kGuardLog) || (emitted && !prints_surely_f1(score))) unsure = 2;
             }
-            if (SS.res[kResP1] < target) {
-              SS.lo[1] = fh;
-              SS.hi[1] = 1.0;
-              SS.vlo[1] = SS.res[kResPlmax];
-              SS.vhi[1] = SS.res[kResP1];
-              SS.iter[1] = 0;
-              SS.active[1] = (1.0 - fh) > tol ? 1 : 0;
-              SS.upper = fh;
+            if (level == 0 && have_v && emitted && unsure == 0) {
+              if (u) unsure = 1;
+              if (SS.done && !(prints_surely_e(out0, P.places) && (out1 == 1.0 || prints_surely_e(out1, P.places)))) unsure = 1;
             }
-          }
-          // the speculative levels evaluated with the profiles are walked like a round's path
-          for (int side = 0; side < 2; side++) {
-            SS.path[side] = 1;
-            SS.depth[side] = SS.spec[side];
+            SS.unsure = unsure;
+            if (unsure) SS.done = 1;
           }
         }
-        if (ph >= prof_ph) {
-          // walk each open bound down the evaluated levels: every level is one sequential
-          // bisection step (interval halved at 0.5 * (lo + hi), ≤ 40 steps, stop at width ≤ tol)
-          for (int side = 0; side < 2; side++) {
-            if (!SS.active[side]) continue;
-            const double* r = &SS.res[kResBisect + side * kBisectPts];
-            const bool path = SS.path[side] != 0;
-            double l = SS.lo[side], h = SS.hi[side];
-            double vl = SS.vlo[side], vh = SS.vhi[side];
-            int i = SS.iter[side];
-            int node = 0, advanced = 0;
-            for (int level = 0; level < SS.depth[side]; level++) {
-              if (level > 0 && !(i < 40 && (h - l) > tol)) break;
-              const double m = 0.5 * (l + h);
-              // a path's midpoint at this level is the sequential one only while every earlier
-              // decision followed the path (off it, the interval and so its midpoint differ)
-              if (path && m != SS.pts[side][level]) break;
-              // lower bound: a profile >= target moves hi down; upper bound: moves lo up
-              const double v = r[node];
-              const bool ge = v >= SS.target;
-              const bool left = (side == 0) ? ge : !ge;   // the interval kept is [l, m]
-              if (left) {
-                h = m;
-                vh = v;
-              } else {
-                l = m;
-                vl = v;
-              }
-              i++;
-              advanced++;
-              node = path ? level + 1 : 2 * node + (left ? 1 : 2);
-            }
-            if (ph > prof_ph && path && advanced < 3) SS.tree_only[side] = 1;
-            SS.lo[side] = l;
-            SS.hi[side] = h;
-            SS.vlo[side] = vl;
-            SS.vhi[side] = vh;
-            SS.iter[side] = i;
-            SS.active[side] = (i < 40 && (h - l) > tol) ? 1 : 0;
-            if (side == 0) SS.lower = h;
-            else SS.upper = l;
-          }
-        }
-        // midpoints of the next round, each the midpoint of the interval a sequential bisection
-        // would hold there: along the predicted path, or breadth-first over a full tree
-        const bool both = SS.active[0] && SS.active[1];
-        for (int side = 0; side < 2 && ph >= prof_ph; side++) {
-          if (!SS.active[side]) {
-            SS.depth[side] = 0;
-            continue;
-          }
-          const double lo = SS.lo[side], hi = SS.hi[side];
-          double* pt = SS.pts[side];
-          if (!SS.tree_only[side]) {
-            const int depth = both ? kBisectPts / 2 : kBisectPts;
-            const double fs = predict_crossing(side, lo, hi, SS.vlo[side], SS.vhi[side], SS.full_f[variant],
-                                               SS.res[kResPlmax], SS.target, n);
-            double a = lo, b = hi;
-            for (int d = 0; d < depth; d++) {
-              const double m = 0.5 * (a + b);
-              pt[d] = m;
-              const bool left = (side == 0) ? (fs <= m) : (fs < m);
-              if (left) b = m;
-              else a = m;
-            }
-            SS.path[side] = 1;
-            SS.depth[side] = depth;
-            continue;
-          }
-          SS.path[side] = 0;
-          SS.depth[side] = both ? 2 : 3;
-          const double m0 = 0.5 * (lo + hi);
-          const double m1 = 0.5 * (lo + m0), m2 = 0.5 * (m0 + hi);
-          pt[0] = m0;
-          pt[1] = m1;
-          pt[2] = m2;
-          pt[3] = 0.5 * (lo + m1);
-          pt[4] = 0.5 * (m1 + m0);
-          pt[5] = 0.5 * (m0 + m2);
-          pt[6] = 0.5 * (m2 + hi);
-        }
-        if (ph >= prof_ph) SS.done = (SS.active[0] || SS.active[1]) ? 0 : 1;
+        __syncthreads();
+        if (SS.done) break;
       }
-      __syncthreads();
-      if (SS.done) break;
+      const int unsure = uniform_i(SS.unsure);
+      if (level == 2 || unsure == 0) break;
+      level = max(level + 1, unsure);
+      __syncthreads();   // every wavefront has read the verdict before it is cleared
     }
     if (tid == 0) {
       RaOut out;
@@ -1036,12 +1496,11 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(3
       out.pad[0] = out.pad[1] = out.pad[2] = 0;
       out.n = (uint32_t)n;
       for (int b = 0; b < 5; b++) out.f[b] = SS.full_f[b];
-      out.variant_score = (variant != 5 && n > 0) ? (SS.res[kResFull] - SS.res[kResNull]) - P.log10_ref_length
-                                                  : __longlong_as_double(0x7ff8000000000000LL);
-      out.lower = emitted ? SS.lower : 0.0;
-      out.upper = emitted ? SS.upper : 1.0;
-      out.ks_p = emitted ? SS.ks_p : 1.0;
-      out.fisher_p = emitted ? SS.fisher_p : 1.0;
+      out.variant_score = have_v ? (SS.full_ll - SS.null_ll) - P.log10_ref_length : __longlong_as_double(0x7ff8000000000000LL);
+      out.lower = emitted ? SS.out[0] : 0.0;
+      out.upper = emitted ? SS.out[1] : 1.0;
+      out.ks_p = (emitted && n > 0) ? SS.ks_p : 1.0;
+      out.fisher_p = (emitted && n > 0) ? SS.fisher_p : 1.0;
       int tt = 0, tb = 0;
       for (int b = 0; b < 5; b++) {
         out.cov[b][0] = SS.cov[b][2];

@@ -155,8 +155,9 @@ struct Session {
   DBuf<uint32_t> d_key_scratch;      // read lists of the scorer and k_fix_columns for deep samples
   DBuf<uint8_t> d_col_flags;
   DBuf<int32_t> d_col_unique, d_col_total;
-  DBuf<int2> d_cand;
-  DBuf<int32_t> d_counters;   // [0] n_cand, [1] n_ins, [2] n_runs, [3] error bits, [4] n_fix
+  DBuf<int2> d_cand, d_score;
+  DBuf<int32_t> d_counters;   // [0] n_cand, [1] n_ins, [2] n_runs, [3] error bits, [4] n_fix,
+                              // [5] score_next, [6] n_score
   DBuf<int32_t> d_fix;
   DBuf<IdRec> d_idrec;
   DBuf<uint32_t> d_ct_u, d_ct_raw, d_ct_beg;   // BAM2COV column counts (coverage table)
@@ -1264,6 +1265,7 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   const int ins_cap = std::max<int>(std::max<int>(1 << 14, S.n_pos / 256), S.id_caps.ins);
   const int run_cap = std::max<int>(std::max<int>(1 << 16, S.n_pos / 16), S.id_caps.runs);
   S.d_cand.alloc(cand_cap);
+  S.d_score.alloc(cand_cap);
   S.d_ins.alloc(ins_cap);
   S.d_ra.alloc(cand_cap);
   S.d_runrec.alloc(run_cap);
@@ -1297,6 +1299,7 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   P.mutation_cutoff = a->mutation_cutoff;
   P.polymorphism_cutoff = a->polymorphism_cutoff;
   P.precision_decimal = a->polymorphism_precision_decimal;
+  P.places = (int32_t)std::min<uint32_t>(a->polymorphism_precision_places, 1000u);
   P.screen_margin = 0.1;
   P.screen_off = screen_off;
   P.col_flags = S.d_col_flags.p;
@@ -1304,17 +1307,25 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   P.col_total = S.d_col_total.p;
   P.cand = S.d_cand.p;
   P.n_cand = S.d_counters.p + 0;
+  P.score = S.d_score.p;
+  P.n_score = S.d_counters.p + 6;
   P.score_next = S.d_counters.p + 5;
   P.cand_cap = cand_cap;
   P.ins = S.d_ins.p;
   P.n_ins = S.d_counters.p + 1;
   P.ins_cap = ins_cap;
   P.key_cap = std::max(64, S.max_window_reads);
-  // a candidate's read list (4 B per read of its window) stays in LDS while it takes at most half
-  // of the scorer's dynamic LDS; deeper samples keep it in a device scratch list per block
-  const size_t score_dyn_budget = kScoreLdsBudget - kScoreStaticLds;
+  // a candidate's read list (4 B per read of its window) stays in LDS up to kScoreKeyLds; deeper
+  // samples keep it in a device scratch list per block.  The rest of the scorer's dynamic LDS
+  // holds its rows: per distinct table key the ratios twice (96 B), the model values (16 B), the key
+  // and its reads (8 B).
   const size_t key_list_bytes = ((size_t)P.key_cap * sizeof(uint32_t) + 15) & ~(size_t)15;
-  P.keys_global = (key_list_bytes > score_dyn_budget / 2) ? 1 : 0;
+  P.keys_global = (key_list_bytes > kScoreKeyLds) ? 1 : 0;
+  // four blocks per CU while that leaves room for as many rows as a column has distinct keys at
+  // usual depths (some 60 at 100x, 200 at 3,000x); a longer read list takes more LDS per block
+  const size_t score_lds_budget = (key_list_bytes + 220 * kScoreRowBytes + kScoreStaticLds <= kScoreLdsBudget) ? kScoreLdsBudget
+                                                                                                            : kScoreLdsDeep;
+  const size_t score_dyn_budget = score_lds_budget - kScoreStaticLds;
   const size_t key_bytes = P.keys_global ? 0 : key_list_bytes;
   if (P.keys_global) {
     S.d_key_scratch.alloc((size_t)kScoreGrid * (size_t)P.key_cap);
@@ -1322,8 +1333,8 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   } else {
     P.key_scratch = nullptr;
   }
-  P.rows_cap = (int32_t)((score_dyn_budget - key_bytes) / (6 * sizeof(double)));
-  const size_t score_lds = key_bytes + (size_t)P.rows_cap * 6 * sizeof(double);
+  P.rows_cap = (int32_t)((score_dyn_budget - key_bytes) / kScoreRowBytes);
+  const size_t score_lds = key_bytes + (size_t)P.rows_cap * kScoreRowBytes;
   P.ra_out = S.d_ra.p;
   P.err = (uint32_t*)(S.d_counters.p + 3);
   P.fix = S.d_fix.p;
@@ -1375,8 +1386,9 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   S.h_tab_r.alloc(L.rr.size());
   std::copy(L.rr.begin(), L.rr.end(), S.h_tab_r.p);
   HIP_OK(hipMemcpyAsync(S.d_tab_r.p, S.h_tab_r.p, L.rr.size() * sizeof(double), hipMemcpyHostToDevice, S.stream));
-  // the insert slots and the scorer need no coverage cutoff: queued before the host waits for the fit
-  hipLaunchKernelGGL(k_insert_slots, dim3(1024), dim3(64), 0, S.stream, P);
+  // the candidates and the scorer need no coverage cutoff: queued before the host waits for the fit
+  const size_t route_lds = (P.tab_keys <= kRouteKeys) ? kRouteWaves * sizeof(uint32_t) * route_words(P.tab_keys) : 0;
+  hipLaunchKernelGGL(k_route_candidates, dim3(kRouteGrid), dim3(64 * kRouteWaves), route_lds, S.stream, P);
   HIP_OK(hipGetLastError());
   HIP_OK(hipEventRecord(S.evk[1], S.stream));
   if (P.keys_global)
@@ -1386,7 +1398,7 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   HIP_OK(hipGetLastError());
   HIP_OK(hipEventRecord(S.ev1, S.stream));
   // MC/UN runs read only the final column flags and coverage and the fitted cutoffs, so they run on
-  // the side stream beside the insert slots and the scorer
+  // the side stream beside the candidates and the scorer
   HIP_OK(hipStreamWaitEvent(S.stream2, S.evk[3], 0));
   std::vector<double> prop_final(a->deletion_propagation_cutoff, a->deletion_propagation_cutoff + S.n_targets);
   if (late) {
@@ -1418,7 +1430,7 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   if (S.gd_on_device) {
     // the writer reads the MC/UN runs too: the stream waits for them
     HIP_OK(hipStreamWaitEvent(S.stream, S.evk[5], 0));
-    gd_in.n_cand = S.d_counters.p + 0;
+    gd_in.n_cand = S.d_counters.p + 6;
     gd_in.cand_cap = cand_cap;
     gd_in.n_runs = S.d_counters.p + 2;
     gd_in.run_cap = run_cap;
@@ -1501,13 +1513,13 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
     minimum = (int32_t)want;
     grow = true;
   };
-  need(counters[0], cand_cap, S.id_caps.cand);
+  need(std::max(counters[0], counters[6]), cand_cap, S.id_caps.cand);
   need(counters[1], ins_cap, S.id_caps.ins);
   need(counters[2], run_cap, S.id_caps.runs);
   need(counters[4], fix_cap, S.id_caps.fix);
   if (grow) return false;
   raise_err_bits(errbits);
-  const int n_cand = counters[0];
+  const int n_cand = counters[6];
   S.timing.candidates = n_cand;
   if (S.gd_on_device) {
     const double t1 = now_ms();
