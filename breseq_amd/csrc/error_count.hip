@@ -5,14 +5,12 @@
 // Both outputs are integer sums, so they do not depend on the order in which pileup entries are
 // visited.  Pass 1 therefore walks each alignment once (read-parallel) instead of walking columns:
 //
-//   k_ec_reads       32 consecutive alignments per work item.  First the item's counted
-//                    single-run alignments of at most 168 bases, three to a wavefront (21 lanes
-//                    each, eight query positions per lane); then its other alignments one per
-//                    wavefront, each lane four consecutive query positions of an M/=/X run.  Bases
-//                    and qualities are dword loads from 8-byte aligned read starts, reference codes
-//                    aligned dword loads.  Covariates go to an LDS-privatized count table.  The
-//                    first lane of an alignment adds +1/-1 at the ends of each aligned run to a
-//                    per-column difference array (unique or redundant).
+//   k_ec_reads       64 consecutive alignments per work item of a wavefront, which steps through
+//                    their M/=/X runs together.  The runs become items of eight query positions that
+//                    the 64 lanes share evenly.  Bases and qualities are 8-byte loads from 8-byte
+//                    aligned groups.  Covariates go to an LDS-privatized count table.  The lane of an
+//                    alignment adds +1/-1 at the ends of each aligned run to a per-column difference
+//                    array (unique or redundant).
 //   k_cov_tile_sums  phase 1 of the prefix scan of the difference arrays (per 4096-column tile)
 //   k_cov_tile_scan  phase 2: exclusive scan of the tile sums (one block)
 //   k_cov_hist       phase 3: per-column unique and redundant coverage -> histogram of the unique
@@ -48,21 +46,27 @@ __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = v;
 }
 
-// BAM 4-bit base code -> A0 C1 G2 T3; every other code -> 15.
-__device__ __forceinline__ uint32_t base_idx(uint32_t b) {
-  const uint32_t i = (uint32_t)(0xFFFFFFF3FFF2F10FULL >> ((b & 15u) * 4u)) & 15u;
-  return b > 15u ? 15u : i;
+__device__ __forceinline__ int wave_sum(int v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
 }
 
-// Complement of a base index when rv == 3 (A<->T, C<->G); other codes are unchanged.
-__device__ __forceinline__ uint32_t comp_if(uint32_t i, uint32_t rv) { return i < 4u ? (i ^ rv) : i; }
+// Inclusive scan across the 64 lanes of a wavefront.
+__device__ __forceinline__ int wave_incl_scan(int v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(v, o, 64);
+    if (lane >= o) v += u;
+  }
+  return v;
+}
 
-typedef __attribute__((address_space(4))) const uint32_t ConstU32;
-typedef __attribute__((address_space(4))) const int32_t ConstI32;
 
 // Indel carried by the entry of the last base of the reference-consuming operation at index k
 // (htslib resolve_cigar2 as breseq reads it; same rule as entry_at).
-__device__ __forceinline__ int run_end_indel(const ConstU32* c, int k, int n) {
+__device__ __forceinline__ int run_end_indel(const uint32_t* c, int k, int n) {
   if (k + 1 >= n) return 0;
   const uint32_t op2 = c[k + 1] & 15u;
   int indel = 0;
@@ -93,13 +97,6 @@ __device__ __forceinline__ int run_end_indel(const ConstU32* c, int k, int n) {
 
 __device__ __forceinline__ uint32_t byte_of(uint32_t w, int k) { return (w >> (8 * k)) & 0xFFu; }
 
-// Bin of (read set rs, reference class ri, observed class oi, quality q) in the count table,
-// rs + S*(ri + 5*oi + 25*q), as full-rate 24-bit multiply-adds: every operand is below 2^16
-// (classes below 16, qualities below 256, S at most 256).
-__device__ __forceinline__ uint32_t ec_bin(uint32_t rs, uint32_t S, uint32_t ri, uint32_t oi, uint32_t q) {
-  return __umul24(__umul24(q, 25u) + __umul24(oi, 5u) + ri, S) + rs;
-}
-
 // Strand-folded base indices as 4-bit lookup tables: read bases by BAM code (A1 C2 G4 T8), reference
 // bases by kRef* code (A0 C1 G2 T3 '.'4 N5).  The reverse-strand tables complement A<->T, C<->G, as
 // count_alignment_position does before indexing (error_count.cpp:887-903).  15 = not a base.
@@ -108,250 +105,338 @@ constexpr uint64_t kReadLutRev = 0xFFFFFFF0FFF1F23FULL;
 constexpr uint32_t kRefLutFwd = 0xFF543210u;
 constexpr uint32_t kRefLutRev = 0xFF540123u;
 
-// count_alignment_position (error_count.cpp:854-986) for the aligned bases [x, x+len) <-> query
-// [y, y+len) of one unique read; the last base carries `last_indel`.  Each lane takes four
-// consecutive query positions of a 4-aligned group: reads start at 8-byte aligned offsets, so the
-// bases and qualities of the group and of the next four positions are two dword loads each; the
-// five reference codes the group needs come from two aligned dwords of ref_idx.  Per base: the
-// base/reference observation (1) and the '..' pair observation (2) are one LDS atomic each; the
-// one-base deletion (3) and insertion (4) observations can only occur at the run's last base and
-// are handled there.
-template <bool kRev>
-__device__ __forceinline__ void ec_count_run(const EcParams& P, const uint8_t* __restrict__ sq,
-                                             const uint8_t* __restrict__ ql, const DRead& R, int x, int y, int len,
-                                             int last_indel, uint32_t* table, uint32_t& err) {
-  const uint32_t S = (uint32_t)P.read_set_max, Q = (uint32_t)P.quality_max;
-  const uint64_t rlut = kRev ? kReadLutRev : kReadLutFwd;
-  const uint32_t flut = kRev ? kRefLutRev : kRefLutFwd;
-  const uint32_t rs = R.rfile;
-  const uint32_t pair_base = rs + 24u * S;   // ref '.', obs '.'
-  const int lane = threadIdx.x & 63;
-  const int yend = y + len;
-  const int last = yend - 1;
-  const int qe0 = (int)R.qe0;
-  // pair observations end at q_end, and at the last base when a deletion or insertion follows it
-  const int pair_end = (last_indel != 0) ? min(qe0, last) : qe0;
-  for (int q0 = (y & ~3) + 4 * lane; q0 < yend; q0 += 256) {
-    const uint32_t bw0 = *(const uint32_t*)(sq + q0), bw1 = *(const uint32_t*)(sq + q0 + 4);
-    const uint32_t qw0 = *(const uint32_t*)(ql + q0), qw1 = *(const uint32_t*)(ql + q0 + 4);
-    const int c0 = x + (q0 - y);   // column of query position q0 (>= x - 3; ref_idx is front-padded)
-    const uint32_t* rp = (const uint32_t*)(P.ref_idx + (c0 & ~3));
-    const uint32_t rw0 = rp[0], rw1 = rp[1];
-    const int sh = c0 & 3;
-    const uint32_t rlo = __builtin_amdgcn_alignbyte(rw1, rw0, sh);   // codes of columns c0 .. c0+3
-    const uint32_t r4 = (rw1 >> (8 * sh)) & 0xFFu;                   // code of column c0+4
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const int qpos = q0 + k;
-      const bool in = qpos >= y && qpos <= last;
-      const uint32_t b = byte_of(bw0, k), q = byte_of(qw0, k);
-      const uint32_t r0 = byte_of(rlo, k);
-      // (1) base against reference (:877-903)
-      const uint32_t oi = (b > 15u) ? 15u : (uint32_t)(rlut >> (4u * b)) & 15u;
-      const uint32_t ri = (flut >> (4u * r0)) & 15u;
-      const bool v1 = in && b != 15u && r0 != kRefN;
-      const bool good1 = v1 && oi < 4u && ri < 4u && q < Q;
-      if (v1 && !good1) err |= (oi > 3u) ? kErrBaseCode : (ri > 3u) ? kErrRefChar : kErrQuality;
-      if (good1) atomicAdd(&table[ec_bin(rs, S, ri, oi, q)], 1u);
-      // (2) '..' pair (:909-928): the base after qpos in read direction (qpos+1 forward, qpos
-      // itself reverse) against the reference after it in reference direction
-      const uint32_t b2 = kRev ? b : ((k < 3) ? byte_of(bw0, k + 1) : byte_of(bw1, 0));
-      const uint32_t q2 = kRev ? q : ((k < 3) ? byte_of(qw0, k + 1) : byte_of(qw1, 0));
-      const uint32_t rp2 = kRev ? r0 : ((k < 3) ? byte_of(rlo, k + 1) : r4);
-      const bool v2 = in && qpos < pair_end && b2 != 15u && rp2 != kRefN;
-      if (v2 && q2 >= Q) err |= kErrQuality;
-      if (v2 && q2 < Q) atomicAdd(&table[__umul24(q2, 25u * S) + pair_base], 1u);
-    }
+// A block's count table in LDS: 25 words per (read set, quality) row, ri + 5*oi, and after the rows
+// one signed word per row for the '..' pairs (below).
+constexpr uint32_t kEcRow = 25;
+
+struct EcTable {
+  uint32_t* bins;
+  int32_t* pairs;
+  __device__ __forceinline__ void add(uint32_t row, uint32_t ri, uint32_t oi) const {
+    atomicAdd(&bins[row * kEcRow + ri + 5u * oi], 1u);
   }
-  if (last_indel != -1 && last_indel != 1) return;
-  // (3) one-base deletion (:934-956) / (4) one-base insertion (:963-982) after the last base
-  if (lane != 0) return;
-  const int qpos = last, p = x + len - 1;
-  const uint32_t b = sq[qpos], q = ql[qpos];
-  const uint32_t r1 = P.ref_idx[p + 1];
+};
+
+// Four positions' table offsets: bytes of (ri + 5*oi) * 4, or 96 where nothing is counted (N base,
+// N reference).  Byte-wise on whole words: v_perm_b32 looks four codes up at once (its selectors 13
+// and above give 0xFF, and 8 the sign of table byte 1, here 0), the strand is an XOR (the classes are
+// numbered T0 G1 C2 A3, the complement of A0 C1 G2 T3).  `odd` becomes nonzero when a byte needs the
+// position-wise path: a code that is no base, a reference that is neither base nor N, or a quality
+// that may be at or above the maximum.
+__device__ __forceinline__ uint32_t ec_classes(uint32_t b, uint32_t q, uint32_t r, uint32_t strand, uint32_t q_add,
+                                               uint32_t& odd) {
+  const uint32_t rd = __builtin_amdgcn_perm(0x00000010u, 0x00203000u, b);   // 16 * class, N 0xFF
+  const uint32_t rf = __builtin_amdgcn_perm(0x40408040u, 0x0004080Cu, r);   // 4 * class, N 0x80, other 0x40
+  const uint32_t u = rd | rf;
+  // the code that the class stands for, against the code itself
+  const uint32_t back = __builtin_amdgcn_perm(0u, 0x01020408u, (rd >> 4) & 0x0F0F0F0Fu);
+  odd |= ((back ^ b) & 0x0F0F0F0Fu) | (b & 0xF0F0F0F0u);
+  odd |= u & ~(u >> 1) & 0x40404040u;
+  odd |= (((q & 0x7F7F7F7Fu) + q_add) | q) & 0x80808080u;
+  const uint32_t x = (u ^ strand) & 0x3C3C3C3Cu;
+  const uint32_t c = x + ((x >> 2) & 0x0C0C0C0Cu);
+  const uint32_t none = __builtin_amdgcn_perm(u, u << 8, 0x0B090A08u);      // bit 7 spread over its byte
+  return (none & 0x60606060u) | (c & ~none);
+}
+
+// Counts base against reference (count_alignment_position's first observation, error_count.cpp:
+// 877-903) of eight consecutive query positions: bytes [lo, hi) of the base, quality and reference
+// words, all in the run.  Nothing-counted bytes go to bin 24 of their row, which is never read.
+__device__ __forceinline__ void ec_eight(uint2 b, uint2 q, const uint2 r, int lo, int hi, bool rev, uint32_t row0,
+                                         uint32_t Q, const EcTable& T, uint32_t& err) {
+  const uint64_t in = (~0ull << (8 * max(lo, 0))) & (~0ull >> (64 - 8 * min(hi, 8)));
+  const uint32_t in0 = (uint32_t)in, in1 = (uint32_t)(in >> 32);
+  b.x = (b.x & in0) | (0x0F0F0F0Fu & ~in0);   // outside the run: N bases of quality 0
+  b.y = (b.y & in1) | (0x0F0F0F0Fu & ~in1);
+  q.x &= in0;
+  q.y &= in1;
+  const uint32_t strand = rev ? 0u : 0x3C3C3C3Cu;
+  const uint32_t q_add = (Q <= 128u) ? (128u - Q) * 0x01010101u : 0u;
+  uint32_t odd = 0;
+  const uint32_t c0 = ec_classes(b.x, q.x, r.x, strand, q_add, odd);
+  const uint32_t c1 = ec_classes(b.y, q.y, r.y, strand, q_add, odd);
+  unsigned char* base = (unsigned char*)(T.bins + row0 * kEcRow);
+  if (odd == 0) {
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const uint32_t off = __umul24(byte_of(k < 4 ? q.x : q.y, k & 3), 4u * kEcRow) + byte_of(k < 4 ? c0 : c1, k & 3);
+      atomicAdd((uint32_t*)(base + off), 1u);
+    }
+    return;
+  }
+  const uint64_t rlut = rev ? kReadLutRev : kReadLutFwd;
+  const uint32_t flut = rev ? kRefLutRev : kRefLutFwd;
+  for (int k = 0; k < 8; k++) {
+    const uint32_t bk = byte_of(k < 4 ? b.x : b.y, k & 3), qk = byte_of(k < 4 ? q.x : q.y, k & 3);
+    const uint32_t rk = byte_of(k < 4 ? r.x : r.y, k & 3);
+    if (bk == 15u || rk == kRefN) continue;
+    const uint32_t oi = (bk > 15u) ? 15u : (uint32_t)(rlut >> (4u * bk)) & 15u;
+    const uint32_t ri = (flut >> (4u * rk)) & 15u;
+    if (oi > 3u) err |= kErrBaseCode;
+    else if (ri > 3u) err |= kErrRefChar;
+    else if (qk >= Q) err |= kErrQuality;
+    else T.add(row0 + qk, ri, oi);
+  }
+}
+
+// The '..' pair observation (error_count.cpp:909-928) of a position takes the base after it in read
+// direction against the reference after it in reference direction: for a forward read position
+// j = qpos + 1, for a reverse read j = qpos, and both count the quality at j where neither the base
+// nor the reference at j is N -- the condition under which the base observation counts j.  So over a
+// run [y, last] the pairs are the run's base observations except one at the run's first position
+// (forward) or last (reverse), and one more where the pairs reach past the run.  The flush adds the
+// 16 base bins of a row up, and `pairs` holds these corrections: one LDS atomic per run in place of
+// one per position.  q_end is never before a run's last base, since only soft clips behind it are
+// taken off it.
+__device__ __forceinline__ void ec_pair(const EcParams& P, const uint8_t* sq, const uint8_t* ql, int j, int col,
+                                        uint32_t row0, int v, const EcTable& T, uint32_t& err) {
+  const uint32_t b = sq[j], q = ql[j];
+  if (b == 15u || P.ref_idx[col] == kRefN) return;
+  if (q >= (uint32_t)P.quality_max) err |= kErrQuality;
+  else atomicAdd(&T.pairs[row0 + q], v);
+}
+
+__device__ __forceinline__ void ec_run_pairs(const EcParams& P, const uint8_t* sq, const uint8_t* ql, bool rev, int x,
+                                             int y, int len, int last_indel, int qe0, uint32_t row0, const EcTable& T,
+                                             uint32_t& err) {
+  const int last = y + len - 1;
+  const bool past = last_indel == 0 && qe0 > last;   // the run's last position has a pair
+  if (!rev) ec_pair(P, sq, ql, y, x, row0, -1, T, err);
+  if (past != rev) ec_pair(P, sq, ql, past ? last + 1 : last, past ? x + len : x + len - 1, row0, past ? 1 : -1, T, err);
+}
+
+// a[at] += v from every lane with at >= 0, one atomic for consecutive lanes of the same address: in a
+// deep sample dozens of neighbouring alignments start (and, of equal length, end) at one column.
+__device__ __forceinline__ void add_equal(int32_t* a, int at, int v) {
+  const int lane = threadIdx.x & 63;
+  const int prev = __shfl_up(at, 1, 64);
+  const bool head = lane == 0 || prev != at;
+  const unsigned long long later = __ballot(head) & ~((2ull << lane) - 1ull);
+  const int n = (later ? __builtin_ctzll(later) : 64) - lane;
+  if (head && at >= 0) atomicAdd(&a[at], v * n);
+}
+
+__device__ __forceinline__ uint2 load8(const uint8_t* p) {
+  uint2 v;
+  __builtin_memcpy(&v, p, 8);   // one load; the hardware takes any alignment
+  return v;
+}
+
+// The one-base deletion (error_count.cpp:934-956) or insertion (:963-982) after a run's last base.
+__device__ __forceinline__ void ec_run_indel(const EcParams& P, const uint8_t* sq, const uint8_t* ql, const DRead& R,
+                                             int x, int y, int len, int last_indel, uint32_t row0, const EcTable& T,
+                                             uint32_t& err) {
+  const uint32_t Q = (uint32_t)P.quality_max;
+  const bool rev = (R.flags & kReadReversed) != 0;
+  const int last = y + len - 1;
   if (last_indel == -1) {
-    if (!kRev && qpos + 1 >= (int)R.l_qseq) {
+    if (!rev && last + 1 >= (int)R.l_qseq) {
       err |= kErrQueryIndex;
       return;
     }
-    const uint32_t b2 = kRev ? b : (uint32_t)sq[qpos + 1];
-    const uint32_t q2 = kRev ? q : (uint32_t)ql[qpos + 1];
-    if (b2 == 15u || r1 == kRefN) return;
-    const uint32_t rd = (flut >> (4u * r1)) & 15u;
+    const uint32_t b = sq[rev ? last : last + 1], q = ql[rev ? last : last + 1];
+    const uint32_t r = P.ref_idx[x + len];
+    if (b == 15u || r == kRefN) return;
+    const uint32_t rd = ((rev ? kRefLutRev : kRefLutFwd) >> (4u * r)) & 15u;
     if (rd > 4u) err |= kErrRefChar;
-    else if (q2 >= Q) err |= kErrQuality;
-    else atomicAdd(&table[rs + S * rd + 20u * S + 25u * S * q2], 1u);
-  } else {
-    const int mq = qpos + 1;
+    else if (q >= Q) err |= kErrQuality;
+    else if (rd == 4u) atomicAdd(&T.pairs[row0 + q], 1);   // the bin of the pairs
+    else T.add(row0 + q, rd, 4u);
+  } else if (last_indel == 1) {
+    const int mq = last + 1;
     if (mq >= (int)R.l_qseq) {
       err |= kErrQueryIndex;
       return;
     }
-    if (mq > qe0 || mq < (int)R.qs0) return;
-    const uint32_t b3 = sq[mq];
-    if (b3 == 15u) return;
-    const uint32_t oi = (b3 > 15u) ? 15u : (uint32_t)(rlut >> (4u * b3)) & 15u;
-    const uint32_t q3 = ql[mq];
+    if (mq > (int)R.qe0 || mq < (int)R.qs0) return;
+    const uint32_t b = sq[mq], q = ql[mq];
+    if (b == 15u) return;
+    const uint32_t oi = (b > 15u) ? 15u : (uint32_t)((rev ? kReadLutRev : kReadLutFwd) >> (4u * b)) & 15u;
     if (oi > 3u) err |= kErrBaseCode;
-    else if (q3 >= Q) err |= kErrQuality;
-    else atomicAdd(&table[rs + 4u * S + 5u * S * oi + 25u * S * q3], 1u);
+    else if (q >= Q) err |= kErrQuality;
+    else T.add(row0 + q, 4u, oi);
   }
 }
 
-// Observations (1) and (2) of ec_count_run for one lane's four query positions [q0, q0 + 4) of an
-// alignment whose M/=/X run is [x, x + len) <-> [y, y + len) and whose last base carries no indel,
-// with the strand a run-time value (the three alignments of a shared wavefront differ in strand).
-__device__ __forceinline__ void ec_group4(const EcParams& P, const uint8_t* __restrict__ sq,
-                                          const uint8_t* __restrict__ ql, uint32_t rs, bool rev, int x, int y,
-                                          int last, int pair_end, int q0, uint32_t* table, uint32_t& err) {
-  const uint32_t S = (uint32_t)P.read_set_max, Q = (uint32_t)P.quality_max;
-  const uint64_t rlut = rev ? kReadLutRev : kReadLutFwd;
-  const uint32_t flut = rev ? kRefLutRev : kRefLutFwd;
-  const uint32_t pair_base = rs + 24u * S;   // ref '.', obs '.'
-  const uint32_t bw0 = *(const uint32_t*)(sq + q0), bw1 = *(const uint32_t*)(sq + q0 + 4);
-  const uint32_t qw0 = *(const uint32_t*)(ql + q0), qw1 = *(const uint32_t*)(ql + q0 + 4);
-  const int c0 = x + (q0 - y);   // column of query position q0 (>= x - 3; ref_idx is front-padded)
-  const uint32_t* rp = (const uint32_t*)(P.ref_idx + (c0 & ~3));
-  const uint32_t rw0 = rp[0], rw1 = rp[1];
-  const int sh = c0 & 3;
-  const uint32_t rlo = __builtin_amdgcn_alignbyte(rw1, rw0, sh);   // codes of columns c0 .. c0+3
-  const uint32_t r4 = (rw1 >> (8 * sh)) & 0xFFu;                   // code of column c0+4
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int qpos = q0 + k;
-    const bool in = qpos >= y && qpos <= last;
-    const uint32_t b = byte_of(bw0, k), q = byte_of(qw0, k);
-    const uint32_t r0 = byte_of(rlo, k);
-    const uint32_t oi = (b > 15u) ? 15u : (uint32_t)(rlut >> (4u * b)) & 15u;
-    const uint32_t ri = (flut >> (4u * r0)) & 15u;
-    const bool v1 = in && b != 15u && r0 != kRefN;
-    const bool good1 = v1 && oi < 4u && ri < 4u && q < Q;
-    if (v1 && !good1) err |= (oi > 3u) ? kErrBaseCode : (ri > 3u) ? kErrRefChar : kErrQuality;
-    if (good1) atomicAdd(&table[ec_bin(rs, S, ri, oi, q)], 1u);
-    const uint32_t b2 = rev ? b : ((k < 3) ? byte_of(bw0, k + 1) : byte_of(bw1, 0));
-    const uint32_t q2 = rev ? q : ((k < 3) ? byte_of(qw0, k + 1) : byte_of(qw1, 0));
-    const uint32_t rp2 = rev ? r0 : ((k < 3) ? byte_of(rlo, k + 1) : r4);
-    const bool v2 = in && qpos < pair_end && b2 != 15u && rp2 != kRefN;
-    if (v2 && q2 >= Q) err |= kErrQuality;
-    if (v2 && q2 < Q) atomicAdd(&table[__umul24(q2, 25u * S) + pair_base], 1u);
-  }
-}
-
-constexpr int kEcGroup = 21;   // lanes per alignment when three share a wavefront (8 positions each)
-
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) k_ec_reads(EcParams P) {
-  extern __shared__ uint32_t table[];
-  for (int i = threadIdx.x; i < P.n_bins; i += blockDim.x) table[i] = 0;
+// What bounds it: 4.6 Mb at 100x of 150-base reads reads 0.95 GB at 2.7 TB/s (360 us), with the vector
+// unit about 60% busy (17 instructions a position, 125 M in all) and the LDS 30% (one atomic a
+// position).  One alignment of up to 168 bases to 21 lanes, position-wise selects and an atomic each
+// for the base and its pair took 409 M instructions and 871 us; alignments with an indel went one at a
+// time, and a wavefront whose alignments all cross one took 165 us alone.  Measured before -> now, in
+// us: 2.05 Mb at 83x of 36 bases (five of 21 lanes had work) 1166 -> 226, 48 kb at 206x of 100 bases
+// 165 -> 29, 701 kb at 57x of 300 bases (one alignment at a time) 248 -> 63, 1 Mb at 300x 553 -> 259,
+// 20 kb at 3,000x 137 -> 82 (the difference array's atomics, hence add_equal).  64 alignments a work
+// item rather than 32: the loads before the items (record, target) are paid once for twice the items.
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_ec_reads(EcParams P) {
+  extern __shared__ uint32_t ec_lds[];
+  // A run as the lanes that share it read it, in terms of the wavefront's item number i (eight
+  // positions each, the runs' items one after the other): first byte at + 8 i, its column col + 8 i,
+  // and the bytes from begin - 8 i to end - 8 i in the run: {at, col, end, begin * 2 + reversed}.
+  __shared__ uint4 ec_rec[kEcWaves][kEcChunk];
+  __shared__ uint32_t ec_row[kEcWaves][kEcChunk];
+  __shared__ uint32_t ec_first[kEcWaves][2 * kEcSteps];   // bit i: item i is its run's first
+  const int S = P.read_set_max, Q = P.quality_max, rows = S * Q;
+  const EcTable T{ec_lds, (int32_t*)(ec_lds + (size_t)rows * kEcRow)};
+  for (int i = threadIdx.x; i < rows * (int)(kEcRow + 1); i += blockDim.x) ec_lds[i] = 0;
   __syncthreads();
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t gw = ((int64_t)xcd_major_block() * blockDim.x + threadIdx.x) >> 6;
   const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  const ConstI32* pos_target = (const ConstI32*)P.pos_target;
-  const ConstI32* scored = (const ConstI32*)P.target_scored;
-  int32_t* diff_u = P.cov_diff;
-  int32_t* diff_r = P.cov_diff + P.n_pos + 1;
   uint32_t err = 0;
-  // one alignment at a time, wave-uniform (scalar loads; any CIGAR, redundant alignments)
-  auto one = [&](int64_t r) {
-    const DRead R = load_read(P.reads, (int)r);
-    const int t = pos_target[R.gpos];
-    if (t < 0 || !scored[t]) return;
-    const bool red = R.x1 > 1;
-    int32_t* diff = red ? diff_r : diff_u;
-    bool count = !red && P.do_errors;
-    if (count && (int)R.rfile >= P.read_set_max) {   // covariate read_set out of range: ASSERT in the reference
-      err |= kErrReadSet;
-      count = false;
-    }
-    const uint8_t* sq = P.bases + R.seq_off;
-    const uint8_t* ql = P.quals + R.seq_off;
-    if (R.flags & kReadSimple) {
-      if (lane == 0) {
-        atomicAdd(&diff[R.gpos], 1);
-        atomicAdd(&diff[R.gend], -1);
+  for (int64_t c0 = gw * kEcChunk; c0 < P.n_reads; c0 += nw * kEcChunk) {
+    // Lane i takes alignment i and steps through its M/=/X runs; the runs that the lanes are at
+    // become items of eight positions, which the wavefront's lanes share evenly whatever the runs'
+    // lengths (the counts are integers, so the order does not matter).  A run longer than
+    // kEcReadItems items takes several turns.
+    const DRead* rp = P.reads + c0 + lane;
+    bool live = false, count = false;   // more to come; its bases are counted
+    int k = 0;                          // next CIGAR operation
+    int cx = 0, cy = 0;                 // column and query position at it
+    int x = 0, y = 0, len = 0, left = 0;   // the run, and how much of it is still to be counted
+    if (c0 + lane < P.n_reads) {
+      const DRead R = *rp;
+      const int t = P.pos_target[R.gpos];
+      live = t >= 0 && P.target_scored[t];
+      count = live && R.x1 <= 1 && P.do_errors;
+      if (count && (int)R.rfile >= S) {   // covariate read_set out of range: ASSERT in the reference
+        err |= kErrReadSet;
+        count = false;
       }
-      if (count) {
-        if (R.flags & kReadReversed) ec_count_run<true>(P, sq, ql, R, R.gpos, R.y0, R.gend - R.gpos, 0, table, err);
-        else ec_count_run<false>(P, sq, ql, R, R.gpos, R.y0, R.gend - R.gpos, 0, table, err);
+      cx = R.gpos;
+      if (R.flags & kReadSimple) {
+        k = -1;
+        cy = R.y0;
       }
-      return;
     }
-    const ConstU32* c = (const ConstU32*)(P.cigar + R.cig_off);
-    const int n = R.n_cigar;
-    int x = R.gpos, y = 0;
-    for (int k = 0; k < n; k++) {
-      const uint32_t w = c[k];
-      const uint32_t op = w & 15u;
-      const int l = (int)(w >> 4);
-      if (op == OP_M || op == OP_EQ || op == OP_X) {
-        if (l > 0) {
-          if (lane == 0) {
-            atomicAdd(&diff[x], 1);
-            atomicAdd(&diff[x + l], -1);
+    while (__any(live)) {
+      bool fresh = false;
+      int last_indel = 0;
+      if (live && left == 0) {   // the next run
+        if (k < 0) {
+          x = cx;
+          y = cy;
+          len = rp->gend - x;
+          fresh = true;
+        } else {
+          const int n = rp->n_cigar;
+          const uint32_t* c = P.cigar + rp->cig_off;
+          for (; k < n && !fresh; k++) {
+            const uint32_t op = c[k] & 15u;
+            const int l = (int)(c[k] >> 4);
+            if (op == OP_M || op == OP_EQ || op == OP_X) {
+              if (l > 0) {
+                x = cx;
+                y = cy;
+                len = l;
+                last_indel = run_end_indel(c, k, n);
+                fresh = true;
+              }
+              cx += l;
+              cy += l;
+            } else if (op == OP_I || op == OP_S) {
+              cy += l;
+            } else if (op == OP_D || op == OP_N) {
+              cx += l;
+            }
           }
-          if (count) {
-            const int li = run_end_indel(c, k, n);
-            if (R.flags & kReadReversed) ec_count_run<true>(P, sq, ql, R, x, y, l, li, table, err);
-            else ec_count_run<false>(P, sq, ql, R, x, y, l, li, table, err);
+          if (!fresh) {
+            live = false;
+            if (cx != rp->gend) err |= kErrCigar;
           }
         }
-        x += l;
-        y += l;
-      } else if (op == OP_I || op == OP_S) {
-        y += l;
-      } else if (op == OP_D || op == OP_N) {
-        x += l;
+        left = (fresh && count) ? len : 0;
       }
-    }
-    if (x != R.gend) err |= kErrCigar;
-  };
-  const int grp = lane / kEcGroup, gl = lane - kEcGroup * grp;
-  for (int64_t c0 = gw * kEcChunk; c0 < P.n_reads; c0 += nw * kEcChunk) {
-    const int n = (int)min<int64_t>(kEcChunk, P.n_reads - c0);
-    // Counted single-run alignments of at most 168 bases go three to a wavefront (lanes
-    // 21g .. 21g+20 take one, eight query positions per lane), which fills the lanes that one
-    // 150-base alignment leaves idle; the chunk's other alignments then go one at a time.  The
-    // counts are integers, so the order does not matter.
-    bool fit = false;
-    if (lane < n) {
-      const DRead R = P.reads[c0 + lane];
-      const int t = pos_target[R.gpos];
-      fit = t >= 0 && scored[t] && (R.flags & kReadSimple) && R.x1 <= 1 && P.do_errors &&
-            (int)R.rfile < P.read_set_max && (R.y0 & 3) + (R.gend - R.gpos) <= 8 * kEcGroup;
-    }
-    unsigned long long fm = __ballot(fit);
-    unsigned long long sm = ((n == 64) ? ~0ull : ((1ull << n) - 1ull)) & ~fm;
-    while (fm) {
-      const int ja = __builtin_ctzll(fm);
-      fm &= fm - 1ull;
-      const int jb = fm ? __builtin_ctzll(fm) : -1;
-      if (jb >= 0) fm &= fm - 1ull;
-      const int jc = fm ? __builtin_ctzll(fm) : -1;
-      if (jc >= 0) fm &= fm - 1ull;
-      const int mine = (grp == 0) ? ja : (grp == 1) ? jb : (grp == 2) ? jc : -1;
-      if (mine < 0) continue;
-      const DRead R = P.reads[c0 + mine];
-      if (gl == 0) {
-        atomicAdd(&diff_u[R.gpos], 1);
-        atomicAdd(&diff_u[R.gend], -1);
+      const int py = y + len - left;   // query position of the part still to be counted
+      const int items = min(((py & 7) + left + 7) >> 3, left > 0 ? kEcReadItems : 0);
+      const int part = (items > 0) ? min(left, 8 * items - (py & 7)) : 0;
+      const int incl = wave_incl_scan(items);
+      const int total = __builtin_amdgcn_readlane(incl, 63);
+      if (total > 0) {
+        for (int i = lane; i < 2 * kEcSteps; i += 64) ec_first[wave][i] = 0;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        if (items > 0) {
+          const int start = incl - items;
+          const int at = __popcll(__ballot(true) & ((1ull << lane) - 1ull));
+          const int begin = (py & 7) + 8 * start;
+          ec_rec[wave][at] = make_uint4((uint32_t)rp->seq_off + (uint32_t)(py & ~7) - 8u * (uint32_t)start,
+                                        (uint32_t)(x + (py - y) - begin), (uint32_t)(begin + part),
+                                        ((uint32_t)begin << 1) | ((rp->flags & kReadReversed) ? 1u : 0u));
+          ec_row[wave][at] = (uint32_t)rp->rfile * (uint32_t)Q;
+          atomicOr(&ec_first[wave][start >> 5], 1u << (start & 31));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        struct Item {
+          uint2 b, q, r;
+          int lo, hi;
+          uint32_t rev, row;
+        };
+        int before = -1;   // runs whose items start before the step, less one
+        auto fetch = [&](int i0) {
+          Item it;
+          const uint32_t f0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)ec_first[wave][i0 >> 5]);
+          const uint32_t f1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)ec_first[wave][(i0 >> 5) + 1]);
+          const uint64_t f = ((uint64_t)f1 << 32) | f0, g = f >> 1;
+          const int id = before + (int)(f0 & 1u) +
+                         (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(g >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)g, 0u));
+          before += __popcll(f);
+          const int i = i0 + lane;
+          it.hi = 0;
+          if (i < total) {
+            const uint4 rec = ec_rec[wave][id];
+            it.row = ec_row[wave][id];
+            const uint32_t at = rec.x + 8u * (uint32_t)i;
+            it.b = *(const uint2*)(P.bases + at);
+            it.q = *(const uint2*)(P.quals + at);
+            it.r = load8(P.ref_idx + ((int)rec.y + 8 * i));   // from 7 columns before the run on; ref_idx is padded
+            it.lo = ((int)rec.w >> 1) - 8 * i;
+            it.hi = (int)rec.z - 8 * i;
+            it.rev = rec.w & 1u;
+          }
+          return it;
+        };
+        auto add = [&](const Item& it) {
+          if (it.hi > 0) ec_eight(it.b, it.q, it.r, it.lo, it.hi, it.rev != 0u, it.row, (uint32_t)Q, T, err);
+        };
+        Item a = fetch(0);
+        for (int i0 = 64; i0 < total; i0 += 64) {   // the next items' bytes are on the way while one is counted
+          const Item b = fetch(i0);
+          add(a);
+          a = b;
+        }
+        add(a);
       }
-      const uint8_t* sq = P.bases + R.seq_off;
-      const uint8_t* ql = P.quals + R.seq_off;
-      const int y = R.y0, yend = y + (R.gend - R.gpos), last = yend - 1;
-      const bool rev = (R.flags & kReadReversed) != 0;
-      const int q0 = (y & ~3) + 8 * gl;
-      if (q0 < yend) ec_group4(P, sq, ql, R.rfile, rev, R.gpos, y, last, (int)R.qe0, q0, table, err);
-      if (q0 + 4 < yend) ec_group4(P, sq, ql, R.rfile, rev, R.gpos, y, last, (int)R.qe0, q0 + 4, table, err);
+      left -= part;
+      // the difference array and the run's ends come last: the loads above would wait for these atomics
+      const int array = (fresh && rp->x1 > 1) ? P.n_pos + 1 : 0;
+      add_equal(P.cov_diff, fresh ? array + x : -1, 1);
+      add_equal(P.cov_diff, fresh ? array + x + len : -1, -1);
+      if (fresh && count) {
+        const DRead R = *rp;
+        const uint8_t* sq = P.bases + R.seq_off;
+        const uint8_t* ql = P.quals + R.seq_off;
+        const uint32_t row0 = (uint32_t)R.rfile * (uint32_t)Q;
+        ec_run_pairs(P, sq, ql, (R.flags & kReadReversed) != 0, x, y, len, last_indel, (int)R.qe0, row0, T, err);
+        ec_run_indel(P, sq, ql, R, x, y, len, last_indel, row0, T, err);
+      }
+      if (k < 0 && left == 0) live = false;   // a single run, counted
     }
-    while (sm) {
-      const int j = __builtin_ctzll(sm);
-      sm &= sm - 1ull;
-      one(c0 + j);
-    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < P.n_bins; i += blockDim.x)
-    if (table[i]) atomicAdd(&P.counts[i], (unsigned long long)table[i]);
+  // bin of (read set rs, reference class ri, observed class oi, quality q): rs + S*(ri + 5*oi + 25*q)
+  for (int i = threadIdx.x; i < P.n_bins; i += blockDim.x) {
+    const int row = i / (int)kEcRow, c = i - row * (int)kEcRow;
+    const int rs = row / Q, q = row - rs * Q;
+    long long v;
+    if (c == 24) {
+      v = T.pairs[row];
+      for (int oi = 0; oi < 4; oi++)
+        for (int ri = 0; ri < 4; ri++) v += T.bins[row * (int)kEcRow + ri + 5 * oi];
+    } else {
+      v = T.bins[i];
+    }
+    if (v) atomicAdd(&P.counts[rs + S * (c + 25 * q)], (unsigned long long)v);
+  }
   if (err) atomicOr(P.err, err);
 }
 
@@ -410,23 +495,6 @@ __global__ void __launch_bounds__(256) k_read_starts(EcParams P) {
 
 /* ------------------------------------------------------------------------------------------ */
 /* Coverage histogram: prefix scan of the difference arrays                                    */
-
-__device__ __forceinline__ int wave_sum(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
-// Inclusive scan across the 64 lanes of a wavefront.
-__device__ __forceinline__ int wave_incl_scan(int v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(v, o, 64);
-    if (lane >= o) v += u;
-  }
-  return v;
-}
 
 __global__ void __launch_bounds__(256) k_cov_tile_sums(CovParams C) {
   __shared__ int red[2][4];

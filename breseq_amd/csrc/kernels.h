@@ -51,8 +51,14 @@ struct CovParams {
   unsigned long long* start_counts; // per target: (position, strand) pairs without / with a start
 };
 constexpr int kCovTile = 4096;      // columns per block of the coverage scan (256 threads x 16)
-constexpr int kEcChunk = 32;        // consecutive alignments per wavefront work item of k_ec_reads
+constexpr int kEcChunk = 64;        // consecutive alignments per wavefront work item of k_ec_reads
 constexpr int kEcWaves = 4;         // wavefronts per k_ec_reads block (256 threads)
+constexpr int kEcGrid = 1280;       // most blocks of k_ec_reads: five per CU are resident
+constexpr int kEcReadItems = 40;    // most items of eight positions of an alignment that shares its wavefront's lanes
+constexpr int kEcSteps = kEcChunk * kEcReadItems / 64;   // steps of 64 items of a work item
+static_assert(kEcChunk <= 64 && kEcChunk * kEcReadItems % 64 == 0, "k_ec_reads has a lane per alignment");
+// LDS of a k_ec_reads block: 25 bins and one pair count per (read set, quality)
+constexpr size_t kEcRowBytes = 26 * sizeof(uint32_t);
 
 // One row of the strand-folded likelihood table: a read of quality q from read file rs with
 // MAPQ slot m observing read-strand base o reads row ((m*S + rs)*Q + q)*5 + o.  Hypotheses are in

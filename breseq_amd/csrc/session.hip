@@ -803,18 +803,17 @@ static void run_error_count(Session& S, const bsq_error_count_args* args, bsq_ec
     C.start_bits = S.d_start_bits.p;
     C.start_counts = S.d_start_counts.p;
   }
-  const size_t lds_table = (size_t)n_bins * sizeof(uint32_t);
+  const size_t lds_table = (size_t)Sm * Q * kEcRowBytes;
   const size_t lds_hist = (size_t)C.n_groups_lds * C.hist_lds * sizeof(uint32_t);
-  if (lds_table > 64 * 1024) throw BsqError(BSQ_ERR_LIMIT, "covariate table too large for LDS");
-  // Two work items per wavefront, in the grid that splits the items evenly over the wavefronts
-  // (rounded up to a multiple of the 8 XCDs, so that no wavefront takes a third item while the
-  // others idle).  Measured on the MI355X, balanced grids of 1-4 items per wavefront all ran about
-  // 20% faster than 2,048 blocks of 11-12 items per wavefront; the per-block flush of the LDS
-  // table does not limit it.
+  if ((size_t)n_bins * sizeof(uint32_t) > 64 * 1024) throw BsqError(BSQ_ERR_LIMIT, "covariate table too large for LDS");
+  // No more blocks than the device holds at once: every block adds its count table to the result's
+  // few cache lines when it ends, and 12,000 blocks of a 4.6 Mb, 100x sample doing so took as long as
+  // the counting (660 us against 385).  The work items are split evenly over the wavefronts, in a
+  // grid rounded up to a multiple of the 8 XCDs.
   const int64_t chunks = (S.n_dreads + kEcChunk - 1) / kEcChunk;
-  int64_t ec_blocks = std::max<int64_t>(1, (chunks + 2 * kEcWaves - 1) / (2 * kEcWaves));
+  const int64_t ec_per_wave = std::max<int64_t>(1, (chunks + kEcGrid * kEcWaves - 1) / (kEcGrid * kEcWaves));
+  int64_t ec_blocks = std::max<int64_t>(1, (chunks + ec_per_wave * kEcWaves - 1) / (ec_per_wave * kEcWaves));
   if (ec_blocks >= 8) ec_blocks = (ec_blocks + 7) / 8 * 8;
-  if (ec_blocks > INT32_MAX) throw BsqError(BSQ_ERR_LIMIT, "too many reads for one error_count launch");
   const int ec_grid = (int)ec_blocks;
   S.timing.host_pre_ms = now_ms() - th0;
   HIP_OK(hipEventRecord(S.ev0, S.stream));
