@@ -61,15 +61,15 @@ static_assert(kEcChunk <= 64 && kEcChunk * kEcReadItems % 64 == 0, "k_ec_reads h
 constexpr size_t kEcRowBytes = 26 * sizeof(uint32_t);
 
 // One row of the strand-folded likelihood table: a read of quality q from read file rs with
-// MAPQ slot m observing read-strand base o reads row ((m*S + rs)*Q + q)*5 + o.  Hypotheses are in
+// MAPQ slot m observing read-strand base o reads row ((m*S + rs)*(Q + 1) + q + 1)*5 + o; the five rows
+// before quality 0 of a (m, rs) block are zeros.  Hypotheses are in
 // read-strand order; a reverse-strand read maps hypothesis b to t[comp(b)].  FP32: the column pass
 // sums these with an explicit error bound and certifies its decisions (exact FP64 values are used
 // by the scorer and k_fix_columns).
 struct FoldRow {
   float t[5];     // log10 P(o | hypothesis), fill_read_base_likelihoods (identify_mutations.cpp:3359-3384)
   float lpmax;    // max_b t[b]
-  float diag;     // t[o]: the read's own observation as the hypothesis
-  float pad;
+  float pad[2];
 };
 static_assert(sizeof(FoldRow) == 32, "FoldRow is two 16-byte LDS words");
 
@@ -81,11 +81,14 @@ struct IdRec {
   int32_t qoff;             // simple alignments: query position = column + qoff
   uint32_t trim;            // slot 0: trimmed when qpos < (trim & 0xFFFF) or qpos >= (trim >> 16)
                             // (alignment.h:389-410)
-  uint32_t row_base;        // ((mslot*S + read file)*Q)*5, 0xFFFFFFFF when the read file is >= S
-  uint32_t x1_flags;        // X1 | (kReadReversed | kReadSimple) << 16
+  uint32_t row_block;       // mslot*S + read file, 0xFFFFFFFF when the read file is >= S
+  uint32_t x1_flags;        // X1 | (kReadReversed | kReadSimple) << 16 | kIdPlain
   uint32_t pad;
 };
 static_assert(sizeof(IdRec) == 32, "IdRec is eight dwords");
+// A unique single-run alignment of a read file in the table, all of whose base codes are legal and
+// whose qualities are all below the maximum (and that below 129).
+constexpr uint32_t kIdPlain = 1u << 24;
 
 struct ImParams {
   const DRead* reads;
@@ -106,9 +109,9 @@ struct ImParams {
   const double* tab_r;          // per key: 10^(lp - lpmax) for b = 0..4, then lpmax
   int32_t tab_keys;             // rows of tab_lp / tab_r
   int32_t n_reads;              // alignments in reads[] (and idrec[])
-  const FoldRow* fold;          // strand-folded rows (mslot, read file, quality, read-strand obs);
-                                // row fold_rows is all zeros (the row of a read that adds nothing)
+  const FoldRow* fold;          // strand-folded rows (mslot, read file, quality, read-strand obs)
   int32_t fold_rows;
+  int32_t col_split;            // 1: a window's alignments are shared by the wavefronts of its block
   int32_t fold_lds;             // 1: stage the folded table in LDS
   double log10_ref_length;
   double mutation_cutoff;
@@ -168,17 +171,30 @@ struct RunParams {
 
 __global__ void k_fill_i32(int32_t* p, int64_t n, int32_t v);
 __global__ void k_repack_reads(const DRead* reads, const int64_t* raw_off, int64_t n_reads, const uint8_t* src_b,
-                               const uint8_t* src_q, uint8_t* dst_b, uint8_t* dst_q);
+                               const uint8_t* src_q, uint8_t* dst_b, uint8_t* dst_q, uint8_t* byte_max);
+constexpr int kBytesFrontPad = 16;    // bytes of the read arrays before the first alignment's (loads may start at -8)
 constexpr int kRefIdxFrontPad = 16;   // ref_idx bytes before column 0 (aligned loads may start at -4)
 __global__ void k_ec_reads(EcParams P);
 __global__ void k_cov_tile_sums(CovParams C);
 __global__ void k_cov_tile_scan(CovParams C);
 __global__ void k_cov_hist(CovParams C);
+constexpr int kColResident = 4096;           // wavefronts of the column kernel that the device holds
 constexpr int kColWaves = 8;                 // wavefronts per block of the column kernel (default; 4 also built)
-constexpr size_t kFoldLdsBytes = 48 * 1024;  // largest likelihood table staged in LDS (1535 rows)
+constexpr size_t kFoldLdsBytes = 48 * 1024;  // largest likelihood table staged in LDS
+constexpr size_t kFoldLdsRow = 152;          // its bytes per (MAPQ, read file, quality)
+// LDS words per column of a wavefront's window: the rare observations' sums and the counts, or, where a
+// block's wavefronts share a window, everything that they add up
+constexpr int kColWords = 11, kColSplitWords = 20;
+// alignments of a wavefront's list (16 bytes each): a batch of 64, 7 left over of either strand, and up to
+// 7 of no columns that fill the last eight of either up
+constexpr int kColList = 96;
+static_assert(kColList >= 64 + 2 * 7 + 2 * 7, "the two strands' alignments do not meet");
+inline size_t column_lds(int waves, bool split) {
+  return (size_t)waves * ((split ? kColSplitWords : kColWords) * 256 + kColList * 16 + 192);
+}
 template <bool kLds, int kWaves>
 __global__ void k_identify_columns_t(ImParams P);
-__global__ void k_prep_reads(const DRead* reads, int64_t n, int32_t S, int32_t Q, IdRec* out);
+__global__ void k_prep_reads(const DRead* reads, const uint8_t* byte_max, int64_t n, int32_t S, int32_t Q, IdRec* out);
 template <bool kKeysGlobal>
 __global__ void k_fix_columns_t(ImParams P);
 // A column that only the column pass's bound could not rule out: k_route_candidates tests it again

@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(64 * kRouteWaves) k_route_candidates(ImParams 
               use = o >= 0 && o < 4 && qpos >= (rc.x & 0xFFFFu) && qpos < (rc.x >> 16) &&
                     q - (uint32_t)P.base_quality_cutoff < qspan && rc.y != 0xffffffffu;
               obs = o;
-              key = rc.y * 2u + q * 10u + (uint32_t)o * 2u + ((flags & kReadReversed) ? 1u : 0u);
+              key = (rc.y * (uint32_t)P.quality_max + q) * 10u + (uint32_t)o * 2u + ((flags & kReadReversed) ? 1u : 0u);
             } else {
               // data errors of this read were reported by the column pass
               int strand_idx = 0;

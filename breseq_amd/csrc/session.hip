@@ -132,7 +132,8 @@ struct Session {
   // device buffers
   DBuf<DRead> d_reads;
   DBuf<uint32_t> d_cigar;
-  DBuf<uint8_t> d_bases, d_quals;
+  DBuf<uint8_t> d_bases, d_quals;   // kBytesFrontPad bytes, then the alignments
+  DBuf<uint8_t> d_byte_max;         // k_repack_reads
   DBuf<char> d_ref;
   DBuf<uint8_t> d_ref_idx;        // kRef* code per global column
   DBuf<int32_t> d_cov_diff;       // pass-1 coverage difference arrays (unique, redundant)
@@ -606,21 +607,22 @@ static void session_load(Session& S, const bsq_reference* ref, const bsq_alignme
   const size_t nbases = (size_t)a->seq_off[a->n_reads];
   // the column pass addresses a read's bytes with a 32-bit offset
   if (dev_bytes + 16 >= ((int64_t)1 << 32)) throw BsqError(BSQ_ERR_LIMIT, "more than 4 GiB of read bases");
-  S.d_bases.alloc((size_t)dev_bytes + 16);
-  S.d_quals.alloc((size_t)dev_bytes + 16);
-  HIP_OK(hipMemsetAsync(S.d_bases.p, 0, (size_t)dev_bytes + 16, S.stream));
-  HIP_OK(hipMemsetAsync(S.d_quals.p, 0, (size_t)dev_bytes + 16, S.stream));
+  S.d_bases.alloc((size_t)dev_bytes + kBytesFrontPad + 16);
+  S.d_quals.alloc((size_t)dev_bytes + kBytesFrontPad + 16);
+  S.d_byte_max.alloc((size_t)std::max<int64_t>(1, n_pack));
+  HIP_OK(hipMemsetAsync(S.d_bases.p + kBytesFrontPad + dev_bytes, 0, 16, S.stream));   // k_repack_reads writes the rest
+  HIP_OK(hipMemsetAsync(S.d_quals.p + kBytesFrontPad + dev_bytes, 0, 16, S.stream));
   if (nbases && n_pack > 0) {
     // the uploaded arrays stay with the session for its next sample (no allocation per load)
-    S.d_raw_b.alloc(nbases);
-    S.d_raw_q.alloc(nbases);
+    S.d_raw_b.alloc(nbases + 8);
+    S.d_raw_q.alloc(nbases + 8);
     S.d_raw_off.alloc(raw_off.size());
     upload_staged(S, S.d_raw_b.p, a->seq, nbases);
     upload_staged(S, S.d_raw_q.p, a->qual, nbases);
     HIP_OK(hipMemcpyAsync(S.d_raw_off.p, raw_off.data(), raw_off.size() * sizeof(int64_t), hipMemcpyHostToDevice,
                           S.stream));
     hipLaunchKernelGGL(k_repack_reads, dim3(2048), dim3(256), 0, S.stream, S.d_reads.p, S.d_raw_off.p, (int64_t)n_pack,
-                       S.d_raw_b.p, S.d_raw_q.p, S.d_bases.p, S.d_quals.p);
+                       S.d_raw_b.p, S.d_raw_q.p, S.d_bases.p + kBytesFrontPad, S.d_quals.p + kBytesFrontPad, S.d_byte_max.p);
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(S.stream));
   }
@@ -760,8 +762,8 @@ static void run_error_count(Session& S, const bsq_error_count_args* args, bsq_ec
   EcParams P;
   P.reads = S.d_reads.p;
   P.cigar = S.d_cigar.p;
-  P.bases = S.d_bases.p;
-  P.quals = S.d_quals.p;
+  P.bases = S.d_bases.p + kBytesFrontPad;
+  P.quals = S.d_quals.p + kBytesFrontPad;
   P.ref_idx = S.d_ref_idx.p + kRefIdxFrontPad;
   P.pos_target = S.d_pos_target.p;
   P.target_scored = S.d_target_scored.p;
@@ -840,7 +842,7 @@ static void run_error_count(Session& S, const bsq_error_count_args* args, bsq_ec
   S.idrec_sm = S.idrec_q = -1;
   if (queue_idrec) {
     S.d_idrec.alloc((size_t)std::max<int64_t>(1, S.n_dreads));
-    hipLaunchKernelGGL(k_prep_reads, dim3(1024), dim3(256), 0, S.stream, S.d_reads.p, S.n_dreads, Sm, Q, S.d_idrec.p);
+    hipLaunchKernelGGL(k_prep_reads, dim3(1024), dim3(256), 0, S.stream, S.d_reads.p, S.d_byte_max.p, S.n_dreads, Sm, Q, S.d_idrec.p);
     HIP_OK(hipGetLastError());
     S.idrec_sm = Sm;
     S.idrec_q = Q;
@@ -943,8 +945,8 @@ static void build_column_tables(const Session& S, const bsq_identify_args* a, Li
   const size_t nm = S.mapq_values.size();
   L.keys = nm * Sm * Q * 10;
   L.lp.assign(L.keys * 5, 0.0);
-  // one extra all-zero row: the row a filtered read reads
-  L.fold.assign(nm * Sm * Q * 5 + 1, FoldRow{{0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, 0.0f, 0.0f, 0.0f});
+  // zero rows before every block's first quality: the rows a filtered read reads
+  L.fold.assign(nm * Sm * (Q + 1) * 5, FoldRow{{0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, 0.0f, {0.0f, 0.0f}});
   // the bins and rows of one quality depend on nothing else (a thread pool's wake-up costs more
   // than the few thousand logarithms this takes, so the qualities run in order)
   std::vector<double> prob(a->n_bins);
@@ -972,10 +974,9 @@ static void build_column_tables(const Session& S, const bsq_identify_args* a, Li
               L.lp[bot * 5 + comp_class(b)] = l[b];
             }
             // read-strand row == top-strand row for a top-strand read
-            const size_t row = ((m * Sm + rs) * Q + q) * 5 + obs;
+            const size_t row = ((m * Sm + rs) * (Q + 1) + q + 1) * 5 + obs;
             for (int b = 0; b < 5; b++) L.fold[row].t[b] = (float)l[b];
             L.fold[row].lpmax = (float)mx;
-            L.fold[row].diag = (float)l[obs];
           }
         }
     }
@@ -1031,6 +1032,13 @@ struct GdQueued {
   size_t prefix = 0;    // text bytes copied back with the counters
 };
 
+// Whether the wavefronts of a block share each window's alignments.  With fewer windows than wavefronts
+// that the device holds (two blocks of eight per CU), a wavefront per window leaves the device idle, and
+// sharing took the column pass of 48 kb at 206x from 401 to 117 us and of 20 kb at 3,000x from 2182 to
+// 220 us; with more windows the batches of a shared window are too short and its sums are added up
+// twice: 701 kb (10,960 windows) took 576 us shared and 187 us not, 4.6 Mb 4345 and 1042 us.
+static bool column_split(const Session& S) { return S.n_windows < kColResident; }
+
 // Blocks of the column pass.  A set count is kept to at most one window per wavefront and rounded
 // down to a multiple of the 8 XCDs from 8 blocks up (the windows of one block then sit on one XCD's
 // L2).  The default takes the fewest windows per wavefront k that keeps the grid within 2048
@@ -1038,12 +1046,13 @@ struct GdQueued {
 // up to a multiple of 8: a wavefront with one window more than the others holds its block.
 static int64_t column_blocks(const Session& S) {
   const int64_t w = S.col_waves;
-  const int64_t full = std::max<int64_t>(1, (S.n_windows + w - 1) / w);
+  const int64_t full = column_split(S) ? std::max<int64_t>(1, S.n_windows) : std::max<int64_t>(1, (S.n_windows + w - 1) / w);
   if (S.col_blocks > 0) {
     int64_t g = std::min<int64_t>(full, (int64_t)S.col_blocks);
     if (g >= 8) g &= ~(int64_t)7;
     return g;
   }
+  if (column_split(S)) return full;
   const int64_t k = std::max<int64_t>(1, (S.n_windows + w * 2048 - 1) / (w * 2048));
   int64_t g = std::max<int64_t>(1, (S.n_windows + w * k - 1) / (w * k));
   if (g >= 8) g = (g + 7) / 8 * 8;
@@ -1223,7 +1232,7 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   HIP_OK(hipEventRecord(S.ev0, S.stream));
   if (S.idrec_sm != Sm || S.idrec_q != Q) {   // not already queued by the pipeline's error_count
     S.d_idrec.alloc((size_t)std::max<int64_t>(1, S.n_dreads));
-    hipLaunchKernelGGL(k_prep_reads, dim3(1024), dim3(256), 0, S.stream, S.d_reads.p, S.n_dreads, Sm, Q, S.d_idrec.p);
+    hipLaunchKernelGGL(k_prep_reads, dim3(1024), dim3(256), 0, S.stream, S.d_reads.p, S.d_byte_max.p, S.n_dreads, Sm, Q, S.d_idrec.p);
     HIP_OK(hipGetLastError());
   }
   S.idrec_sm = S.idrec_q = -1;   // a later pass builds its own
@@ -1274,8 +1283,8 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   P.reads = S.d_reads.p;
   P.idrec = S.d_idrec.p;
   P.cigar = S.d_cigar.p;
-  P.bases = S.d_bases.p;
-  P.quals = S.d_quals.p;
+  P.bases = S.d_bases.p + kBytesFrontPad;
+  P.quals = S.d_quals.p + kBytesFrontPad;
   P.ref = S.d_ref.p;
   P.pos_target = S.d_pos_target.p;
   P.targets = S.d_targets.p;
@@ -1291,8 +1300,8 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   P.tab_keys = (int32_t)L.keys;
   P.n_reads = (int32_t)S.n_dreads;
   P.fold = S.d_fold.p;
-  P.fold_rows = (int32_t)fold.size() - 1;
-  const size_t fold_bytes = fold.size() * sizeof(FoldRow);
+  P.fold_rows = (int32_t)fold.size();
+  const size_t fold_bytes = fold.size() / 5 * kFoldLdsRow;
   P.fold_lds = (fold_bytes <= kFoldLdsBytes && S.col_lds) ? 1 : 0;
   P.log10_ref_length = log10(total_len);
   P.mutation_cutoff = a->mutation_cutoff;
@@ -1364,12 +1373,14 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
     const int64_t g = column_blocks(S);
     HIP_OK(hipEventRecord(S.evc, S.stream));
     const dim3 blk(S.col_waves * 64);
+    P.col_split = column_split(S) ? 1 : 0;
+    const size_t lds = column_lds(S.col_waves, P.col_split != 0) + (P.fold_lds ? (fold_bytes + 15) & ~(size_t)15 : 0);
     if (S.col_waves == 4) {
-      if (P.fold_lds) hipLaunchKernelGGL((k_identify_columns_t<true, 4>), dim3((int)g), blk, fold_bytes, S.stream, P);
-      else hipLaunchKernelGGL((k_identify_columns_t<false, 4>), dim3((int)g), blk, 0, S.stream, P);
+      if (P.fold_lds) hipLaunchKernelGGL((k_identify_columns_t<true, 4>), dim3((int)g), blk, lds, S.stream, P);
+      else hipLaunchKernelGGL((k_identify_columns_t<false, 4>), dim3((int)g), blk, lds, S.stream, P);
     } else {
-      if (P.fold_lds) hipLaunchKernelGGL((k_identify_columns_t<true, 8>), dim3((int)g), blk, fold_bytes, S.stream, P);
-      else hipLaunchKernelGGL((k_identify_columns_t<false, 8>), dim3((int)g), blk, 0, S.stream, P);
+      if (P.fold_lds) hipLaunchKernelGGL((k_identify_columns_t<true, 8>), dim3((int)g), blk, lds, S.stream, P);
+      else hipLaunchKernelGGL((k_identify_columns_t<false, 8>), dim3((int)g), blk, lds, S.stream, P);
     }
   }
   HIP_OK(hipGetLastError());
@@ -2160,7 +2171,7 @@ int bsq_session_alignment_trims(bsq_session* s, int32_t* xl, int32_t* xr, int64_
     d_xr.alloc((size_t)std::max<int64_t>(1, nd));
     if (nd > 0)
       hipLaunchKernelGGL(k_alignment_trims, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, S.stream, S.d_reads.p, nd,
-                         S.d_cigar.p, S.d_bases.p, d_trims.p, d_trims.p + S.n_pos, d_xl.p, d_xr.p);
+                         S.d_cigar.p, S.d_bases.p + kBytesFrontPad, d_trims.p, d_trims.p + S.n_pos, d_xl.p, d_xr.p);
     HIP_OK(hipGetLastError());
     std::vector<int32_t> hl((size_t)nd), hr((size_t)nd);
     if (nd > 0) {
