@@ -38,6 +38,18 @@ __device__ __forceinline__ DRead load_read(const DRead* reads, int r) {
   return d;
 }
 
+// Read bases by BAM code as 16 * class (T0 G1 C2 A3), N as 0xFF, four at once: v_perm_b32 takes its
+// selectors 13 and above as 0xFF, and 8 as the sign of table byte 1, here 0.
+__device__ __forceinline__ uint32_t read_classes(uint32_t b) { return __builtin_amdgcn_perm(0x00000010u, 0x00203000u, b); }
+
+// Nonzero when one of four base codes b, of read_classes rd, is none of A, C, G, T and N: the code that
+// the class stands for, against the code itself.
+__device__ __forceinline__ uint32_t not_bases(uint32_t b, uint32_t rd) {
+  const uint32_t back = __builtin_amdgcn_perm(0u, 0x01020408u, (rd >> 4) & 0x0F0F0F0Fu);
+  return ((back ^ b) & 0x0F0F0F0Fu) | (b & 0xF0F0F0F0u);
+}
+__device__ __forceinline__ uint32_t not_bases(uint32_t b) { return not_bases(b, read_classes(b)); }
+
 __device__ __forceinline__ bool is_ref_op(uint32_t op) {
   return op == OP_M || op == OP_D || op == OP_N || op == OP_EQ || op == OP_X;
 }

@@ -26,18 +26,6 @@
 
 namespace bsq {
 
-// Read bases by BAM code as 16 * class (T0 G1 C2 A3), N as 0xFF, four at once: v_perm_b32 takes its
-// selectors 13 and above as 0xFF, and 8 as the sign of table byte 1, here 0.
-__device__ __forceinline__ uint32_t read_classes(uint32_t b) { return __builtin_amdgcn_perm(0x00000010u, 0x00203000u, b); }
-
-// Nonzero when one of four base codes b, of read_classes rd, is none of A, C, G, T and N: the code that
-// the class stands for, against the code itself.
-__device__ __forceinline__ uint32_t not_bases(uint32_t b, uint32_t rd) {
-  const uint32_t back = __builtin_amdgcn_perm(0u, 0x01020408u, (rd >> 4) & 0x0F0F0F0Fu);
-  return ((back ^ b) & 0x0F0F0F0Fu) | (b & 0xF0F0F0F0u);
-}
-__device__ __forceinline__ uint32_t not_bases(uint32_t b) { return not_bases(b, read_classes(b)); }
-
 // Copies each alignment's bases and qualities to its 8-byte aligned offset (DRead::seq_off) in the
 // device layout, the bytes behind its last group's end as zeros.  Sixteen lanes take an alignment, in
 // groups of eight bytes, and note its largest quality (byte_max; 255 as well when a base code is none of

@@ -240,8 +240,8 @@ constexpr size_t kScoreKeyLds = 32 * 1024;      // most LDS for a candidate's re
 template <bool kKeysGlobal>
 __global__ void k_score_candidates_t(ImParams P);
 // reference and alignment trims (extra.hip)
-__global__ void k_repeat_extent(const char* s, int64_t len, uint8_t* m);
-__global__ void k_trim_gather(const uint8_t* m, int64_t len, uint8_t* left_out, uint8_t* right_out);
+constexpr int kTrimTile = 1024;              // positions of a k_sequence_trims block
+__global__ void k_sequence_trims(const char* s, int64_t len, uint8_t* left_out, uint8_t* right_out);
 __global__ void k_alignment_trims(const DRead* reads, int64_t n, const uint32_t* cigar, const uint8_t* bases,
                                   const uint8_t* left, const uint8_t* right, int32_t* xl, int32_t* xr);
 __global__ void k_read_starts(EcParams P);

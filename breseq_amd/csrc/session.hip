@@ -2154,17 +2154,14 @@ int bsq_session_alignment_trims(bsq_session* s, int32_t* xl, int32_t* xr, int64_
     if (!S.loaded) throw BsqError(BSQ_ERR_ARG, "session has no sample loaded");
     if (n != S.n_input_reads) throw BsqError(BSQ_ERR_ARG, "output arrays must hold one entry per loaded alignment");
     // the SequenceTrims of every target at its global columns: left row, then right row
-    DBuf<uint8_t> d_m, d_trims;
+    DBuf<uint8_t> d_trims;
     DBuf<int32_t> d_xl, d_xr;
-    d_m.alloc((size_t)S.n_pos);
     d_trims.alloc((size_t)2 * S.n_pos);
     for (int t = 0; t < S.n_targets; t++) {
       const int64_t len = S.lengths[t], off = S.tgt_off[t];
       if (len == 0) continue;
-      const unsigned blocks = (unsigned)((len + 255) / 256);
-      hipLaunchKernelGGL(k_repeat_extent, dim3(blocks), dim3(256), 0, S.stream, S.d_ref.p + off, len, d_m.p + off);
-      hipLaunchKernelGGL(k_trim_gather, dim3(blocks), dim3(256), 0, S.stream, d_m.p + off, len, d_trims.p + off,
-                         d_trims.p + S.n_pos + off);
+      hipLaunchKernelGGL(k_sequence_trims, dim3((unsigned)((len + kTrimTile - 1) / kTrimTile)), dim3(256), 0, S.stream,
+                         S.d_ref.p + off, len, d_trims.p + off, d_trims.p + S.n_pos + off);
     }
     const int64_t nd = S.n_dreads;
     d_xl.alloc((size_t)std::max<int64_t>(1, nd));
