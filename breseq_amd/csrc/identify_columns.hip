@@ -247,6 +247,17 @@ __device__ __forceinline__ double genotype_score_approx(const float lps[5], int 
   return ((double)lps[best] - (double)off) - (double)log10f(tot);
 }
 
+// A mask of lanes as one of columns, where lane 8 a + b has column 8 b + a: the transpose of the mask as
+// eight rows of eight bits, by swaps of 1x1, 2x2 and 4x4 blocks.
+__device__ __forceinline__ unsigned long long lanes_to_columns(unsigned long long m) {
+  unsigned long long t = (m ^ (m >> 7)) & 0x00AA00AA00AA00AAull;
+  m ^= t ^ (t << 7);
+  t = (m ^ (m >> 14)) & 0x0000CCCC0000CCCCull;
+  m ^= t ^ (t << 14);
+  t = (m ^ (m >> 28)) & 0x00000000F0F0F0F0ull;
+  return m ^ t ^ (t << 28);
+}
+
 __device__ __forceinline__ void finish_column(const ImParams& P, int p, int t, int ref_idx, const float lps[5],
                                               double red_bot, double red_top, int uniq, bool insert_slot,
                                               const Screen& A, uint32_t& err) {
@@ -298,7 +309,15 @@ __device__ __forceinline__ void finish_column(const ImParams& P, int p, int t, i
   const bool cand = sure || screen_passes(A, lps, ref_idx, P.log10_ref_length, P.polymorphism_cutoff, P.screen_margin);
   if (cand) {
     fl |= kPosCandidate;
-    const int slot = atomicAdd(P.n_cand, 1);
+    // In column order, for the candidate test: four neighbouring columns share a block of it, and so
+    // the lines of the same alignments.  (In lane order, columns eight apart, the test of 19,731
+    // candidates at 3,000x took 1814 us, in column order 1025.)
+    const unsigned long long m = __ballot(true);
+    const int leader = __builtin_ctzll(m);
+    int first = 0;
+    if ((int)(threadIdx.x & 63) == leader) first = atomicAdd(P.n_cand, __popcll(m));
+    const int slot = __builtin_amdgcn_readlane(first, leader) +
+                     __popcll(lanes_to_columns(m) & ((1ull << (p & (kWaveCols - 1))) - 1ull));
     if (slot < P.cand_cap) P.cand[slot] = make_int2(p, sure ? 0 : kCandScreened);
     else err |= kErrCapacity;
   }

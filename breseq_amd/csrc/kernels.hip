@@ -198,7 +198,7 @@ __device__ __forceinline__ bool may_be_emitted(const ImParams& P, const uint16_t
 // insertions, and the column pass's candidates, those that its bound alone let through tested
 // again by may_be_emitted.  At 3,000 reads a column the bound of the column pass rules out next to
 // nothing (19,743 of 20,011 columns passed it, of which some 30 are emitted) and the exact null fit of
-// each took the scorer 35.6 ms; this test takes 0.98 ms and leaves 36 (1 Mb at 300x with
+// each took the scorer 35.6 ms; this test takes 1.02 ms and leaves 36 (1 Mb at 300x with
 // 390 variants: 7,852 candidates, 0.17 ms, leaves 451).
 // LDS: a count per table key, and the list of the keys that occur.
 __global__ void __launch_bounds__(64 * kRouteWaves) k_route_candidates(ImParams P) {
