@@ -133,6 +133,11 @@ struct Session {
   DBuf<DRead> d_reads;
   DBuf<uint32_t> d_cigar;
   DBuf<uint8_t> d_bases, d_quals;   // kBytesFrontPad bytes, then the alignments
+  // bsq_session_alignment_trims, kept for the session's next call (allocating and freeing them took more
+  // than the kernels): the per-column trims, and both results of every alignment
+  DBuf<uint8_t> d_trims;
+  DBuf<int32_t> d_aln_trims;
+  PinnedBuf<int32_t> h_aln_trims;
   DBuf<uint8_t> d_byte_max;         // k_repack_reads
   DBuf<char> d_ref;
   DBuf<uint8_t> d_ref_idx;        // kRef* code per global column
@@ -2154,8 +2159,7 @@ int bsq_session_alignment_trims(bsq_session* s, int32_t* xl, int32_t* xr, int64_
     if (!S.loaded) throw BsqError(BSQ_ERR_ARG, "session has no sample loaded");
     if (n != S.n_input_reads) throw BsqError(BSQ_ERR_ARG, "output arrays must hold one entry per loaded alignment");
     // the SequenceTrims of every target at its global columns: left row, then right row
-    DBuf<uint8_t> d_trims;
-    DBuf<int32_t> d_xl, d_xr;
+    DBuf<uint8_t>& d_trims = S.d_trims;
     d_trims.alloc((size_t)2 * S.n_pos);
     for (int t = 0; t < S.n_targets; t++) {
       const int64_t len = S.lengths[t], off = S.tgt_off[t];
@@ -2164,22 +2168,21 @@ int bsq_session_alignment_trims(bsq_session* s, int32_t* xl, int32_t* xr, int64_
                          S.d_ref.p + off, len, d_trims.p + off, d_trims.p + S.n_pos + off);
     }
     const int64_t nd = S.n_dreads;
-    d_xl.alloc((size_t)std::max<int64_t>(1, nd));
-    d_xr.alloc((size_t)std::max<int64_t>(1, nd));
+    S.d_aln_trims.alloc((size_t)std::max<int64_t>(1, 2 * nd));   // XL, then XR
+    S.h_aln_trims.alloc((size_t)std::max<int64_t>(1, 2 * nd));
+    int32_t* const dx = S.d_aln_trims.p;
     if (nd > 0)
       hipLaunchKernelGGL(k_alignment_trims, dim3((unsigned)((nd + 255) / 256)), dim3(256), 0, S.stream, S.d_reads.p, nd,
-                         S.d_cigar.p, S.d_bases.p + kBytesFrontPad, d_trims.p, d_trims.p + S.n_pos, d_xl.p, d_xr.p);
+                         S.d_cigar.p, S.d_bases.p + kBytesFrontPad, d_trims.p, d_trims.p + S.n_pos, dx, dx + nd);
     HIP_OK(hipGetLastError());
-    std::vector<int32_t> hl((size_t)nd), hr((size_t)nd);
-    if (nd > 0) {
-      HIP_OK(hipMemcpyAsync(hl.data(), d_xl.p, (size_t)nd * sizeof(int32_t), hipMemcpyDeviceToHost, S.stream));
-      HIP_OK(hipMemcpyAsync(hr.data(), d_xr.p, (size_t)nd * sizeof(int32_t), hipMemcpyDeviceToHost, S.stream));
-    }
+    if (nd > 0)
+      HIP_OK(hipMemcpyAsync(S.h_aln_trims.p, dx, (size_t)(2 * nd) * sizeof(int32_t), hipMemcpyDeviceToHost, S.stream));
     HIP_OK(hipStreamSynchronize(S.stream));
     for (int64_t i = 0; i < n; i++) xl[i] = xr[i] = -1;
+    const int32_t *hl = S.h_aln_trims.p, *hr = hl + nd;
     for (int64_t i = 0; i < nd; i++) {
-      xl[S.h_src[(size_t)i]] = hl[(size_t)i];
-      xr[S.h_src[(size_t)i]] = hr[(size_t)i];
+      xl[S.h_src[(size_t)i]] = hl[i];
+      xr[S.h_src[(size_t)i]] = hr[i];
     }
     set_status(status, BSQ_OK, "");
     return BSQ_OK;
