@@ -277,7 +277,7 @@ def main():
     k_score = avg([d[3] for d in im_k])
     k_runs = avg([d[4] for d in im_k])
     kernels = {"k_ec_reads": k_ec, "k_cov_scan+hist": k_cov, "k_identify_columns": k_col,
-               "k_insert_slots": k_ins, "k_score_candidates": k_score, "k_runs": k_runs}
+               "k_route_candidates": k_ins, "k_score_candidates": k_score, "k_runs": k_runs}
     bytes_ec = BYTES_PER_BASE * nab + BYTES_PER_READ * n_reads + BYTES_PER_COLUMN_EC * n_cols
     bytes_im = BYTES_PER_BASE * nab + BYTES_PER_READ * n_reads + BYTES_PER_COLUMN_IM * n_cols
     col_kernels = {"k_ec_reads": (k_ec, bytes_ec), "k_identify_columns": (k_col, bytes_im)}
