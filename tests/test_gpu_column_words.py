@@ -3,7 +3,7 @@ against the oracle: aligned spans of 1 to 200 columns at every offset to the 64-
 either end, N bases, low qualities, alignments left over from the groups of eight, and reads that the
 loops do not take (qualities of N bases past the maximum, qualities above 127); with a window shared by
 its block's wavefronts (few windows) and a wavefront per window (many), and quality cutoffs from none to
-all."""
+all; with likelihood tables of up to the most that is staged in LDS (7 MAPQs of 43 qualities) and beyond."""
 import re
 
 import numpy as np
@@ -62,7 +62,7 @@ def check(s, q_max, **kw):
 
 
 @pytest.mark.parametrize("length", [FEW, MANY])
-@pytest.mark.parametrize("n,n_mapq", [(60, 1), (900, 1), (900, 40)])
+@pytest.mark.parametrize("n,n_mapq", [(60, 1), (900, 1), (900, 7), (900, 8), (900, 40)])
 def test_spans_and_trims(length, n, n_mapq):
     print("[gpu] column words: length", length, "reads", n, "MAPQs", n_mapq, flush=True)
     assert check(sample(n + length, length, n, n_mapq=n_mapq), 43) > 3
