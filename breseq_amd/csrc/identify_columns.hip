@@ -643,7 +643,9 @@ __global__ void __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_e
         (h ? uniq4.y : uniq4.x) += valid >> 7;
         const uint32_t m = __builtin_amdgcn_perm(ok, ok << 8, 0x0B090A08u);   // bit 7 spread over its byte
         (h ? n4.y : n4.x) += m;
-        qz[h] = (q + 0x01010101u) & m;   // the zero rows where nothing is added
+        // The zero rows where nothing is added.  Counted qualities are below 128; bytes before the alignment
+        // are another's and may be 255, which must not carry into its first.
+        qz[h] = ((q & 0x7F7F7F7Fu) + 0x01010101u) & m;
         // the row of the class in read direction: A0 C1 G2 T3 forward, the complement reverse
         cz[h] = (rev ? cls : cls ^ 0x60606060u) & m;
         nr[h] = (cls ^ (h ? refs.y : refs.x)) & m;

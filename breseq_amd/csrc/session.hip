@@ -615,7 +615,10 @@ static void session_load(Session& S, const bsq_reference* ref, const bsq_alignme
   S.d_bases.alloc((size_t)dev_bytes + kBytesFrontPad + 16);
   S.d_quals.alloc((size_t)dev_bytes + kBytesFrontPad + 16);
   S.d_byte_max.alloc((size_t)std::max<int64_t>(1, n_pack));
-  HIP_OK(hipMemsetAsync(S.d_bases.p + kBytesFrontPad + dev_bytes, 0, 16, S.stream));   // k_repack_reads writes the rest
+  // the pads at either end; k_repack_reads writes the rest
+  HIP_OK(hipMemsetAsync(S.d_bases.p, 0, kBytesFrontPad, S.stream));
+  HIP_OK(hipMemsetAsync(S.d_quals.p, 0, kBytesFrontPad, S.stream));
+  HIP_OK(hipMemsetAsync(S.d_bases.p + kBytesFrontPad + dev_bytes, 0, 16, S.stream));
   HIP_OK(hipMemsetAsync(S.d_quals.p + kBytesFrontPad + dev_bytes, 0, 16, S.stream));
   if (nbases && n_pack > 0) {
     // the uploaded arrays stay with the session for its next sample (no allocation per load)
