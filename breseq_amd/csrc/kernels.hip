@@ -243,7 +243,8 @@ __global__ void __launch_bounds__(64 * kRouteWaves) k_route_candidates(ImParams 
           const uint4 ra = src[0], rc = src[1];
           past = (int)ra.x > p;
           const uint32_t xf = rc.z, flags = xf >> 16;
-          if ((uint32_t)p - ra.x < ra.y - ra.x && (xf & 0xFFFFu) == 1u) {
+          // X1 of 0 or 1, as pdata_key
+          if ((uint32_t)p - ra.x < ra.y - ra.x && (xf & 0xFFFFu) <= 1u) {
             if (flags & kReadSimple) {
               const uint32_t qpos = (uint32_t)p + ra.w;
               const uint32_t b = P.bases[ra.z + qpos], q = P.quals[ra.z + qpos];
