@@ -330,6 +330,8 @@ def lib():
     _decl(L, "bsq_session_alignment_trims", C.c_int, [vp, c_i32p, c_i32p, C.c_int64, st])
     _decl(L, "bsq_session_set_gd_writer", C.c_int, [vp, C.c_int32, st])
     _decl(L, "bsq_session_set_gd_capacity", C.c_int, [vp, C.c_int32, st])
+    _decl(L, "bsq_session_set_scorer_guards", C.c_int, [vp, C.c_double, C.c_double, st])
+    _decl(L, "bsq_session_scorer_levels", C.c_int, [vp, c_i64p])
     _decl(L, "bsq_session_set_column_launch", C.c_int, [vp, C.c_int32, C.c_int32, C.c_int32, st])
     _decl(L, "bsq_session_tune_columns", C.c_int, [vp, P(IdentifyArgs), C.c_int32, P(ColumnLaunch), st])
     _decl(L, "bsq_format_doubles_device", C.c_int, [c_f64p, C.c_int64, C.c_int32, C.c_int32, C.c_char_p, c_i32p, st])

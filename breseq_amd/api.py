@@ -284,6 +284,20 @@ class Session:
         L.check(L.lib().bsq_session_set_gd_capacity(self._h, int(entries), C.byref(st)), st)
         return self
 
+    def set_scorer_guards(self, log10_likelihood=1e-8, frequency=1e-12):
+        """Raise the least distance from a decision's boundary below which the exact scorer does a candidate
+        again with sums in read order (diagnostic: results do not change)."""
+        st = _status()
+        L.check(L.lib().bsq_session_set_scorer_guards(self._h, log10_likelihood, frequency, C.byref(st)), st)
+        return self
+
+    def scorer_levels(self):
+        """Candidates of the last identify pass by how they were decided: sums in any order, the full fit and
+        close comparisons in read order, all in read order."""
+        out = (C.c_int64 * 3)()
+        L.lib().bsq_session_scorer_levels(self._h, out)
+        return list(out)
+
     def set_column_launch(self, blocks=0, table_in_lds=True, waves=0):
         """Launch shape of later column passes: blocks (0: the default rule) of `waves` wavefronts
         (4 or 8; 0: 8), and the likelihood table in LDS when it fits, or in global memory."""

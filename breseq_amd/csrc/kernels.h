@@ -120,6 +120,7 @@ struct ImParams {
   int32_t places;               // digits of printed frequencies
   double screen_margin;
   int32_t screen_off;           // 1: every covered column goes to the exact scorer
+  double guard_log, guard_rel;  // least guards of the scorer's sums in any order (log10 likelihoods; frequencies, relative)
   // per-column outputs
   uint8_t* col_flags;
   int32_t* col_unique;
@@ -130,6 +131,7 @@ struct ImParams {
   // candidates of the exact scorer: (global column, insert slot)
   int2* score;
   int32_t* n_score;
+  int32_t* n_level;      // candidates by the scorer's level that decided them: 0, 1 and 2
   int32_t* score_next;   // work counter of the exact scorer: the next candidate a block takes (zeroed per pass)
   int32_t cand_cap;             // capacity of cand and of score
   int32_t* ins;                 // columns with insert slots
@@ -228,6 +230,7 @@ __global__ void k_coverage_columns(CovTabParams C);
 // Downsampled rows (step > 1): one wavefront per row, lanes over the row's reads.
 __global__ void k_coverage_rows(CovTabParams C);
 
+constexpr double kGuardLog = 1e-8, kGuardRel = 1e-12;   // ImParams::guard_log, guard_rel unless set
 constexpr int kScoreWaves = 4;               // wavefronts per candidate in the exact scorer
 // blocks of the exact scorer (each draws candidates from a work counter): four per CU are resident
 constexpr int kScoreGrid = 1024;

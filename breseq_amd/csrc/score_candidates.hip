@@ -9,11 +9,10 @@
 //   * The reference forms every sum in read order, and its output is decided by comparisons and by
 //     printed digits.  The EM loops run with sums in any order, over the candidate's distinct table
 //     keys weighted with their reads (em_full, em_tasks): the same iterations, whose results differ from
-//     the reference's by rounding (about 1e-15 in a frequency, 1e-11 in a log10 likelihood).  Every
-//     decision and every printed digit is then checked to lie farther from its boundary than a
-//     guard some hundred times that (kGuardLog, kGuardRel); the candidates where one does not, about one
-//     in a hundred with 8 printed digits, are done once more with the reference's sums, as are all of
-//     them when the screen is off.
+//     the reference's by rounding, by more the more reads a sum has.  Every decision and every printed
+//     digit is then checked to lie farther from its boundary than a bound on that (the guards below);
+//     the candidates where one does not, about one in a hundred at 100 reads and 8 printed digits, are
+//     done once more with the reference's sums, as are all of them when the screen is off.
 //   * em_exact makes the reference's sums: row g of a wavefront (16 lanes) holds allele g's terms of 16
 //     reads, and a chain of 16 additions whose operand is broadcast from lane k of the row
 //     (v_fmac_f64 with row_newbcast, times 1.0, which rounds like an addition) adds them in order,
@@ -51,17 +50,31 @@ constexpr int kTaskWaves = 3;            // wavefronts of the EM tasks; the four
 constexpr int kTaskSlots = 48;           // most tasks of a round: 4 lanes each, or 24 of 8 lanes
 constexpr int kKsDiag = 100;             // exact KS runs when m*n < 10000, so min(m, n) <= 99
 constexpr double kDrop = 0.587566;       // kProfileLikelihoodLog10Drop (identify_mutations.cpp:3173)
-// How far a result of sums in any order may be from the reference's, generously: the rounding of
-// 50 EM passes leaves a frequency within about 1e-15 (relative) and a log10 likelihood within about
-// 1e-11.  A decision or a printed digit closer to its boundary than this is made on exact sums.
-constexpr double kGuardLog = 1e-8;       // log10 likelihoods and scores
-constexpr double kGuardRel = 1e-12;      // frequencies, relative
+// How far a result of sums in any order may be from the reference's, which adds n terms one after the
+// other: every addition rounds by up to 2^-53 of the sum so far, and where the terms are alike, as those
+// of reads that agree, all in one direction.  The sums here are of fewer, larger terms.
+//   * A pass moves a frequency by up to n 2^-53 of itself, and what it moved stays in the passes after
+//     (EM does not enlarge it: in the frequencies' logarithms a step is the identity less a mean over
+//     the reads): passes * n * 2^-53, relative.
+//   * A log10 likelihood is off by up to n 2^-53 of its size, and by up to n^2 2^-53 because the
+//     frequencies add up to 1 only within n 2^-53; a score has two of them.  Guarded with twice that.
+//   * A loop ends when no frequency moved by tol: a step this close to it, after up to 100 passes (a
+//     profile's start from the full fit's), is not decided here.
+// Measured against correctly rounded sums, most of three mixes of qualities: 5e-14 of a frequency and 7e-11 of
+// a likelihood at 3,000 reads (bounds 1e-12 and 5e-9), 3e-12 and 3e-7 at 200,000 (7e-11 and 2e-5).
+// A decision or a printed digit closer to its boundary than its guard is made on exact sums.  Up to
+// some thousand reads the least guards of a launch hold (ImParams::guard_log, guard_rel).
+constexpr double kHalfUlp = 0x1p-53;
+constexpr double kSumSlack = 64.0;       // additions besides those of the reads: a term's own operations
+constexpr double kStopPasses = 100.0;
 
 struct ScoreShared {
   double full_f[5];
-  double fit[5];                   // frequencies em_exact starts from and leaves
+  double fit[6];                   // frequencies an EM loop starts from and leaves; em_full: its passes
   double full_ll, null_ll;
   double gscore;                   // pure-genotype score
+  double lp_best;                  // log10 likelihood of the best pure genotype
+  double guard_rel, guard_log;     // the candidate's guards; the score's own size comes on top
   double val[kTaskSlots];          // profile values of the round's tasks (without the lpmax sum)
   double pts[2][kTaskSlots];       // bisection midpoints of the round, per bound
   double vlo[2], vhi[2];           // profile values at the ends of each bound's interval
@@ -135,8 +148,9 @@ __device__ __forceinline__ double sum_lanes(double v) {
   return v;
 }
 
-// 1/s correctly rounded for a normal s well inside the exponent range: the hardware's reciprocal
-// estimate, two Newton steps, and the correction step of a division by s (numerator 1), each fused.
+// 1/s within about an ulp for a normal s well inside the exponent range: the hardware's reciprocal
+// estimate and two fused Newton steps.  em_terms, which needs it correctly rounded, adds the correction
+// step of a division by s (numerator 1).
 __device__ __forceinline__ double recip_newton(double s) {
   double y = __builtin_amdgcn_rcp(s);
   y = fma(fma(-s, y, 1.0), y, y);
@@ -488,9 +502,9 @@ struct LogSum {
 // fit_allele_frequencies (identify_mutations.cpp:3240-3318) over all alleles with sums in any order,
 // by one wavefront: 64 lanes share the distinct rows.  Leaves the frequencies in f and returns the
 // log10 likelihood without the sum of the reads' lpmax; NaN where the loop cannot stand for the
-// reference's (a read with s_i = 0, or a last step too close to tol).
+// reference's (a read with s_i = 0, or a step within `stop` of tol).  fit[5]: the passes made.
 template <int kKind>
-__device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble* fit, double tol) {
+__device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble* fit, double tol, double stop) {
   const Rows R = uniform_rows(Rv);
   const int K = uniform_i(Kv), lane = threadIdx.x & 63;
   const double per_n = 1.0 / (double)uniform_i(nv);
@@ -498,7 +512,8 @@ __device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble*
 #pragma unroll
   for (int b = 0; b < 5; b++) f[b] = fl[b] = fit[b];
   bool bad = false;
-  for (int it = 1;; it++) {
+  int it = 1;
+  for (;; it++) {
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     for (int i = lane; i < K; i += 64) {
       double r[6];
@@ -518,7 +533,7 @@ __device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble*
       sum += f[b];
       most = fmax(most, fabs(f[b] - fl[b]));
     }
-    bad = bad || !(sum > 0.5 && sum < 2.0) || (it < 50 && fabs(most - tol) < 1e-6 * tol);
+    bad = bad || !(sum > 0.5 && sum < 2.0) || (it < 50 && fabs(most - tol) < stop);
     if (!(most >= tol) || it >= 50) break;
   }
   LogSum L;
@@ -535,6 +550,7 @@ __device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble*
   if (lane == 0) {
 #pragma unroll
     for (int b = 0; b < 5; b++) fit[b] = f[b];
+    fit[5] = (double)it;
   }
   return __any(bad) ? __longlong_as_double(0x7ff8000000000000LL) : ll;
 }
@@ -545,11 +561,11 @@ __device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble*
 // sums in any order over the candidate's distinct rows.  prow: per row the ratio of the variant, those
 // of the other four alleles in order, and the row's reads.  Returns log10 of the likelihood without
 // the sum of the reads' lpmax, which every such value of a candidate shares; NaN where the value cannot
-// stand for the reference's (a read with s_i = 0, or a last step too close to tol).
+// stand for the reference's (a read with s_i = 0, or a step within `stop` of tol).
 //   start[4]: the other alleles' starting frequencies; scale: 1 / n in the null fit, else 0
 template <int kSub>
 __device__ __noinline__ double em_tasks(const LdsDouble* prow, int Kv, double x, double start0, double start1, double start2,
-                                        double start3, double scale_null, bool active, double tol) {
+                                        double start3, double scale_null, bool active, double tol, double stop) {
   const int K = uniform_i(Kv), sub = threadIdx.x & (kSub - 1);
   double f1 = start0, f2 = start1, f3 = start2, f4 = start3;
   const double rest = (1.0 - x) / 4.0;
@@ -622,7 +638,7 @@ __device__ __noinline__ double em_tasks(const LdsDouble* prow, int Kv, double x,
     const double g3 = some ? scale * a3 : rest, g4 = some ? scale * a4 : rest;
     const double most = fmax(fmax(fabs(g1 - f1), fabs(g2 - f2)), fmax(fabs(g3 - f3), fabs(g4 - f4)));
     // (not-a-number sums fail the first test)
-    bad |= run & (!(others >= 0.0) | ((others > 0.0) & (others < 0x1p-500)) | ((it < 50) & (fabs(most - tol) < 1e-6 * tol)));
+    bad |= run & (!(others >= 0.0) | ((others > 0.0) & (others < 0x1p-500)) | ((it < 50) & (fabs(most - tol) < stop)));
     run &= (most >= tol) & (it < 50);
     // a task that ends keeps this pass's frequencies: the likelihood is theirs
     f1 = run ? g1 : f1;
@@ -923,33 +939,33 @@ __device__ __noinline__ void stats_w(LdsShared* SS, const uint32_t* list, const 
   }
 }
 
-// Whether a value known to kGuardRel prints as the reference's: %.*e with `places` digits, whose
+// Whether a value known within `rel` of itself prints as the reference's: %.*e with `places` digits, whose
 // rounding boundary must not lie within the error.  A decade's end is no boundary: both sides of it
 // print alike.
-__device__ __noinline__ bool prints_surely_e(double v, int places) {
+__device__ __noinline__ bool prints_surely_e(double v, int places, double rel) {
   if (v == 0.0) return true;
   if (!(v > 1e-280) || places > 12) return false;
   const double e = floor(log10(v));
   const double scaled = v * pow(10.0, (double)places - e);
-  return fabs(scaled - floor(scaled) - 0.5) > 2.0 * kGuardRel * scaled;
+  return fabs(scaled - floor(scaled) - 0.5) > 2.0 * rel * scaled;
 }
 
-// The same of a score known to kGuardLog, printed with one decimal.
-__device__ __forceinline__ bool prints_surely_f1(double v) {
+// The same of a score known within `err`, printed with one decimal.
+__device__ __forceinline__ bool prints_surely_f1(double v, double err) {
   const double scaled = 10.0 * fabs(v);
-  return fabs(scaled - floor(scaled) - 0.5) > 10.0 * kGuardLog;
+  return fabs(scaled - floor(scaled) - 0.5) > 10.0 * err;
 }
 
 // Whether the full fit's decisions (which alleles count, and their order) hold for any frequencies
-// within kGuardRel of these, and the frequencies that are printed print alike.
-__device__ __noinline__ bool fit_is_sure(const LdsDouble* f, uint32_t n, int places) {
+// within `rel` of these, and the frequencies that are printed print alike.
+__device__ __noinline__ bool fit_is_sure(const LdsDouble* f, uint32_t n, int places, double rel) {
   const double thr = 0.5 / (double)n;
   for (int a = 0; a < 5; a++) {
     if (f[a] < fmin(0.5 * thr, 0.01)) continue;
-    if (fabs(f[a] - thr) <= 4.0 * kGuardRel * thr) return false;
+    if (fabs(f[a] - thr) <= 4.0 * rel * thr) return false;
     for (int b = 0; b < a; b++)
-      if (fabs(f[a] - f[b]) <= 4.0 * kGuardRel * f[a]) return false;
-    if (f[a] >= thr && !prints_surely_e(f[a], places)) return false;
+      if (fabs(f[a] - f[b]) <= 4.0 * rel * f[a]) return false;
+    if (f[a] >= thr && !prints_surely_e(f[a], places, rel)) return false;
   }
   return true;
 }
@@ -1169,9 +1185,12 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
     // close to its boundary (or every candidate is to be exact), once more with the reference's sums
     int major = 5, minor = 5, variant = 5;
     bool have_v = false;
+    const double nu = ((double)n + kSumSlack) * kHalfUlp;
+    const double stop = fmax(1e-6 * tol, 2.0 * kStopPasses * nu);
     // level 0: sums in any order; 1: the full fit and close comparisons with the reference's sums; 2: the
     // score's likelihoods too
-    for (int level = (P.screen_off || kind != kRowsLds) ? 2 : 0;;) {
+    int level = (P.screen_off || kind != kRowsLds) ? 2 : 0;
+    for (;;) {
       const bool in_order = level > 0;
       if (wave == 0) {
         // full fit, from 0.5 + one per observing read, normalized (identical values from every lane)
@@ -1190,7 +1209,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
           if (in_order) {
             ll = fit_exact(1, -1, 0.0);
           } else {
-            ll = em_full<kRowsLds>(RR, K, n, (LdsDouble*)SS.fit, tol);
+            ll = em_full<kRowsLds>(RR, K, n, (LdsDouble*)SS.fit, tol, stop);
             unsure = !(fabs(ll) < 1e300);
           }
         }
@@ -1209,6 +1228,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
         if (lane == 0) {
           SS.best = best;
           SS.gscore = gscore;
+          SS.lp_best = (n > 0) ? lps[best] : 0.0;
         }
       }
       __syncthreads();
@@ -1256,7 +1276,11 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
         SS.depth[0] = SS.depth[1] = 0;
         SS.out[0] = 0.0;
         SS.out[1] = 1.0;
-        if (!in_order && n > 0 && SS.unsure == 0 && !fit_is_sure((LdsDouble*)SS.full_f, (uint32_t)n, P.places)) SS.unsure = 1;
+        if (level == 0) SS.guard_rel = fmax(P.guard_rel, SS.fit[5] * nu);
+        SS.guard_log = fmax(P.guard_log, 4.0 * nu * ((double)n + fabs(SS.lp_best)));
+        if (!in_order && n > 0 && SS.unsure == 0 &&
+            !fit_is_sure((LdsDouble*)SS.full_f, (uint32_t)n, P.places, SS.guard_rel))
+          SS.unsure = 1;
       }
       __syncthreads();
       // ---- rounds: the null fit, the profiles at the ML frequency, 0 and 1 and the bounds' midpoints |
@@ -1371,8 +1395,8 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
                                   : (other > 0.0) ? (1.0 - x) * SS.full_f[at] / other : (1.0 - x) / 4.0;
               }
               const double sc = null_task ? 1.0 / (double)n : 0.0;
-              const double val = both ? em_tasks<4>(pr, K, x, st[0], st[1], st[2], st[3], sc, active, tol)
-                                      : em_tasks<8>(pr, K, x, st[0], st[1], st[2], st[3], sc, active, tol);
+              const double val = both ? em_tasks<4>(pr, K, x, st[0], st[1], st[2], st[3], sc, active, tol, stop)
+                                      : em_tasks<8>(pr, K, x, st[0], st[1], st[2], st[3], sc, active, tol, stop);
               if (first && active) {
                 if (null_task) SS.null_ll = val;
                 else SS.val[slot_i] = val;
@@ -1387,7 +1411,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
           const bool walker = (lane & 31) == 0;
           bool close = false;   // a comparison the tasks' values do not decide
           const bool tasks = kind == kRowsLds;
-          const double guard = P.screen_off ? INFINITY : kGuardLog;
+          const double guard = P.screen_off ? INFINITY : SS.guard_log;
           Bound B;
           if (round == 0) {
             // (used if emitted)
@@ -1441,7 +1465,8 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
           }
           // neither end of the search may hang on the last bits of the ML frequency
           const double width = B.hi - B.lo;
-          if (!in_order && (fabs(width - tol) < 1e-11 || fabs(2.0 * width - tol) < 1e-11)) close = true;
+          const double bits = fmax(1e-11, 4.0 * SS.guard_rel);
+          if (!in_order && (fabs(width - tol) < bits || fabs(2.0 * width - tol) < bits)) close = true;
           if (walker) {
             SS.lo[side] = B.lo;
             SS.hi[side] = B.hi;
@@ -1465,11 +1490,14 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
             SS.done = (!emitted || !have_v || !open) ? 1 : 0;
             int unsure = 0;
             if (level < 2 && have_v) {
-              if (!(fabs(score - P.polymorphism_cutoff) > kGuardLog) || (emitted && !prints_surely_f1(score))) unsure = 2;
+              const double err = SS.guard_log + 4.0 * nu * fabs(score);
+              if (!(fabs(score - P.polymorphism_cutoff) > err) || (emitted && !prints_surely_f1(score, err))) unsure = 2;
             }
             if (level == 0 && have_v && emitted && unsure == 0) {
               if (u) unsure = 1;
-              if (SS.done && !(prints_surely_e(out0, P.places) && (out1 == 1.0 || prints_surely_e(out1, P.places)))) unsure = 1;
+              if (SS.done && !(prints_surely_e(out0, P.places, SS.guard_rel) &&
+                                (out1 == 1.0 || prints_surely_e(out1, P.places, SS.guard_rel))))
+                unsure = 1;
             }
             SS.unsure = unsure;
             if (unsure) SS.done = 1;
@@ -1511,6 +1539,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
       out.total_top = tt;
       out.total_bot = tb;
       P.ra_out[ci] = out;
+      atomicAdd(&P.n_level[level], 1);
     }
     __syncthreads();
   }

@@ -124,7 +124,7 @@ struct Session {
   PinnedBuf<TargetInfo> h_targets;     // per-target parameters with the fitted cutoffs
   PinnedBuf<double> h_tab_lp;          // the likelihood tables of the column pass
   PinnedBuf<FoldRow> h_fold;
-  PinnedBuf<int32_t> h_counters;       // [0..7] the pass's counters, [8] MC/UN runs found
+  PinnedBuf<int32_t> h_counters;       // [0..9] the pass's counters, [10] MC/UN runs found
   std::vector<int32_t> h_gpos;        // global first column of each packed read (sorted)
   std::vector<int64_t> h_src;         // input alignment index of each packed read
   int64_t n_input_reads = 0;          // alignments the sample was loaded from (packed or not)
@@ -163,7 +163,7 @@ struct Session {
   DBuf<int32_t> d_col_unique, d_col_total;
   DBuf<int2> d_cand, d_score;
   DBuf<int32_t> d_counters;   // [0] n_cand, [1] n_ins, [2] n_runs, [3] error bits, [4] n_fix,
-                              // [5] score_next, [6] n_score
+                              // [5] score_next, [6] n_score, [7..9] n_level
   DBuf<int32_t> d_fix;
   DBuf<IdRec> d_idrec;
   DBuf<uint32_t> d_ct_u, d_ct_raw, d_ct_beg;   // BAM2COV column counts (coverage table)
@@ -176,6 +176,8 @@ struct Session {
   int32_t col_blocks = 0;   // 0: one window per wavefront, at most 2048 blocks
   int32_t col_lds = 1;      // 1: the likelihood table staged in LDS when it fits; 0: read from global memory
   int32_t col_waves = kColWaves;   // wavefronts per block: 8 or 4
+  double guard_log = kGuardLog, guard_rel = kGuardRel;   // bsq_session_set_scorer_guards
+  int64_t score_levels[3] = {0, 0, 0};                   // of the last identify pass
   // device writer of the genome diff (gd_emit.hip)
   bool gd_on_device = true;
   int gd_cap = 4096;                       // entries the writer's lists hold (grows when a pass needs more)
@@ -665,7 +667,7 @@ static void session_load(Session& S, const bsq_reference* ref, const bsq_alignme
   HIP_OK(hipMemcpyAsync(S.d_win_rb.p, rb.data(), rb.size() * sizeof(int32_t), hipMemcpyHostToDevice, S.stream));
   HIP_OK(hipMemcpyAsync(S.d_win_re.p, re.data(), re.size() * sizeof(int32_t), hipMemcpyHostToDevice, S.stream));
   S.d_err.alloc(1);
-  S.d_counters.alloc(8);
+  S.d_counters.alloc(10);
   HIP_OK(hipStreamSynchronize(S.stream));
   S.timing.pack_ms = t1 - t0;
   S.timing.h2d_ms = now_ms() - t2;
@@ -1326,6 +1328,9 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   P.score = S.d_score.p;
   P.n_score = S.d_counters.p + 6;
   P.score_next = S.d_counters.p + 5;
+  P.n_level = S.d_counters.p + 7;
+  P.guard_log = S.guard_log;
+  P.guard_rel = S.guard_rel;
   P.cand_cap = cand_cap;
   P.ins = S.d_ins.p;
   P.n_ins = S.d_counters.p + 1;
@@ -1374,7 +1379,7 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
     P.audit = S.d_audit.p;
   }
   S.last_P = P;
-  HIP_OK(hipMemsetAsync(S.d_counters.p, 0, 8 * sizeof(int32_t), S.stream));
+  HIP_OK(hipMemsetAsync(S.d_counters.p, 0, 10 * sizeof(int32_t), S.stream));
   const double th1 = now_ms();
   // the whole pass is queued without a host round trip: later kernels read the counts on device
   {
@@ -1437,9 +1442,9 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   hipLaunchKernelGGL(k_runs, dim3((S.n_pos + 255) / 256), dim3(256), 0, S.stream2, R);
   HIP_OK(hipGetLastError());
   HIP_OK(hipEventRecord(S.evk[5], S.stream2));
-  S.h_counters.alloc(9);
+  S.h_counters.alloc(11);
   int32_t* counters = S.h_counters.p;
-  HIP_OK(hipMemcpyAsync(counters + 8, S.d_counters.p + 2, sizeof(int32_t), hipMemcpyDeviceToHost, S.stream2));
+  HIP_OK(hipMemcpyAsync(counters + 10, S.d_counters.p + 2, sizeof(int32_t), hipMemcpyDeviceToHost, S.stream2));
   std::vector<int32_t> order = target_order(S, a->call_target);
   std::vector<int64_t> rank(S.n_targets, -1);
   for (size_t i = 0; i < order.size(); i++) rank[order[i]] = (int64_t)i;
@@ -1459,10 +1464,10 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
     gd_in.places = a->polymorphism_precision_places;
     gd_q = queue_gd_on_device(S, gd_in);
   }
-  HIP_OK(hipMemcpyAsync(counters, S.d_counters.p, 8 * sizeof(int32_t), hipMemcpyDeviceToHost, S.stream));
+  HIP_OK(hipMemcpyAsync(counters, S.d_counters.p, 10 * sizeof(int32_t), hipMemcpyDeviceToHost, S.stream));
   std::vector<GdEntry> run_entries;
   HIP_OK(hipStreamSynchronize(S.stream2));
-  const int32_t n_runs_seen = counters[8];
+  const int32_t n_runs_seen = counters[10];
   const double tr0 = now_ms();
   if (!S.gd_on_device && n_runs_seen <= run_cap) {   // past the cap the call fails below, with the other limit checks
     std::vector<RunRec> runs(n_runs_seen);
@@ -1539,6 +1544,7 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   raise_err_bits(errbits);
   const int n_cand = counters[6];
   S.timing.candidates = n_cand;
+  for (int k = 0; k < 3; k++) S.score_levels[k] = counters[7 + k];
   if (S.gd_on_device) {
     const double t1 = now_ms();
     int64_t n_ra = 0, n_mc = 0, n_un = 0;
@@ -2212,6 +2218,23 @@ int bsq_session_set_gd_capacity(bsq_session* s, int32_t entries, bsq_status* sta
   }
   s->s.gd_cap = entries;
   set_status(status, BSQ_OK, "");
+  return BSQ_OK;
+}
+
+int bsq_session_set_scorer_guards(bsq_session* s, double log10_likelihood, double frequency, bsq_status* status) {
+  if (!s || !(log10_likelihood >= kGuardLog) || !(frequency >= kGuardRel)) {
+    set_status(status, BSQ_ERR_ARG, "null session, or a guard below its default");
+    return BSQ_ERR_ARG;
+  }
+  s->s.guard_log = log10_likelihood;
+  s->s.guard_rel = frequency;
+  set_status(status, BSQ_OK, "");
+  return BSQ_OK;
+}
+
+int bsq_session_scorer_levels(const bsq_session* s, int64_t counts[3]) {
+  if (!s || !counts) return BSQ_ERR_ARG;
+  for (int k = 0; k < 3; k++) counts[k] = s->s.score_levels[k];
   return BSQ_OK;
 }
 
