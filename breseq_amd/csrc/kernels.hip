@@ -88,8 +88,8 @@ __device__ __forceinline__ void wave_lds_sync() {
 
 // One EM pass over a column's distinct keys (lane = key, 64 at a time): S[b] = Sum_i r_i(b) / s_i,
 // s_i = Sum_b f_b r_i(b), and the log10 likelihood Sum_i log10 s_i (without the lpmax sum), each key
-// weighted with its reads.  The logarithms are FP32 (each within 2e-6 for s_i above 1e-30).  False
-// when a read has no likelihood to speak of.
+// weighted with its reads.  The logarithms are FP32: within an ulp of log2 s_i, 3.8e-6 below 64, and the
+// rounding of s_i, so each log10 within 2e-6 for s_i between 2^-64 and 2^64.  False when a read's is not.
 __device__ __forceinline__ bool key_pass(const ImParams& P, const uint16_t* keys, const uint32_t* hist, int K, int lane,
                                          const double f[5], double S[5], double& ll) {
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, l2 = 0.0;
@@ -106,7 +106,7 @@ __device__ __forceinline__ bool key_pass(const ImParams& P, const uint16_t* keys
       r[b] = t[b];
       s = fma(f[b], r[b], s);
     }
-    bad = bad || !(s > 1e-30 && s < 1e30);
+    bad = bad || !(s > 0x1p-64 && s < 0x1p64);
     double y = __builtin_amdgcn_rcp(s);
     y = fma(fma(-s, y, 1.0), y, y);
     y = fma(fma(-s, y, 1.0), y, y) * h;
