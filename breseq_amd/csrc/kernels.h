@@ -132,6 +132,7 @@ struct ImParams {
   int2* score;
   int32_t* n_score;
   int32_t* n_level;      // candidates by the scorer's level that decided them: 0, 1 and 2
+  int32_t route_slots;   // hash slots of a wavefront of the candidate test, a power of two (0: one per table key)
   int32_t* score_next;   // work counter of the exact scorer: the next candidate a block takes (zeroed per pass)
   int32_t cand_cap;             // capacity of cand and of score
   int32_t* ins;                 // columns with insert slots
@@ -201,11 +202,17 @@ template <bool kKeysGlobal>
 __global__ void k_fix_columns_t(ImParams P);
 // A column that only the column pass's bound could not rule out: k_route_candidates tests it again
 constexpr int32_t kCandScreened = 1;
-__global__ void k_route_candidates(ImParams P);
-__host__ __device__ inline size_t route_words(int tab_keys) { return (size_t)tab_keys + (size_t)(tab_keys + 1) / 2; }
-constexpr int kRouteWaves = 4;              // wavefronts per block of k_route_candidates, a candidate each
-constexpr int kRouteGrid = 2048;            // its blocks
-constexpr int kRouteKeys = 2048;            // most table keys a wavefront's LDS histogram holds (6 bytes each)
+template <bool kHash>
+__global__ void k_route_candidates_t(ImParams P);
+// LDS words of a wavefront: a count and a 16-bit list entry per slot, and a key where slots are hashed
+__host__ __device__ inline size_t route_words(bool hash, int slots) {
+  return (size_t)slots * (hash ? 2 : 1) + (size_t)(slots + 1) / 2;
+}
+constexpr int kRouteWaves = 4;              // most wavefronts per block of k_route_candidates, a candidate each
+constexpr int kRouteGrid = 8192;            // its wavefronts
+constexpr int kRouteKeys = 2048;            // most table keys counted in a slot each (12 KiB a wavefront)
+constexpr int kRouteSlots = 4096;           // most hash slots of a column's keys (40 KiB)
+constexpr int kRouteProbes = 256;           // slots tried before a column counts as having too many keys
 // BAM2COV per-column counts over a region (coverage_output.cpp:307-503): lane = column, the window's
 // reads in file order.
 struct CovTabParams {
@@ -237,7 +244,8 @@ constexpr int kScoreGrid = 1024;
 constexpr int kFixGrid = 256;                // blocks of k_fix_columns (at most kScoreGrid)
 constexpr size_t kScoreStaticLds = 6656;   // bound on the scorer's static LDS
 constexpr size_t kScoreLdsBudget = 39 * 1024;   // static + dynamic LDS of a scorer block: four per CU
-constexpr size_t kScoreLdsDeep = 64 * 1024;     // the same for samples whose read lists need more
+constexpr size_t kScoreLdsDeep = 79 * 1024;     // the same for samples that need more: two per CU
+constexpr size_t kScoreLdsMost = 158 * 1024;    // one per CU
 constexpr size_t kScoreRowBytes = 120;          // dynamic LDS of a distinct key of the candidate
 constexpr size_t kScoreKeyLds = 32 * 1024;      // most LDS for a candidate's read list
 template <bool kKeysGlobal>

@@ -86,20 +86,55 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// A wavefront's count per distinct key of a column, in LDS.  kHash: slots found by linear probing from the key's
+// hash (tables of many keys); else a slot per key of the table.
+template <bool kHash>
+struct KeyCounts {
+  uint32_t* count;     // per slot; 0: unused
+  uint32_t* keys;      // kHash: the slot's key
+  uint16_t* list;      // the used slots
+  int slots;           // kHash: a power of two
+  int shift;           // kHash: 32 - log2 slots
+  static constexpr uint32_t kNone = 0xffffffffu;
+  __device__ __forceinline__ uint32_t key(uint32_t slot) const { return kHash ? keys[slot] : slot; }
+  // counts the key of every lane with `use`; false when one found no slot
+  __device__ __forceinline__ bool add(bool use, uint32_t k) const {
+    if constexpr (!kHash) {
+      if (use) atomicAdd(&count[k], 1u);
+      return true;
+    } else {
+      uint32_t slot = (k * 0x9E3779B1u) >> shift;
+      for (int probe = 0; probe < kRouteProbes && __any(use); probe++) {
+        if (use) {
+          const uint32_t old = atomicCAS(&keys[slot], kNone, k);
+          if (old == kNone || old == k) {
+            atomicAdd(&count[slot], 1u);
+            use = false;
+          } else {
+            slot = (slot + 1u) & (uint32_t)(slots - 1);
+          }
+        }
+      }
+      return !__any(use);
+    }
+  }
+};
+
 // One EM pass over a column's distinct keys (lane = key, 64 at a time): S[b] = Sum_i r_i(b) / s_i,
 // s_i = Sum_b f_b r_i(b), and the log10 likelihood Sum_i log10 s_i (without the lpmax sum), each key
 // weighted with its reads.  The logarithms are FP32: within an ulp of log2 s_i, 3.8e-6 below 64, and the
 // rounding of s_i, so each log10 within 2e-6 for s_i between 2^-64 and 2^64.  False when a read's is not.
-__device__ __forceinline__ bool key_pass(const ImParams& P, const uint16_t* keys, const uint32_t* hist, int K, int lane,
-                                         const double f[5], double S[5], double& ll) {
+template <bool kHash>
+__device__ __forceinline__ bool key_pass(const ImParams& P, const KeyCounts<kHash>& C, int K, int lane, const double f[5],
+                                         double S[5], double& ll) {
   double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, l2 = 0.0;
   bool bad = false;
   for (int k0 = 0; k0 < K; k0 += WAVE) {
     const int k = k0 + lane;
     if (k >= K) continue;
-    const uint32_t key = keys[k];
-    const double h = (double)hist[key];
-    const double* t = P.tab_r + (size_t)key * 6;
+    const uint32_t slot = C.list[k];
+    const double h = (double)C.count[slot];
+    const double* t = P.tab_r + (size_t)C.key(slot) * 6;
     double r[5], s = 0.0;
 #pragma unroll
     for (int b = 0; b < 5; b++) {
@@ -133,8 +168,9 @@ __device__ __forceinline__ bool key_pass(const ImParams& P, const uint16_t* keys
 // The reads' likelihoods depend on their table keys alone, so the passes run over the distinct keys
 // with their counts.  The comparison keeps the margin of the column pass's screen, plus the
 // rounding of the FP32 logarithms (2e-6 a read and likelihood).
-__device__ __forceinline__ bool may_be_emitted(const ImParams& P, const uint16_t* keys, const uint32_t* hist, int K,
-                                               const uint32_t cnt[5], int ref_idx, int lane) {
+template <bool kHash>
+__device__ __forceinline__ bool may_be_emitted(const ImParams& P, const KeyCounts<kHash>& C, int K, const uint32_t cnt[5],
+                                               int ref_idx, int lane) {
   double n = 0.0;
 #pragma unroll
   for (int b = 0; b < 5; b++) n += (double)cnt[b];
@@ -150,7 +186,7 @@ __device__ __forceinline__ bool may_be_emitted(const ImParams& P, const uint16_t
 #pragma unroll
     for (int b = 0; b < 5; b++) f[b] /= total;
     for (int it = 0; it < 4; it++) {
-      if (!key_pass(P, keys, hist, K, lane, f, S, ll)) return true;
+      if (!key_pass(P, C, K, lane, f, S, ll)) return true;
       double g = 0.0;
 #pragma unroll
       for (int b = 0; b < 5; b++) {
@@ -175,7 +211,7 @@ __device__ __forceinline__ bool may_be_emitted(const ImParams& P, const uint16_t
     for (int b = 0; b < 5; b++) f[b] /= total;
     bool clear = false;
     for (int it = 0; it < 8; it++) {
-      if (!key_pass(P, keys, hist, K, lane, f, S, ll)) return true;
+      if (!key_pass(P, C, K, lane, f, S, ll)) return true;
       if (upper - ll < need) {
         clear = true;
         break;
@@ -200,19 +236,30 @@ __device__ __forceinline__ bool may_be_emitted(const ImParams& P, const uint16_t
 // nothing (19,743 of 20,011 columns passed it, of which some 30 are emitted) and the exact null fit of
 // each took the scorer 35.6 ms; this test takes 1.02 ms and leaves 36 (1 Mb at 300x with
 // 390 variants: 7,852 candidates, 0.17 ms, leaves 451).
-// LDS: a count per table key, and the list of the keys that occur.
-__global__ void __launch_bounds__(64 * kRouteWaves) k_route_candidates(ImParams P) {
-  extern __shared__ uint32_t route_lds[];   // per wavefront: tab_keys counts, then tab_keys 16-bit keys
-  const int lane = threadIdx.x & (WAVE - 1), wave = uniform_i((int)threadIdx.x / WAVE);
-  const int wv = blockIdx.x * kRouteWaves + wave, n_wv = gridDim.x * kRouteWaves;
-  uint32_t* route_hist = route_lds + (size_t)wave * route_words(P.tab_keys);
-  uint16_t* list = (uint16_t*)(route_hist + P.tab_keys);
+// LDS per wavefront: a count per table key and the list of those that occur; where the table has more than
+// kRouteKeys keys (from three MAPQs of paired reads on), a hash of the column's own keys (kHash), so that
+// the test does not depend on the table's size.  While such tables went without the test, all screened columns
+// went to the scorer (before -> now test and scorer, in ms; paired reads): 1 Mb at 300x, 3 MAPQs 1.6 -> 0.20 + 0.57,
+// 10 MAPQs 9.6 -> 0.24 + 0.65, 40 MAPQs 10.0 -> 0.28 + 0.69; 20 kb at 3,000x, 3 MAPQs 14.9 -> 1.35 + 0.66,
+// 40 MAPQs 34.1 -> 3.9 + 5.5.
+template <bool kHash>
+__global__ void __launch_bounds__(64 * kRouteWaves) k_route_candidates_t(ImParams P) {
+  extern __shared__ uint32_t route_lds[];
+  const int lane = threadIdx.x & (WAVE - 1), wave = uniform_i((int)threadIdx.x / WAVE), waves = (int)blockDim.x / WAVE;
+  const int wv = blockIdx.x * waves + wave, n_wv = gridDim.x * waves;
+  KeyCounts<kHash> C;
+  C.slots = kHash ? P.route_slots : P.tab_keys;
+  C.shift = kHash ? __clz(P.route_slots) + 1 : 0;
+  C.count = route_lds + (size_t)wave * route_words(kHash, C.slots);
+  C.keys = C.count + C.slots;
+  C.list = (uint16_t*)(kHash ? C.keys + C.slots : C.keys);
   uint32_t err = 0;
   const int n_ins = min(*P.n_ins, P.ins_cap);
   for (int i = wv; i < n_ins; i += n_wv) route_insert_slots(P, uniform_i(P.ins[i]), lane, err);
-  const bool test = P.tab_keys <= kRouteKeys;
-  if (test)
-    for (int i = lane; i < P.tab_keys; i += WAVE) route_hist[i] = 0;
+  for (int i = lane; i < C.slots; i += WAVE) {
+    C.count[i] = 0;
+    if (kHash) C.keys[i] = C.kNone;
+  }
   wave_lds_sync();
   const int n_cand = min(*P.n_cand, P.cand_cap);
   for (int ci = wv; ci < n_cand; ci += n_wv) {
@@ -224,7 +271,7 @@ __global__ void __launch_bounds__(64 * kRouteWaves) k_route_candidates(ImParams 
       continue;
     }
     bool keep = true;
-    if (uniform_i(cd.y) == kCandScreened && test) {
+    if (uniform_i(cd.y) == kCandScreened) {
       const int rb = uniform_i(P.win_rb[w]), re = uniform_i(P.win_re[w]);
       if (rb < 0 || re < rb || re > P.n_reads) {
         err |= kErrIndex;
@@ -232,7 +279,8 @@ __global__ void __launch_bounds__(64 * kRouteWaves) k_route_candidates(ImParams 
       }
       const uint32_t qspan = (uint32_t)max(0, P.quality_max - P.base_quality_cutoff);
       uint32_t cnt[5] = {0, 0, 0, 0, 0};
-      for (int r0 = rb; r0 < re; r0 += WAVE) {
+      bool full = false;
+      for (int r0 = rb; r0 < re && !full; r0 += WAVE) {
         const int r = r0 + lane;
         bool use = false;
         uint32_t key = 0;
@@ -263,24 +311,29 @@ __global__ void __launch_bounds__(64 * kRouteWaves) k_route_candidates(ImParams 
           }
         }
         use = use && key < (uint32_t)P.tab_keys;
-        if (use) atomicAdd(&route_hist[key], 1u);
+        const bool counted = C.add(use, key);
+        full = full || !counted;
 #pragma unroll
         for (int b = 0; b < 5; b++) cnt[b] += (uint32_t)__popcll(__ballot(use && obs == b));
         if (__all(past)) break;
       }
       wave_lds_sync();
       int K = 0;
-      for (int k0 = 0; k0 < P.tab_keys; k0 += WAVE) {
-        const bool on = k0 + lane < P.tab_keys && route_hist[k0 + lane] != 0;
+      for (int k0 = 0; k0 < C.slots; k0 += WAVE) {
+        const bool on = k0 + lane < C.slots && C.count[k0 + lane] != 0;
         const unsigned long long m = __ballot(on);
-        if (on) list[K + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)(k0 + lane);
+        if (on) C.list[K + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)(k0 + lane);
         K += __popcll(m);
       }
       wave_lds_sync();
       const int c = char_index(P.ref[p]);
-      keep = K > 0 && may_be_emitted(P, list, route_hist, K, cnt, c < 0 ? 5 : c, lane);
+      keep = full || (K > 0 && may_be_emitted(P, C, K, cnt, c < 0 ? 5 : c, lane));
       wave_lds_sync();
-      for (int k = lane; k < K; k += WAVE) route_hist[list[k]] = 0;
+      for (int k = lane; k < K; k += WAVE) {
+        const uint32_t slot = C.list[k];
+        C.count[slot] = 0;
+        if (kHash) C.keys[slot] = C.kNone;
+      }
       wave_lds_sync();
     }
     if (keep && lane == 0) {
@@ -418,5 +471,8 @@ __global__ void __launch_bounds__(256) k_runs(RunParams P) {
   for (uint64_t m = __ballot(mc_open); m; m &= m - 1) walk_mc_run(P, base + first_in(m), lane);
   for (uint64_t m = __ballot(un_open); m; m &= m - 1) walk_un_run(P, base + first_in(m), lane);
 }
+
+template __global__ void k_route_candidates_t<false>(ImParams P);
+template __global__ void k_route_candidates_t<true>(ImParams P);
 
 }  // namespace bsq

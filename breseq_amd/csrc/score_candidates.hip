@@ -28,6 +28,11 @@
 // tasks (0-2): the null fit, the profiles at the ML frequency, 0 and 1 and the bounds' midpoints, 24
 // tasks of eight lanes or 48 of four | KS and Fisher (3, first round).
 //
+// The distinct keys come from a hash of the column's own, so that they cost the same whatever the size of the
+// table; a column of more of them than LDS holds rows for reads the table, a row per read, in the same loops
+// (31 candidates of 3,000 reads and 40 MAPQs: 5.5 ms, where 45 ordered loops one after the other and
+// all candidates took 34 ms, and two ordered tasks per wavefront 26 ms).
+//
 // With 669 candidates of about 100 reads the kernel takes 0.26 ms (1.23 ms with two ordered EM tasks per
 // wavefront in LDS and three rounds of bisection); 28 candidates of 206 reads take 0.15 ms (1.40 ms),
 // 36 of 3,000 reads 0.39 ms.
@@ -49,6 +54,8 @@ static_assert(kSW == 4, "phase roles are laid out for four wavefronts");
 constexpr int kTaskWaves = 3;            // wavefronts of the EM tasks; the fourth has the statistics
 constexpr int kTaskSlots = 48;           // most tasks of a round: 4 lanes each, or 24 of 8 lanes
 constexpr int kKsDiag = 100;             // exact KS runs when m*n < 10000, so min(m, n) <= 99
+constexpr uint32_t kNoKey = 0xffffffffu;
+constexpr int kScoreProbes = 256;        // hash slots tried before a column counts as having too many distinct keys
 constexpr double kDrop = 0.587566;       // kProfileLikelihoodLog10Drop (identify_mutations.cpp:3173)
 // How far a result of sums in any order may be from the reference's, which adds n terms one after the
 // other: every addition rounds by up to 2^-53 of the sum so far, and where the terms are alike, as those
@@ -100,6 +107,7 @@ struct ScoreShared {
   int32_t exact;                   // bounds: 0 a round of tasks, 1 + side: an exact comparison is needed
   int32_t exact_have;              // exact_target is known
   int32_t bad_r;                   // a ratio outside the fast division's range
+  int32_t crowded;                 // a key found no slot in the hash
   int32_t unsure;                  // a result too close to a boundary: the candidate is done again exactly
   int32_t emitted;
   int32_t done;
@@ -158,12 +166,19 @@ __device__ __forceinline__ double recip_newton(double s) {
   return y;
 }
 
+template <bool kListGlobal>
+__device__ __forceinline__ uint32_t list_at(const uint32_t* list, int i) {
+  if constexpr (kListGlobal) return list[i];
+  else return ((const __attribute__((address_space(3))) uint32_t*)list)[i];
+}
+
 // The candidate's reads.  A read's likelihoods depend on its table key alone, so the rows
 // r[0..4] = 10^(lp_b - lpmax), r[5] = lpmax are kept once per distinct key, with the number of its
 // reads, and the reads' list holds each read's row.  Where the rows are is a compile-time choice
 // of the loops over them:
 //   kRowsLds     in LDS (they fit)
-//   kRowsGlobal  in the table in HBM: the list holds keys, and every read is a row of its own
+//   kRowsGlobal  in the table in HBM (more distinct keys than rows fit): the list holds keys, and every read is a
+//                row of its own
 enum { kRowsLds = 0, kRowsGlobal = 1 };
 
 struct Rows {
@@ -185,10 +200,10 @@ struct Rows {
     }
   }
   // row `i` of the distinct rows, and its reads
-  template <int kKind>
+  template <int kKind, bool kListGlobal>
   __device__ __forceinline__ uint32_t distinct(int i, double r[6]) const {
     if constexpr (kKind == kRowsGlobal) {
-      row<kKind>((int)list[i], r);
+      row<kKind>((int)list_at<kListGlobal>(list, i), r);
       return 1u;
     } else {
       row<kKind>(i, r);
@@ -208,12 +223,6 @@ __device__ __forceinline__ T* uniform_p(T* q) {
 }
 __device__ __forceinline__ Rows uniform_rows(const Rows& R) {
   return Rows{uniform_p(R.list), uniform_p(R.lds), uniform_p(R.reads), uniform_p(R.tab_r)};
-}
-
-template <bool kListGlobal>
-__device__ __forceinline__ uint32_t list_at(const uint32_t* list, int i) {
-  if constexpr (kListGlobal) return list[i];
-  else return ((const __attribute__((address_space(3))) uint32_t*)list)[i];
 }
 
 // One step of the two in-order chains: a += (lane K of this lane's row of ta), b likewise.
@@ -503,7 +512,7 @@ struct LogSum {
 // by one wavefront: 64 lanes share the distinct rows.  Leaves the frequencies in f and returns the
 // log10 likelihood without the sum of the reads' lpmax; NaN where the loop cannot stand for the
 // reference's (a read with s_i = 0, or a step within `stop` of tol).  fit[5]: the passes made.
-template <int kKind>
+template <int kKind, bool kListGlobal>
 __device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble* fit, double tol, double stop) {
   const Rows R = uniform_rows(Rv);
   const int K = uniform_i(Kv), lane = threadIdx.x & 63;
@@ -517,7 +526,7 @@ __device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble*
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     for (int i = lane; i < K; i += 64) {
       double r[6];
-      const uint32_t h = R.distinct<kKind>(i, r);
+      const uint32_t h = R.distinct<kKind, kListGlobal>(i, r);
       double s = f[0] * r[0];
 #pragma unroll
       for (int b = 1; b < 5; b++) s = fma(f[b], r[b], s);
@@ -539,7 +548,7 @@ __device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble*
   LogSum L;
   for (int i = lane; i < K; i += 64) {
     double r[6];
-    const uint32_t h = R.distinct<kKind>(i, r);
+    const uint32_t h = R.distinct<kKind, kListGlobal>(i, r);
     double s = fl[0] * r[0];
 #pragma unroll
     for (int b = 1; b < 5; b++) s = fma(fl[b], r[b], s);
@@ -555,17 +564,44 @@ __device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble*
   return __any(bad) ? __longlong_as_double(0x7ff8000000000000LL) : ll;
 }
 
+// The rows of em_tasks: get() returns row i's ratios, the variant's first and the other four alleles' in
+// order, and its reads.
+struct TaskRowsLds {      // six doubles a row, laid out so
+  const LdsDouble* prow;
+  __device__ __forceinline__ TaskRowsLds uniform() const { return *this; }
+  __device__ __forceinline__ double get(int i, double r[5]) const {
+    const LdsDouble* p = prow + i * 6;
+#pragma unroll
+    for (int b = 0; b < 5; b++) r[b] = p[b];
+    return p[5];
+  }
+};
+template <bool kListGlobal>
+struct TaskRowsGlobal {   // rows of the table, a read each: the variant comes first through the columns' addresses
+  const uint32_t* list;
+  const double* __restrict__ tab_r;
+  int variant;
+  __device__ __forceinline__ TaskRowsGlobal uniform() const { return {uniform_p(list), uniform_p(tab_r), uniform_i(variant)}; }
+  __device__ __forceinline__ double get(int i, double r[5]) const {
+    const uint32_t at = list_at<kListGlobal>(list, i) * 48u;
+    r[0] = *(const double*)((const char*)(tab_r + variant) + at);
+#pragma unroll
+    for (int b = 0; b < 4; b++) r[b + 1] = *(const double*)((const char*)(tab_r + b + (b >= variant ? 1 : 0)) + at);
+    return 1.0;
+  }
+};
+
 // The EM tasks of one wavefront, kSub lanes each: the null fit (the variant held out, from the counts
 // of the reads' observations) or profile_log10_likelihood (identify_mutations.cpp:3094-3143: the
 // variant pinned to x, the others from the full fit rescaled), the same iterations as em_exact's with
-// sums in any order over the candidate's distinct rows.  prow: per row the ratio of the variant, those
-// of the other four alleles in order, and the row's reads.  Returns log10 of the likelihood without
+// sums in any order over the candidate's K rows (Src: TaskRowsLds or TaskRowsGlobal).  Returns log10 of the likelihood without
 // the sum of the reads' lpmax, which every such value of a candidate shares; NaN where the value cannot
 // stand for the reference's (a read with s_i = 0, or a step within `stop` of tol).
 //   start[4]: the other alleles' starting frequencies; scale: 1 / n in the null fit, else 0
-template <int kSub>
-__device__ __noinline__ double em_tasks(const LdsDouble* prow, int Kv, double x, double start0, double start1, double start2,
+template <int kSub, class Src>
+__device__ __noinline__ double em_tasks(const Src Sv, int Kv, double x, double start0, double start1, double start2,
                                         double start3, double scale_null, bool active, double tol, double stop) {
+  const Src rows = Sv.uniform();
   const int K = uniform_i(Kv), sub = threadIdx.x & (kSub - 1);
   double f1 = start0, f2 = start1, f3 = start2, f4 = start3;
   const double rest = (1.0 - x) / 4.0;
@@ -582,10 +618,8 @@ __device__ __noinline__ double em_tasks(const LdsDouble* prow, int Kv, double x,
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const int i = i0 + u * kSub;
-        const LdsDouble* p = prow + min(i, K - 1) * 6;
-#pragma unroll
-        for (int b = 0; b < 5; b++) r[u][b] = p[b];
-        h[u] = (i < K) ? p[5] : 0.0;
+        h[u] = rows.get(min(i, K - 1), r[u]);
+        h[u] = (i < K) ? h[u] : 0.0;
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -648,10 +682,11 @@ __device__ __noinline__ double em_tasks(const LdsDouble* prow, int Kv, double x,
   }
   LogSum L;
   for (int i = sub; i < K; i += kSub) {
-    const LdsDouble* p = prow + i * 6;
+    double p[5];
+    const double reads = rows.get(i, p);
     const double s = fma(f4, p[4], fma(f3, p[3], fma(f2, p[2], fma(f1, p[1], x * p[0]))));
     bad = bad || !(s > 0x1p-100);
-    L.add(s, (uint32_t)p[5]);
+    L.add(s, (uint32_t)reads);
   }
   const double ll = sum_lanes<kSub>(L.value());
   // one lane that saw a read it cannot stand for spoils its task
@@ -669,8 +704,10 @@ __device__ __noinline__ double em_tasks(const LdsDouble* prow, int Kv, double x,
 // bracket's ends are joined by a line.  Once profile values are known at the interval's ends, the model
 // is corrected by the line through its errors there.  On 669 candidates of a 100x sample the path it
 // gives is right to the last of some 20 levels for 96% of the bounds.
-//   pre: per row d_i, t_i; prow: per row, its reads at [5]
+//   pre: per row d_i, t_i; prow: per row, its reads at [5] (null: one each)
+//   Kv: the rows, or as many of them as pre holds: fewer than all only predict less well
 //   known: the values vlo / vhi hold (else the target is m at the ML frequency, minus the drop)
+template <bool kOnes>
 __device__ __noinline__ double model_root(const LdsDouble* prow, const LdsDouble* pre, int Kv, double lo, double hi, bool known,
                                           double vlo, double vhi, double target) {
   const int K = uniform_i(Kv);
@@ -682,7 +719,7 @@ __device__ __noinline__ double model_root(const LdsDouble* prow, const LdsDouble
     double l2 = 0.0;
 #pragma unroll 4
     for (int i = 0; i < K; i++)
-      l2 = fma(prow[6 * i + 5], (double)__builtin_amdgcn_logf((float)fma(x, pre[2 * i], pre[2 * i + 1])), l2);
+      l2 = fma(kOnes ? 1.0 : prow[6 * i + 5], (double)__builtin_amdgcn_logf((float)fma(x, pre[2 * i], pre[2 * i + 1])), l2);
     const double m = l2 * 0.30102999566398119521;
     if (round == 0) {
       const double m_lo = __shfl(m, 32 * side, 64), m_hi = __shfl(m, 32 * side + 31, 64);
@@ -1019,15 +1056,15 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
     key_lds = ((size_t)P.key_cap * sizeof(uint32_t) + 15) & ~(size_t)15;
   }
   // P.rows_cap rows (six doubles each), the same with the variant first (em_tasks), their two model
-  // values, their keys and reads; before the rows are filled, a count and then a row number per table
-  // key lie in their place
+  // values, their keys and reads; before the rows are filled, the hash of the distinct keys lies in
+  // their place (a key and its first read, then its row, per slot); where they don't fit, the model values of the
+  // first pre_cap reads
   double* rows = (double*)(dyn + key_lds);
   double* prow = rows + (size_t)P.rows_cap * 6;
   double* pre = prow + (size_t)P.rows_cap * 6;
   uint32_t* key_of = (uint32_t*)(pre + (size_t)P.rows_cap * 2);
   uint32_t* row_reads = key_of + P.rows_cap;
-  uint32_t* row_of = (uint32_t*)rows;
-  const bool direct = (size_t)P.tab_keys * sizeof(uint32_t) <= (size_t)P.rows_cap * 96;
+  const int pre_cap = (int)((size_t)P.rows_cap * kScoreRowBytes / 16);
   constexpr bool kLG = kKeysGlobal;
   __shared__ ScoreShared SS;
   const int tid = threadIdx.x;
@@ -1113,45 +1150,73 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
     }
     const int n = __builtin_amdgcn_readfirstlane(min(SS.n_keys, P.key_cap));
     if (tid < 5) SS.obs[tid] = SS.cov[tid][0] + SS.cov[tid][2];
-    // ---- the distinct keys: counted per table key, numbered in key order by a block scan.  A
-    // table too large for that keeps a row per read.
+    // ---- the distinct keys, numbered in the order of their first reads, through a hash of the keys
     int K = n;
-    bool dedup = false;
-    if (direct) {
-      for (int i = tid; i < P.tab_keys; i += kSW * 64) row_of[i] = 0;
+    bool dedup = true;
+    {
+      // half full at most, unless the rows' LDS holds fewer slots
+      const int slots = min(1 << (32 - __clz(max(2 * n, 512) - 1)), 1 << (31 - __clz(P.rows_cap * 12)));
+      const int shift = __clz(slots) + 1;
+      uint32_t *hkey = (uint32_t*)rows, *hrow = hkey + slots;
+      for (int i = tid; i < slots; i += kSW * 64) hkey[i] = hrow[i] = kNoKey;
+      if (tid == 0) SS.crowded = 0;
       __syncthreads();
-      for (int i = tid; i < n; i += kSW * 64) atomicAdd(&row_of[list[i]], 1u);
-      __syncthreads();
-      const int per = (P.tab_keys + kSW * 64 - 1) / (kSW * 64);
-      const int k0 = min(tid * per, P.tab_keys), k1 = min(k0 + per, P.tab_keys);
-      int mine = 0;
-      for (int k = k0; k < k1; k++) mine += row_of[k] ? 1 : 0;
-      int incl = mine;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int u = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += u;
-      }
-      if (lane == 63) SS.wcount[wave] = (uint32_t)incl;
-      __syncthreads();
-      int at = incl - mine;
-      K = 0;
-      for (int k = 0; k < kSW; k++) {
-        if (k < wave) at += (int)SS.wcount[k];
-        K += (int)SS.wcount[k];
-      }
-      K = uniform_i(K);
-      dedup = K <= P.rows_cap;
-      if (dedup) {
-        for (int k = k0; k < k1; k++)
-          if (row_of[k]) {
-            key_of[at] = (uint32_t)k;
-            row_reads[at] = row_of[k];
-            row_of[k] = (uint32_t)at++;
+      // the slot of a key: its own, or the next free one (atomics only where a look does not settle it: most
+      // reads of a deep column share a few keys)
+      auto slot_of = [&](uint32_t key, bool insert) {
+        uint32_t at = (key * 0x9E3779B1u) >> shift;
+        for (int probe = 0; probe < kScoreProbes; probe++) {
+          uint32_t old = hkey[at];
+          if (insert && old == kNoKey) {
+            old = atomicCAS(&hkey[at], kNoKey, key);
+            if (old == kNoKey) return at;
           }
-        __syncthreads();
-        for (int i = tid; i < n; i += kSW * 64) list[i] = row_of[list[i]];
+          if (old == key) return at;
+          at = (at + 1u) & (uint32_t)(slots - 1);
+        }
+        return kNoKey;
+      };
+      for (int i = tid; i < n; i += kSW * 64) {
+        const uint32_t at = slot_of(list[i], true);
+        if (at == kNoKey) SS.crowded = 1;
+        else if (hrow[at] > (uint32_t)i) atomicMin(&hrow[at], (uint32_t)i);
       }
+      __syncthreads();
+      dedup = uniform_i(SS.crowded) == 0;
+      if (dedup) {
+        // a key's row: how many first reads come before its own.  (A slot whose row is already there holds
+        // less than any read still to be looked at.)
+        K = 0;
+        for (int i0 = 0; i0 < n; i0 += kSW * 64) {
+          const int i = i0 + tid;
+          const uint32_t at = (i < n) ? slot_of(list[i], false) : kNoKey;
+          const bool first = at != kNoKey && hrow[at] == (uint32_t)i;
+          const unsigned long long m = __ballot(first);
+          if (lane == 0) SS.wcount[wave] = (uint32_t)__popcll(m);
+          __syncthreads();
+          int row = K + __popcll(m & ((1ull << lane) - 1ull));
+          for (int k = 0; k < kSW; k++) {
+            if (k < wave) row += (int)SS.wcount[k];
+            K += (int)SS.wcount[k];
+          }
+          if (first) {
+            hrow[at] = (uint32_t)row;
+            if (row < P.rows_cap) {
+              key_of[row] = list[i];
+              row_reads[row] = 0;
+            }
+          }
+          __syncthreads();
+        }
+        K = uniform_i(K);
+        dedup = K <= P.rows_cap;
+      }
+      if (dedup)
+        for (int i = tid; i < n; i += kSW * 64) {
+          const uint32_t row = hrow[slot_of(list[i], false)];
+          list[i] = row;
+          atomicAdd(&row_reads[row], 1u);
+        }
     }
     const int kind = (dedup || n <= P.rows_cap) ? kRowsLds : kRowsGlobal;
     if (!dedup) {
@@ -1165,9 +1230,9 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
     }
     __syncthreads();
     bool bad_r = false;
-    const int n_check = (kind == kRowsLds) ? K * 6 : P.tab_keys * 6;
+    const int n_check = K * 6;   // (every read a row of its own where the rows are not in LDS)
     for (int i = tid; i < n_check; i += kSW * 64) {
-      const double r = P.tab_r[kind == kRowsLds ? (size_t)key_of[i / 6] * 6 + i % 6 : (size_t)i];
+      const double r = P.tab_r[(size_t)(kind == kRowsLds ? key_of[i / 6] : list[i / 6]) * 6 + i % 6];
       if (kind == kRowsLds) rows[i] = r;
       bad_r = bad_r || (i % 6 != 5 && r != 0.0 && !(r >= 0x1p-100 && r <= 2.0));
     }
@@ -1189,7 +1254,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
     const double stop = fmax(1e-6 * tol, 2.0 * kStopPasses * nu);
     // level 0: sums in any order; 1: the full fit and close comparisons with the reference's sums; 2: the
     // score's likelihoods too
-    int level = (P.screen_off || kind != kRowsLds) ? 2 : 0;
+    int level = P.screen_off ? 2 : 0;
     for (;;) {
       const bool in_order = level > 0;
       if (wave == 0) {
@@ -1209,7 +1274,8 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
           if (in_order) {
             ll = fit_exact(1, -1, 0.0);
           } else {
-            ll = em_full<kRowsLds>(RR, K, n, (LdsDouble*)SS.fit, tol, stop);
+            ll = kind == kRowsLds ? em_full<kRowsLds, kLG>(RR, K, n, (LdsDouble*)SS.fit, tol, stop)
+                                  : em_full<kRowsGlobal, kLG>(RR, K, n, (LdsDouble*)SS.fit, tol, stop);
             unsure = !(fabs(ll) < 1e300);
           }
         }
@@ -1266,6 +1332,18 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
           prow[6 * i + 5] = (double)row_reads[i];
           pre[2 * i] = rows[6 * i + variant] - t;
           pre[2 * i + 1] = t;
+        }
+      } else if (have_v) {
+        for (int i = tid; i < min(n, pre_cap); i += kSW * 64) {
+          double r[6], t = 0.0, rv = 0.0;
+          RR.row<kRowsGlobal>((int)list[i], r);
+#pragma unroll
+          for (int b = 0; b < 5; b++) {
+            if (b == variant) rv = r[b];
+            else t = fma((other > 0.0) ? SS.full_f[b] / other : 0.25, r[b], t);
+          }
+          rows[2 * i] = rv - t;
+          rows[2 * i + 1] = t;
         }
       }
       if (tid == 0) {
@@ -1324,7 +1402,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
             // annotate_polymorphism_statistics (identify_mutations.cpp:3009-3033); used if emitted
             if (round == 0 && n > 0 && !(in_order && SS.ks_p != 2.0))
               stats_w((LdsShared*)&SS, list, keys, row_reads, K, Q, major, minor);
-          } else if (have_v && search && kind == kRowsLds) {
+          } else if (have_v && search) {
             // task slots of the round.  Round 0: the profiles at the ML frequency, 0 and 1 and the null
             // fit, then the first path of each bound that may be searched.  Later: per open bound
             // the first levels of the full tree, whatever the prediction, then a path.  A bound needs
@@ -1340,7 +1418,10 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
             const double lo_l = (round == 0) ? (side_l ? fh : 0.0) : SS.lo[side_l];
             const double hi_l = (round == 0) ? (side_l ? 1.0 : fh) : SS.hi[side_l];
             const LdsDouble *pr = (const LdsDouble*)prow, *pm = (const LdsDouble*)pre;
-            const double root = model_root(pr, pm, K, lo_l, hi_l, round > 0, SS.vlo[side_l], SS.vhi[side_l], SS.target);
+            const double root =
+                kind == kRowsLds ? model_root<false>(pr, pm, K, lo_l, hi_l, round > 0, SS.vlo[side_l], SS.vhi[side_l], SS.target)
+                                 : model_root<true>(nullptr, (const LdsDouble*)rows, min(n, pre_cap), lo_l, hi_l, round > 0,
+                                                    SS.vlo[side_l], SS.vhi[side_l], SS.target);
             const double root0 = readlane_d(root, 0), root1 = readlane_d(root, 32);
             const int slot_i = (wave * 64 + lane) >> shift;
             const bool first = (lane & ((1 << shift) - 1)) == 0;
@@ -1395,8 +1476,13 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
                                   : (other > 0.0) ? (1.0 - x) * SS.full_f[at] / other : (1.0 - x) / 4.0;
               }
               const double sc = null_task ? 1.0 / (double)n : 0.0;
-              const double val = both ? em_tasks<4>(pr, K, x, st[0], st[1], st[2], st[3], sc, active, tol, stop)
-                                      : em_tasks<8>(pr, K, x, st[0], st[1], st[2], st[3], sc, active, tol, stop);
+              auto tasks_over = [&](auto src) {
+                typedef decltype(src) Src;
+                return both ? em_tasks<4, Src>(src, K, x, st[0], st[1], st[2], st[3], sc, active, tol, stop)
+                            : em_tasks<8, Src>(src, K, x, st[0], st[1], st[2], st[3], sc, active, tol, stop);
+              };
+              const double val = kind == kRowsLds ? tasks_over(TaskRowsLds{pr})
+                                                  : tasks_over(TaskRowsGlobal<kLG>{list, P.tab_r, variant});
               if (first && active) {
                 if (null_task) SS.null_ll = val;
                 else SS.val[slot_i] = val;
@@ -1410,7 +1496,6 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
           const int side = lane >> 5;
           const bool walker = (lane & 31) == 0;
           bool close = false;   // a comparison the tasks' values do not decide
-          const bool tasks = kind == kRowsLds;
           const double guard = P.screen_off ? INFINITY : SS.guard_log;
           Bound B;
           if (round == 0) {
@@ -1438,11 +1523,11 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
             // are within the guard of the target; the exact ones hold the lpmax sum.)
             B.step(side, SS.exact_v >= SS.exact_target, SS.exact_x[side], target, tol, fh);
           }
-          if (walker && (!exact || !tasks || P.screen_off) && B.active) {
-            const int depth = (exact || !tasks) ? 0 : SS.depth[side];
+          if (walker && (!exact || P.screen_off) && B.active) {
+            const int depth = exact ? 0 : SS.depth[side];
             if (B.active == 2) {
               const double v = side ? B.vhi : B.vlo;
-              close = !tasks || !(fabs(v - target) > guard);
+              close = !(fabs(v - target) > guard);
               if (!close) B.step(side, v >= target, 0.0, v, tol, fh);
             }
             // down the evaluated levels: every level is one sequential bisection step (the interval
@@ -1461,7 +1546,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
               B.step(side, ge, m, v, tol, fh);
               node = 2 * node + (((side == 0) ? ge : !ge) ? 1 : 2);
             }
-            if (B.active == 1 && (!tasks || P.screen_off)) close = true;   // every step exactly
+            if (B.active == 1 && P.screen_off) close = true;   // every step exactly
           }
           // neither end of the search may hang on the last bits of the ML frequency
           const double width = B.hi - B.lo;

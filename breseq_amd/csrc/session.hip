@@ -1329,6 +1329,13 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   P.n_score = S.d_counters.p + 6;
   P.score_next = S.d_counters.p + 5;
   P.n_level = S.d_counters.p + 7;
+  // slots for a column's distinct keys: no more than its window's reads, and far fewer than half of the table's
+  // keys (a quarter at the deepest: few qualities and observed bases are common)
+  P.route_slots = 0;
+  if (P.tab_keys > kRouteKeys) {
+    P.route_slots = 256;
+    while (P.route_slots < kRouteSlots && P.route_slots < std::min(S.max_window_reads, P.tab_keys / 2)) P.route_slots *= 2;
+  }
   P.guard_log = S.guard_log;
   P.guard_rel = S.guard_rel;
   P.cand_cap = cand_cap;
@@ -1342,10 +1349,15 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   // and its reads (8 B).
   const size_t key_list_bytes = ((size_t)P.key_cap * sizeof(uint32_t) + 15) & ~(size_t)15;
   P.keys_global = (key_list_bytes > kScoreKeyLds) ? 1 : 0;
-  // four blocks per CU while that leaves room for as many rows as a column has distinct keys at
-  // usual depths (some 60 at 100x, 200 at 3,000x); a longer read list takes more LDS per block
-  const size_t score_lds_budget = (key_list_bytes + 220 * kScoreRowBytes + kScoreStaticLds <= kScoreLdsBudget) ? kScoreLdsBudget
-                                                                                                            : kScoreLdsDeep;
+  // The LDS of a block: for as many rows as a column has distinct keys, some 60 at 100x and 200 at 3,000x
+  // with one MAPQ (of unique reads; redundant ones may add a second to the table), a quarter of the table's
+  // keys with more, and no more than it has reads.  Four blocks per CU where that holds them, else two, else one.  (20 kb
+  // at 3,000x with 3 MAPQs, 31 candidates of some 600 keys: 5.9 ms with rows read from the table, 0.66 ms with rows in LDS.)
+  const size_t rows_want = std::min<size_t>((size_t)P.key_cap, P.tab_keys <= kRouteKeys ? 220 : (size_t)P.tab_keys / 4);
+  const size_t score_lds_want = (P.keys_global ? 0 : key_list_bytes) + rows_want * kScoreRowBytes + kScoreStaticLds;
+  const size_t score_lds_budget = score_lds_want <= kScoreLdsBudget ? kScoreLdsBudget
+                                  : score_lds_want <= kScoreLdsDeep ? kScoreLdsDeep
+                                                                    : kScoreLdsMost;
   const size_t score_dyn_budget = score_lds_budget - kScoreStaticLds;
   const size_t key_bytes = P.keys_global ? 0 : key_list_bytes;
   if (P.keys_global) {
@@ -1410,8 +1422,15 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   std::copy(L.rr.begin(), L.rr.end(), S.h_tab_r.p);
   HIP_OK(hipMemcpyAsync(S.d_tab_r.p, S.h_tab_r.p, L.rr.size() * sizeof(double), hipMemcpyHostToDevice, S.stream));
   // the candidates and the scorer need no coverage cutoff: queued before the host waits for the fit
-  const size_t route_lds = (P.tab_keys <= kRouteKeys) ? kRouteWaves * sizeof(uint32_t) * route_words(P.tab_keys) : 0;
-  hipLaunchKernelGGL(k_route_candidates, dim3(kRouteGrid), dim3(64 * kRouteWaves), route_lds, S.stream, P);
+  if (P.route_slots == 0) {
+    hipLaunchKernelGGL(k_route_candidates_t<false>, dim3(kRouteGrid / kRouteWaves), dim3(64 * kRouteWaves),
+                       kRouteWaves * sizeof(uint32_t) * route_words(false, P.tab_keys), S.stream, P);
+  } else {
+    // as many wavefronts to a block as 40 KiB hold: four blocks per CU
+    const int waves = std::min(kRouteWaves, kRouteSlots / P.route_slots);
+    hipLaunchKernelGGL(k_route_candidates_t<true>, dim3(kRouteGrid / waves), dim3(64 * waves),
+                       waves * sizeof(uint32_t) * route_words(true, P.route_slots), S.stream, P);
+  }
   HIP_OK(hipGetLastError());
   HIP_OK(hipEventRecord(S.evk[1], S.stream));
   if (P.keys_global)
