@@ -284,7 +284,7 @@ class Session:
         L.check(L.lib().bsq_session_set_gd_capacity(self._h, int(entries), C.byref(st)), st)
         return self
 
-    def set_scorer_guards(self, log10_likelihood=1e-8, frequency=1e-12):
+    def set_scorer_guards(self, log10_likelihood=1e-8, frequency=2e-12):
         """Raise the least distance from a decision's boundary below which the exact scorer does a candidate
         again with sums in read order (diagnostic: results do not change)."""
         st = _status()

@@ -237,7 +237,7 @@ __global__ void k_coverage_columns(CovTabParams C);
 // Downsampled rows (step > 1): one wavefront per row, lanes over the row's reads.
 __global__ void k_coverage_rows(CovTabParams C);
 
-constexpr double kGuardLog = 1e-8, kGuardRel = 1e-12;   // ImParams::guard_log, guard_rel unless set
+constexpr double kGuardLog = 1e-8, kGuardRel = 2e-12;   // ImParams::guard_log, guard_rel unless set
 constexpr int kScoreWaves = 4;               // wavefronts per candidate in the exact scorer
 // blocks of the exact scorer (each draws candidates from a work counter): four per CU are resident
 constexpr int kScoreGrid = 1024;

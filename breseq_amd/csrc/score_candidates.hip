@@ -984,7 +984,7 @@ __device__ __noinline__ bool prints_surely_e(double v, int places, double rel) {
   if (!(v > 1e-280) || places > 12) return false;
   const double e = floor(log10(v));
   const double scaled = v * pow(10.0, (double)places - e);
-  return fabs(scaled - floor(scaled) - 0.5) > 2.0 * rel * scaled;
+  return fabs(scaled - floor(scaled) - 0.5) > rel * scaled;
 }
 
 // The same of a score known within `err`, printed with one decimal.
@@ -999,9 +999,9 @@ __device__ __noinline__ bool fit_is_sure(const LdsDouble* f, uint32_t n, int pla
   const double thr = 0.5 / (double)n;
   for (int a = 0; a < 5; a++) {
     if (f[a] < fmin(0.5 * thr, 0.01)) continue;
-    if (fabs(f[a] - thr) <= 4.0 * rel * thr) return false;
+    if (fabs(f[a] - thr) <= 2.0 * rel * thr) return false;
     for (int b = 0; b < a; b++)
-      if (fabs(f[a] - f[b]) <= 4.0 * rel * f[a]) return false;
+      if (fabs(f[a] - f[b]) <= 2.0 * rel * f[a]) return false;
     if (f[a] >= thr && !prints_surely_e(f[a], places, rel)) return false;
   }
   return true;

@@ -419,7 +419,7 @@ int bsq_session_timing(const bsq_session* s, bsq_timing* out);
 /* Diagnostics of the exact scorer (no counterpart in breseq, which sums in read order throughout).  The
  * scorer first sums in any order and does a candidate again in read order where a decision or a printed
  * digit lies within a guard of its boundary.  set_scorer_guards raises the least guards of later passes
- * (defaults 1e-8 of a log10 likelihood, 1e-12 of a frequency; never below them): more candidates
+ * (defaults 1e-8 of a log10 likelihood, 2e-12 of a frequency; never below them): more candidates
  * are done again, results do not change.  scorer_levels: the candidates of the last identify pass decided
  * by sums in any order, by a full fit and close comparisons in read order, and wholly in read order. */
 int bsq_session_set_scorer_guards(bsq_session* s, double log10_likelihood, double frequency, bsq_status* status);

@@ -36,16 +36,16 @@ def test_every_level(depth, n_mapq):
     try:
         want = gd_text(sess, args, True)
         seen = [0, 0, 0]
-        for guards in [(1e-8, 1e-12), (1e-2, 1e-12), (0.3, 1e-12), (1e-8, 1e-4), (1e-2, 1e-4), (1e9, 1e-12)]:
+        for guards in [(1e-8, 2e-12), (1e-2, 2e-12), (0.3, 2e-12), (1e-8, 1e-4), (1e-2, 1e-4), (1e9, 2e-12)]:
             sess.set_scorer_guards(*guards)
             assert gd_text(sess, args, False) == want, guards
             levels = sess.scorer_levels()
             print("[gpu]   guards", guards, "levels", levels, flush=True)
             assert sum(levels) == sess.timing()["candidates"]
             seen = [a + b for a, b in zip(seen, levels)]
-            if guards == (1e-8, 1e-12):
+            if guards == (1e-8, 2e-12):
                 assert levels[0] > 0
-            if guards == (1e9, 1e-12):
+            if guards == (1e9, 2e-12):
                 assert levels[2] >= want.count("RA\t")
         assert min(seen) > 0
     finally:

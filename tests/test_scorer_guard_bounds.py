@@ -1,7 +1,7 @@
 """How far EM frequencies and log10 likelihoods summed in read order lie from correctly rounded sums, against
 the bounds that the exact scorer's guards are made of: passes * (n + 64) * 2^-53 of a frequency and
 4 (n + 64) 2^-53 (n + |log10 likelihood|).  At 200,000 reads of one quality the differences pass the guards' least values
-(1e-12 and 1e-8), which alone would not do there."""
+(2e-12 and 1e-8), which alone would not do there."""
 import math
 
 import numpy as np
@@ -42,6 +42,6 @@ def test_sums_in_read_order(n):
             assert abs(ll - ll0) <= 4.0 * (n + 64) * U * (n + abs(ll0))
             most_f, most_ll = max(most_f, rel), max(most_ll, abs(ll - ll0))
     if n == 200000:
-        assert most_f > 1e-12 and most_ll > 1e-8
+        assert most_f > 2e-12 and most_ll > 1e-8
     elif n <= 3000:
-        assert most_f < 1e-12 and most_ll < 1e-8
+        assert most_f < 2e-12 and most_ll < 1e-8
