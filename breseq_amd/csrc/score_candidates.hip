@@ -570,7 +570,8 @@ struct TaskRowsLds {      // six doubles a row, laid out so
   const LdsDouble* prow;
   __device__ __forceinline__ TaskRowsLds uniform() const { return *this; }
   __device__ __forceinline__ double get(int i, double r[5]) const {
-    const LdsDouble* p = prow + i * 6;
+    typedef __attribute__((address_space(3))) const char LdsChar;
+    const LdsDouble* p = (const LdsDouble*)((LdsChar*)prow + __umul24((uint32_t)i, 48u));
 #pragma unroll
     for (int b = 0; b < 5; b++) r[b] = p[b];
     return p[5];
@@ -617,9 +618,7 @@ __device__ __noinline__ double em_tasks(const Src Sv, int Kv, double x, double s
       double r[4][5], h[4], s[4], y[4];
 #pragma unroll
       for (int u = 0; u < 4; u++) {
-        const int i = i0 + u * kSub;
-        h[u] = rows.get(min(i, K - 1), r[u]);
-        h[u] = (i < K) ? h[u] : 0.0;
+        h[u] = rows.get(min(i0 + u * kSub, K - 1), r[u]);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -650,7 +649,7 @@ __device__ __noinline__ double em_tasks(const Src Sv, int Kv, double x, double s
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int u = 0; u < 4; u++) y[u] *= h[u];
+      for (int u = 0; u < 4; u++) y[u] *= (i0 + u * kSub < K) ? h[u] : 0.0;   // here: the loads' last values
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int u = 0; u < 4; u++) {
@@ -1158,6 +1157,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
       const int slots = min(1 << (32 - __clz(max(2 * n, 512) - 1)), 1 << (31 - __clz(P.rows_cap * 12)));
       const int shift = __clz(slots) + 1;
       uint32_t *hkey = (uint32_t*)rows, *hrow = hkey + slots;
+#pragma unroll 1
       for (int i = tid; i < slots; i += kSW * 64) hkey[i] = hrow[i] = kNoKey;
       if (tid == 0) SS.crowded = 0;
       __syncthreads();
@@ -1165,6 +1165,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
       // reads of a deep column share a few keys)
       auto slot_of = [&](uint32_t key, bool insert) {
         uint32_t at = (key * 0x9E3779B1u) >> shift;
+#pragma unroll 1
         for (int probe = 0; probe < kScoreProbes; probe++) {
           uint32_t old = hkey[at];
           if (insert && old == kNoKey) {
@@ -1176,6 +1177,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
         }
         return kNoKey;
       };
+#pragma unroll 1
       for (int i = tid; i < n; i += kSW * 64) {
         const uint32_t at = slot_of(list[i], true);
         if (at == kNoKey) SS.crowded = 1;
@@ -1187,6 +1189,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
         // a key's row: how many first reads come before its own.  (A slot whose row is already there holds
         // less than any read still to be looked at.)
         K = 0;
+#pragma unroll 1
         for (int i0 = 0; i0 < n; i0 += kSW * 64) {
           const int i = i0 + tid;
           const uint32_t at = (i < n) ? slot_of(list[i], false) : kNoKey;
@@ -1212,6 +1215,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
         dedup = K <= P.rows_cap;
       }
       if (dedup)
+#pragma unroll 1
         for (int i = tid; i < n; i += kSW * 64) {
           const uint32_t row = hrow[slot_of(list[i], false)];
           list[i] = row;
@@ -1231,6 +1235,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
     __syncthreads();
     bool bad_r = false;
     const int n_check = K * 6;   // (every read a row of its own where the rows are not in LDS)
+#pragma unroll 1
     for (int i = tid; i < n_check; i += kSW * 64) {
       const double r = P.tab_r[(size_t)(kind == kRowsLds ? key_of[i / 6] : list[i / 6]) * 6 + i % 6];
       if (kind == kRowsLds) rows[i] = r;
