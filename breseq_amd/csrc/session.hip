@@ -1043,11 +1043,20 @@ struct GdQueued {
 };
 
 // Whether the wavefronts of a block share each window's alignments.  With fewer windows than wavefronts
-// that the device holds (two blocks of eight per CU), a wavefront per window leaves the device idle, and
-// sharing took the column pass of 48 kb at 206x from 401 to 117 us and of 20 kb at 3,000x from 2182 to
-// 220 us; with more windows the batches of a shared window are too short and its sums are added up
-// twice: 701 kb (10,960 windows) took 576 us shared and 187 us not, 4.6 Mb 4345 and 1042 us.
-static bool column_split(const Session& S) { return S.n_windows < kColResident; }
+// that the device holds (two blocks of eight per CU), a wavefront per window leaves the device idle and takes as long as
+// one window's alignments do; a shared window costs adding up its sums, so it has to hold some
+// work: as many aligned bases as there are windows.  Column pass in us, a wavefront per window / shared:
+//   reads     windows: 313       750        1,250     1,720      2,190      2,810      3,440      4,060
+//   100 b, 20x         74 / 36   56 / 45    64 / 51   60 / 72*   54 / 74*   67 / 92*   82 / 108*  63 / 123*
+//   36 b, 40x          86 / 49   72 / 61    75 / 72   84 / 90    101 / 97   79 / 103*  89 / 120*  102 / 147*
+//   150 b, 60x         172 / 58  135 / 66   153 / 73  167 / 101  157 / 87   165 / 104  166 / 122  145 / 147*
+//   36 b, 83x          170 / 79  127 / 84   136 / 100 155 / 134  173 / 123  151 / 123  161 / 147  177 / 193
+//   150 b, 100x        248 / 76  209 / 85   230 / 93  269 / 125  263 / 106  238 / 119  251 / 136  237 / 177
+// (*: fewer aligned bases in a window than windows; not shared.)  Far above, 701 kb of 300-base reads (10,960
+// windows) took 576 us shared and 187 us not, 4.6 Mb 4345 and 1042 us.
+static bool column_split(const Session& S) {
+  return S.n_windows < kColResident && S.n_windows < S.aligned_bases / std::max<int64_t>(1, S.n_windows);
+}
 
 // Blocks of the column pass.  A set count is kept to at most one window per wavefront and rounded
 // down to a multiple of the 8 XCDs from 8 blocks up (the windows of one block then sit on one XCD's
