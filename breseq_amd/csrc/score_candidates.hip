@@ -65,15 +65,14 @@ constexpr double kDrop = 0.587566;       // kProfileLikelihoodLog10Drop (identif
 //     the reads): passes * n * 2^-53, relative.
 //   * A log10 likelihood is off by up to n 2^-53 of its size, and by up to n^2 2^-53 because the
 //     frequencies add up to 1 only within n 2^-53; a score has two of them.  Guarded with twice that.
-//   * A loop ends when no frequency moved by tol: a step this close to it, after up to 100 passes (a
-//     profile's start from the full fit's), is not decided here.
+//   * A loop ends when no frequency moved by tol.  A step may be off by n 2^-53 for every pass up to it, and
+//     for those of the full fit that a profile starts from; one closer to tol is not decided here.
 // Measured against correctly rounded sums, most of three mixes of qualities: 5e-14 of a frequency and 7e-11 of
 // a likelihood at 3,000 reads (bounds 1e-12 and 5e-9), 3e-12 and 3e-7 at 200,000 (7e-11 and 2e-5).
 // A decision or a printed digit closer to its boundary than its guard is made on exact sums.  Up to
 // some thousand reads the least guards of a launch hold (ImParams::guard_log, guard_rel).
 constexpr double kHalfUlp = 0x1p-53;
 constexpr double kSumSlack = 64.0;       // additions besides those of the reads: a term's own operations
-constexpr double kStopPasses = 100.0;
 
 struct ScoreShared {
   double full_f[5];
@@ -511,9 +510,10 @@ struct LogSum {
 // fit_allele_frequencies (identify_mutations.cpp:3240-3318) over all alleles with sums in any order,
 // by one wavefront: 64 lanes share the distinct rows.  Leaves the frequencies in f and returns the
 // log10 likelihood without the sum of the reads' lpmax; NaN where the loop cannot stand for the
-// reference's (a read with s_i = 0, or a step within `stop` of tol).  fit[5]: the passes made.
+// reference's (a read with s_i = 0, or a step too close to tol).  nu: (n + kSumSlack) 2^-53; fit[5]: the passes
+// made.
 template <int kKind, bool kListGlobal>
-__device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble* fit, double tol, double stop) {
+__device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble* fit, double tol, double nu) {
   const Rows R = uniform_rows(Rv);
   const int K = uniform_i(Kv), lane = threadIdx.x & 63;
   const double per_n = 1.0 / (double)uniform_i(nv);
@@ -542,7 +542,7 @@ __device__ __noinline__ double em_full(const Rows Rv, int Kv, int nv, LdsDouble*
       sum += f[b];
       most = fmax(most, fabs(f[b] - fl[b]));
     }
-    bad = bad || !(sum > 0.5 && sum < 2.0) || (it < 50 && fabs(most - tol) < stop);
+    bad = bad || !(sum > 0.5 && sum < 2.0) || (it < 50 && fabs(most - tol) < fmax(1e-6 * tol, (double)(it + 1) * nu));
     if (!(most >= tol) || it >= 50) break;
   }
   LogSum L;
@@ -597,11 +597,12 @@ struct TaskRowsGlobal {   // rows of the table, a read each: the variant comes f
 // variant pinned to x, the others from the full fit rescaled), the same iterations as em_exact's with
 // sums in any order over the candidate's K rows (Src: TaskRowsLds or TaskRowsGlobal).  Returns log10 of the likelihood without
 // the sum of the reads' lpmax, which every such value of a candidate shares; NaN where the value cannot
-// stand for the reference's (a read with s_i = 0, or a step within `stop` of tol).
+// stand for the reference's (a read with s_i = 0, or a step too close to tol).
+//   nu: (n + kSumSlack) 2^-53; passes: those before the start, and one
 //   start[4]: the other alleles' starting frequencies; scale: 1 / n in the null fit, else 0
 template <int kSub, class Src>
 __device__ __noinline__ double em_tasks(const Src Sv, int Kv, double x, double start0, double start1, double start2,
-                                        double start3, double scale_null, bool active, double tol, double stop) {
+                                        double start3, double scale_null, bool active, double tol, double nu, double passes) {
   const Src rows = Sv.uniform();
   const int K = uniform_i(Kv), sub = threadIdx.x & (kSub - 1);
   double f1 = start0, f2 = start1, f3 = start2, f4 = start3;
@@ -671,7 +672,7 @@ __device__ __noinline__ double em_tasks(const Src Sv, int Kv, double x, double s
     const double g3 = some ? scale * a3 : rest, g4 = some ? scale * a4 : rest;
     const double most = fmax(fmax(fabs(g1 - f1), fabs(g2 - f2)), fmax(fabs(g3 - f3), fabs(g4 - f4)));
     // (not-a-number sums fail the first test)
-    bad |= run & (!(others >= 0.0) | ((others > 0.0) & (others < 0x1p-500)) | ((it < 50) & (fabs(most - tol) < stop)));
+    bad |= run & (!(others >= 0.0) | ((others > 0.0) & (others < 0x1p-500)) | ((it < 50) & (fabs(most - tol) < fmax(1e-6 * tol, ((double)it + passes) * nu))));
     run &= (most >= tol) & (it < 50);
     // a task that ends keeps this pass's frequencies: the likelihood is theirs
     f1 = run ? g1 : f1;
@@ -1256,7 +1257,6 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
     int major = 5, minor = 5, variant = 5;
     bool have_v = false;
     const double nu = ((double)n + kSumSlack) * kHalfUlp;
-    const double stop = fmax(1e-6 * tol, 2.0 * kStopPasses * nu);
     // level 0: sums in any order; 1: the full fit and close comparisons with the reference's sums; 2: the
     // score's likelihoods too
     int level = P.screen_off ? 2 : 0;
@@ -1279,8 +1279,8 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
           if (in_order) {
             ll = fit_exact(1, -1, 0.0);
           } else {
-            ll = kind == kRowsLds ? em_full<kRowsLds, kLG>(RR, K, n, (LdsDouble*)SS.fit, tol, stop)
-                                  : em_full<kRowsGlobal, kLG>(RR, K, n, (LdsDouble*)SS.fit, tol, stop);
+            ll = kind == kRowsLds ? em_full<kRowsLds, kLG>(RR, K, n, (LdsDouble*)SS.fit, tol, nu)
+                                  : em_full<kRowsGlobal, kLG>(RR, K, n, (LdsDouble*)SS.fit, tol, nu);
             unsure = !(fabs(ll) < 1e300);
           }
         }
@@ -1481,10 +1481,11 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
                                   : (other > 0.0) ? (1.0 - x) * SS.full_f[at] / other : (1.0 - x) / 4.0;
               }
               const double sc = null_task ? 1.0 / (double)n : 0.0;
+              const double passes = (level == 0 ? SS.fit[5] : 0.0) + 1.0;
               auto tasks_over = [&](auto src) {
                 typedef decltype(src) Src;
-                return both ? em_tasks<4, Src>(src, K, x, st[0], st[1], st[2], st[3], sc, active, tol, stop)
-                            : em_tasks<8, Src>(src, K, x, st[0], st[1], st[2], st[3], sc, active, tol, stop);
+                return both ? em_tasks<4, Src>(src, K, x, st[0], st[1], st[2], st[3], sc, active, tol, nu, passes)
+                            : em_tasks<8, Src>(src, K, x, st[0], st[1], st[2], st[3], sc, active, tol, nu, passes);
               };
               const double val = kind == kRowsLds ? tasks_over(TaskRowsLds{pr})
                                                   : tasks_over(TaskRowsGlobal<kLG>{list, P.tab_r, variant});
