@@ -275,9 +275,10 @@ __device__ __forceinline__ void ec_run_indel(const EcParams& P, const uint8_t* s
   }
 }
 
-// What bounds it: 4.6 Mb at 100x of 150-base reads reads 0.95 GB at 2.7 TB/s (360 us), with the vector
-// unit about 60% busy (17 instructions a position, 125 M in all) and the LDS 30% (one atomic a
-// position).  One alignment of up to 168 bases to 21 lanes, position-wise selects and an atomic each
+// What bounds it: 4.6 Mb at 100x of 150-base reads needs 1.0 GB and moves 1.8 GB in 360 us, 5.1 TB/s, the
+// rate of a large copy (a run's ends are read a second time, by ec_run_pairs, when their lines have left the
+// L2), with the vector unit about 60% busy (17 instructions a position, 125 M in all) and the LDS 30%
+// (one atomic a position).  One alignment of up to 168 bases to 21 lanes, position-wise selects and an atomic each
 // for the base and its pair took 409 M instructions and 871 us; alignments with an indel went one at a
 // time, and a wavefront whose alignments all cross one took 165 us alone.  Measured before -> now, in
 // us: 2.05 Mb at 83x of 36 bases (five of 21 lanes had work) 1166 -> 226, 48 kb at 206x of 100 bases
