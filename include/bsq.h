@@ -252,7 +252,7 @@ int bsq_sequence_trims(const char* seq, int64_t len, uint8_t* out, bsq_status* s
 /* No counterpart in breseq.  bsq_sequence_trims without any device allocation, for callers that
  * cannot allocate (code under HIP graph capture, serving loops, harnesses that forbid hipMalloc):
  * the sequence, its repeat extents and the trims are staged in a static device array of the
- * library (32 MiB, held on each GPU it runs on until the process ends).  len <= 8388608 bases,
+ * library (24 MiB, held on each GPU it runs on until the process ends).  len <= 8388608 bases,
  * else BSQ_ERR_LIMIT.  Calls that overlap on one GPU share that array and race. */
 int bsq_sequence_trims_static(const char* seq, int64_t len, uint8_t* out, bsq_status* status);
 
