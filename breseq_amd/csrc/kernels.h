@@ -181,6 +181,8 @@ __global__ void k_ec_reads(EcParams P);
 __global__ void k_cov_tile_sums(CovParams C);
 __global__ void k_cov_tile_scan(CovParams C);
 __global__ void k_cov_hist(CovParams C);
+constexpr int kCus = 256;                    // compute units of the device, and their LDS
+constexpr size_t kCuLds = 160 * 1024;
 constexpr int kColResident = 4096;           // wavefronts of the column kernel that the device holds
 constexpr int kColWaves = 8;                 // wavefronts per block of the column kernel (default; 4 also built)
 constexpr size_t kFoldLdsBytes = 48 * 1024;  // largest likelihood table staged in LDS

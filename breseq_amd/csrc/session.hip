@@ -108,6 +108,7 @@ struct Session {
   int32_t max_window_reads = 0;
   int64_t n_dreads = 0;
   int64_t aligned_bases = 0;
+  double col_serial_us = 0.0;   // column_split: the most that a window's alignments take one wavefront, about
   std::vector<int32_t> mapq_values;   // mslot -> MAPQ
   int32_t n_read_files = 1;
   std::vector<int32_t> h_pos_target;
@@ -578,19 +579,28 @@ static void session_load(Session& S, const bsq_reference* ref, const bsq_alignme
   S.n_input_reads = a->n_reads;
   S.h_gpos.resize((size_t)n_pack);
   S.h_gend_max.resize((size_t)n_pack);
+  S.n_windows = ((int64_t)S.n_pos + kWave - 1) / kWave;
+  // alignments per window that the column pass takes one at a time, for column_split: their first and last
+  // windows here, added up with the window index
+  std::vector<int32_t> single(S.n_windows < kColResident ? (size_t)S.n_windows + 1 : 0);
   for (size_t i = 0; i < (size_t)n_pack; i++) {
-    S.h_gpos[i] = dr[i].gpos;
-    S.h_gend_max[i] = std::max(dr[i].gend, i ? S.h_gend_max[i - 1] : (int32_t)-1);
+    const DRead& d = dr[i];
+    S.h_gpos[i] = d.gpos;
+    S.h_gend_max[i] = std::max(d.gend, i ? S.h_gend_max[i - 1] : (int32_t)-1);
+    if (!single.empty() && (!(d.flags & kReadSimple) || d.x1 != 1) && d.gend > d.gpos) {
+      single[(size_t)(d.gpos / kWave)]++;
+      single[(size_t)((d.gend - 1) / kWave) + 1]--;
+    }
   }
   dp_select(a, ref->n_targets, S.dp_reads);
   if (S.n_dreads >= ((int64_t)1 << 31)) throw BsqError(BSQ_ERR_LIMIT, "more than 2^31 alignments");
   S.aligned_bases = nab;
   // window index: alignments overlapping [64w, 64w+64)
-  S.n_windows = ((int64_t)S.n_pos + kWave - 1) / kWave;
   std::vector<int32_t> rb(S.n_windows), re(S.n_windows);
   {
     size_t lo = 0, hi = 0;
     int32_t mx = 0;
+    S.col_serial_us = 0.0;
     for (int64_t w = 0; w < S.n_windows; w++) {
       const int64_t w0 = w * kWave, w1 = w0 + kWave;
       while (lo < (size_t)n_pack && (int64_t)dr[lo].gpos < w0 - maxspan) lo++;
@@ -598,6 +608,10 @@ static void session_load(Session& S, const bsq_reference* ref, const bsq_alignme
       rb[w] = (int32_t)lo;
       re[w] = (int32_t)hi;
       mx = std::max<int32_t>(mx, (int32_t)(hi - lo));
+      if (!single.empty()) {
+        if (w > 0) single[(size_t)w] += single[(size_t)w - 1];
+        S.col_serial_us = std::max(S.col_serial_us, 0.35 * (double)(hi - lo) + 1.7 * single[(size_t)w]);
+      }
     }
     S.max_window_reads = mx;
   }
@@ -1043,19 +1057,24 @@ struct GdQueued {
 };
 
 // Whether the wavefronts of a block share each window's alignments.  With fewer windows than wavefronts
-// that the device holds (two blocks of eight per CU), a wavefront per window leaves the device idle and takes as long as
-// one window's alignments do; a shared window costs adding up its sums, so it has to hold some
-// work: as many aligned bases as there are windows.  Column pass in us, a wavefront per window / shared:
-//   reads     windows: 313       750        1,250     1,720      2,190      2,810      3,440      4,060
-//   100 b, 20x         74 / 36   56 / 45    64 / 51   60 / 72*   54 / 74*   67 / 92*   82 / 108*  63 / 123*
-//   36 b, 40x          86 / 49   72 / 61    75 / 72   84 / 90    101 / 97   79 / 103*  89 / 120*  102 / 147*
-//   150 b, 60x         172 / 58  135 / 66   153 / 73  167 / 101  157 / 87   165 / 104  166 / 122  145 / 147*
-//   36 b, 83x          170 / 79  127 / 84   136 / 100 155 / 134  173 / 123  151 / 123  161 / 147  177 / 193
-//   150 b, 100x        248 / 76  209 / 85   230 / 93  269 / 125  263 / 106  238 / 119  251 / 136  237 / 177
-// (*: fewer aligned bases in a window than windows; not shared.)  Far above, 701 kb of 300-base reads (10,960
-// windows) took 576 us shared and 187 us not, 4.6 Mb 4345 and 1042 us.
+// that the device holds (two blocks of eight per CU), a wavefront per window leaves the device idle, and the
+// pass takes as long as the window with the most work: some 0.35 us an alignment, eight at a time, and 1.7 us for one
+// that goes by itself (S.col_serial_us).  Shared, the wavefronts do an eighth of that each, but a block spends some
+// 18 us on a window however little there is in it (the table, the sums of its wavefronts), 512 blocks at a time.
+// Column pass in us, a wavefront per window / shared (* as chosen), and before windows were shared; poly: few alignments with
+// an indel, cons: whole columns of them:
+//   20 kb, 3,000x poly, 150 b    2843 / 452*   3828        100 kb, 60x cons, 150 b     142 / 78*    148
+//   48 kb, 206x cons, 100 b      457 / 149*    510         100 kb, 150x poly, 150 b    90 / 77*     119
+//   48 kb, 20x cons, 36 b        52 / 50*      55          150 kb, 20x cons, 100 b     65* / 88     62
+//   48 kb, 60x poly, 150 b       69 / 51*      75          150 kb, 300x poly, 150 b    346 / 147*   459
+//   100 kb, 60x poly, 150 b      40* / 65      50          200 kb, 60x poly, 150 b     64* / 109    69
+//   200 kb, 60x cons, 150 b      164 / 141*    165         250 kb, 300x poly, 150 b    223 / 207*   322
+//   100 kb, 40x poly, 36 b       37* / 64      57          200 kb, 83x poly, 36 b      94* / 126    147
+//   100 kb, 40x cons, 36 b       89 / 76*      104         250 kb, 100x poly, 150 b    83* / 144    107
+//   200 kb, 83x cons, 36 b       188 / 190*    236         250 kb, 100x cons, 150 b    259 / 192*   281
+// Far above, 701 kb of 300-base reads (10,960 windows) took 576 us shared and 187 us not, 4.6 Mb 4345 and 1042 us.
 static bool column_split(const Session& S) {
-  return S.n_windows < kColResident && S.n_windows < S.aligned_bases / std::max<int64_t>(1, S.n_windows);
+  return S.n_windows < kColResident && 18.0 * (double)S.n_windows / 512.0 + S.col_serial_us / 8.0 < S.col_serial_us;
 }
 
 // Blocks of the column pass.  A set count is kept to at most one window per wavefront and rounded
@@ -1322,6 +1341,11 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
   P.fold_rows = (int32_t)fold.size();
   const size_t fold_bytes = fold.size() / 5 * kFoldLdsRow;
   P.fold_lds = (fold_bytes <= kFoldLdsBytes && S.col_lds) ? 1 : 0;
+  // A block per window stages the table once a window: only while two blocks still fit on a CU, or there are no more
+  // than two windows to a CU.  (Three MAPQs of pairs, 39 KB: 20 kb at 3,000x 461 us staged, 527 us not; 48 kb at
+  // 60x 81 and 72 us; 250 kb at 100x 282 and 223 us.)
+  P.col_split = column_split(S) ? 1 : 0;
+  if (P.col_split && S.n_windows > 2 * kCus && 2 * (column_lds(S.col_waves, true) + fold_bytes) > kCuLds) P.fold_lds = 0;
   P.log10_ref_length = log10(total_len);
   P.mutation_cutoff = a->mutation_cutoff;
   P.polymorphism_cutoff = a->polymorphism_cutoff;
@@ -1407,7 +1431,6 @@ static bool run_identify_once(Session& S, const bsq_identify_args* a, bsq_im_res
     const int64_t g = column_blocks(S);
     HIP_OK(hipEventRecord(S.evc, S.stream));
     const dim3 blk(S.col_waves * 64);
-    P.col_split = column_split(S) ? 1 : 0;
     const size_t lds = column_lds(S.col_waves, P.col_split != 0) + (P.fold_lds ? (fold_bytes + 15) & ~(size_t)15 : 0);
     if (S.col_waves == 4) {
       if (P.fold_lds) hipLaunchKernelGGL((k_identify_columns_t<true, 4>), dim3((int)g), blk, lds, S.stream, P);

@@ -1,6 +1,7 @@
-"""The column pass on either side of the line between a wavefront per window and windows shared by a block:
-24 windows with just fewer and just more aligned bases than windows in each, one read, and none, against
-the oracle."""
+"""The column pass on either side of the line between a wavefront per window and windows shared by a block,
+which follows from the most alignments of a window and those of them that go one at a time: no read, one to
+four in one of 24 windows, and reads that cross a window's end, single runs and reads with a deletion, against the
+oracle."""
 import numpy as np
 import pytest
 
@@ -12,17 +13,18 @@ from parity_util import compare_gd
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [0, 1, 22, 23, 24, 25, 26])   # of 24 bases: 24 windows of 24 from 24 reads on
-def test_few_bases_a_window(n):
-    print("[gpu] column split:", n, "reads", flush=True)
+@pytest.mark.parametrize("n", [0, 1, 2, 3, 4, 26])
+@pytest.mark.parametrize("cigar", ["24M", "12M1D12M"])
+def test_few_alignments_a_window(n, cigar):
+    print("[gpu] column split:", n, "reads of", cigar, flush=True)
     rng = np.random.default_rng(n)
     ref = "".join(rng.choice(list("ACGT"), 24 * 64 - 1))
     reads = []
-    for pos in sorted(int(x) for x in rng.integers(700, 760, n)):
-        seq = list(ref[pos:pos + 24])
-        if pos <= 750 < pos + 24:
-            seq[750 - pos] = "ACGT"[("ACGT".index(ref[750]) + 1) % 4]
-        reads.append(dict(pos=pos, cigar="24M", seq="".join(seq), flag=16 * int(rng.integers(0, 2))))
+    for pos in sorted(int(x) for x in rng.integers(745, 766, n)):
+        seq = list(ref[pos:pos + 12] + ref[pos + (13 if "D" in cigar else 12):])[:24]
+        if pos <= 766 < pos + 12:
+            seq[766 - pos] = "ACGT"[("ACGT".index(ref[766]) + 1) % 4]
+        reads.append(dict(pos=pos, cigar=cigar, seq="".join(seq), flag=16 * int(rng.integers(0, 2))))
     s = BuiltSample(Built([("t0", ref)], reads))
     ea = B.api.make_error_count_args(s, quality_max=42)
     _, _, l_o, texts = O.error_count(ea)
