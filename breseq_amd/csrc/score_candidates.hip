@@ -60,17 +60,19 @@ constexpr double kDrop = 0.587566;       // kProfileLikelihoodLog10Drop (identif
 // How far a result of sums in any order may be from the reference's, which adds n terms one after the
 // other: every addition rounds by up to 2^-53 of the sum so far, and where the terms are alike, as those
 // of reads that agree, all in one direction.  The sums here are of fewer, larger terms.
-//   * A pass moves a frequency by up to n 2^-53 of itself, and what it moved stays in the passes after
-//     (EM does not enlarge it: in the frequencies' logarithms a step is the identity less a mean over
-//     the reads): passes * n * 2^-53, relative.
+//   * A pass moves a frequency by up to n 2^-53 of itself, and EM forgets most of what earlier passes moved (in
+//     the frequencies' logarithms a step is the identity less a mean over the reads).  Measured against correctly
+//     rounded sums over qualities of 2 to 40 and 30 to 20,000 reads: at most 0.2 n 2^-53 in up to 5 passes, 0.9
+//     in 20, 1.2 in 50.  Guard: (2 + passes / 8) n 2^-53, relative.
 //   * A log10 likelihood is off by up to n 2^-53 of its size, and by up to n^2 2^-53 because the
-//     frequencies add up to 1 only within n 2^-53; a score has two of them.  Guarded with twice that.
+//     frequencies add up to 1 only within n 2^-53; measured: at most 0.09 n 2^-53 (n + |log10 likelihood|).
+//     Guard: eleven times that, for a score with the likelihoods of both its fits.
 //   * A loop ends when no frequency moved by tol.  A step may be off by n 2^-53 for every pass up to it, and
-//     for those of the full fit that a profile starts from; one closer to tol is not decided here.
-// Measured against correctly rounded sums, most of three mixes of qualities: 5e-14 of a frequency and 7e-11 of
-// a likelihood at 3,000 reads (bounds 1e-12 and 5e-9), 3e-12 and 3e-7 at 200,000 (7e-11 and 2e-5).
+//     for those of the full fit that a profile starts from.  Where one is that close to tol, the full fit is done
+//     again in read order; the null fit and the profiles go on until a step is clearly below, and what the
+//     passes since can have added to the likelihood is added to the value's guard.
 // A decision or a printed digit closer to its boundary than its guard is made on exact sums.  Up to
-// some thousand reads the least guards of a launch hold (ImParams::guard_log, guard_rel).
+// some 6,000 reads the least guards of a launch hold (ImParams::guard_log, guard_rel).
 constexpr double kHalfUlp = 0x1p-53;
 constexpr double kSumSlack = 64.0;       // additions besides those of the reads: a term's own operations
 
@@ -82,6 +84,8 @@ struct ScoreShared {
   double lp_best;                  // log10 likelihood of the best pure genotype
   double guard_rel, guard_log;     // the candidate's guards; the score's own size comes on top
   double val[kTaskSlots];          // profile values of the round's tasks (without the lpmax sum)
+  double more[kTaskSlots];         // how far the reference's values may be below them for its last pass
+  double null_more, target_more, end_more[2];
   double pts[2][kTaskSlots];       // bisection midpoints of the round, per bound
   double vlo[2], vhi[2];           // profile values at the ends of each bound's interval
   double lo[2], hi[2];
@@ -596,19 +600,26 @@ struct TaskRowsGlobal {   // rows of the table, a read each: the variant comes f
 // of the reads' observations) or profile_log10_likelihood (identify_mutations.cpp:3094-3143: the
 // variant pinned to x, the others from the full fit rescaled), the same iterations as em_exact's with
 // sums in any order over the candidate's K rows (Src: TaskRowsLds or TaskRowsGlobal).  Returns log10 of the likelihood without
-// the sum of the reads' lpmax, which every such value of a candidate shares; NaN where the value cannot
-// stand for the reference's (a read with s_i = 0, or a step too close to tol).
+// the sum of the reads' lpmax, which every such value of a candidate shares, NaN where it cannot
+// stand for the reference's (a read with s_i = 0), and how far below it the reference's may be because it may
+// have ended some passes earlier: a step from f to g adds at most Sum_b (g_b - f_b) Sum_i r_i(b) / s_i to the likelihood's
+// natural logarithm, which is concave.
 //   nu: (n + kSumSlack) 2^-53; passes: those before the start, and one
 //   start[4]: the other alleles' starting frequencies; scale: 1 / n in the null fit, else 0
+struct TaskValue {
+  double ll, more;
+};
+
 template <int kSub, class Src>
-__device__ __noinline__ double em_tasks(const Src Sv, int Kv, double x, double start0, double start1, double start2,
+__device__ __noinline__ TaskValue em_tasks(const Src Sv, int Kv, double x, double start0, double start1, double start2,
                                         double start3, double scale_null, bool active, double tol, double nu, double passes) {
   const Src rows = Sv.uniform();
   const int K = uniform_i(Kv), sub = threadIdx.x & (kSub - 1);
   double f1 = start0, f2 = start1, f3 = start2, f4 = start3;
   const double rest = (1.0 - x) / 4.0;
   const bool null_fit = scale_null != 0.0;
-  bool run = active, bad = false;
+  bool run = active, bad = false, ended = false;   // ended: the reference's loop may have
+  double more = 0.0;
   for (int it = 1; __any(run); it++) {
     double a1 = 0.0, a2 = 0.0, a3 = 0.0, a4 = 0.0;
     // Four rows of a lane at a time, step by step: a row's chain (five products, a reciprocal, four
@@ -661,10 +672,11 @@ __device__ __noinline__ double em_tasks(const Src Sv, int Kv, double x, double s
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    a1 = f1 * sum_lanes<kSub>(a1);
-    a2 = f2 * sum_lanes<kSub>(a2);
-    a3 = f3 * sum_lanes<kSub>(a3);
-    a4 = f4 * sum_lanes<kSub>(a4);
+    const double q1 = sum_lanes<kSub>(a1), q2 = sum_lanes<kSub>(a2), q3 = sum_lanes<kSub>(a3), q4 = sum_lanes<kSub>(a4);
+    a1 = f1 * q1;
+    a2 = f2 * q2;
+    a3 = f3 * q3;
+    a4 = f4 * q4;
     const double others = (a1 + a2) + (a3 + a4);
     const double scale = null_fit ? scale_null : (1.0 - x) * recip_newton(others);
     const bool some = others > 0.0;
@@ -672,8 +684,14 @@ __device__ __noinline__ double em_tasks(const Src Sv, int Kv, double x, double s
     const double g3 = some ? scale * a3 : rest, g4 = some ? scale * a4 : rest;
     const double most = fmax(fmax(fabs(g1 - f1), fabs(g2 - f2)), fmax(fabs(g3 - f3), fabs(g4 - f4)));
     // (not-a-number sums fail the first test)
-    bad |= run & (!(others >= 0.0) | ((others > 0.0) & (others < 0x1p-500)) | ((it < 50) & (fabs(most - tol) < fmax(1e-6 * tol, ((double)it + passes) * nu))));
-    run &= (most >= tol) & (it < 50);
+    bad |= run & (!(others >= 0.0) | ((others > 0.0) & (others < 0x1p-500)));
+    const double room = fmax(1e-6 * tol, ((double)it + passes) * nu);
+    ended |= run & (most < tol + room);
+    run &= (most >= tol - room) & (it < 50);
+    if (__any(run & ended)) {
+      const double gain = ((g1 - f1) * q1 + (g2 - f2) * q2) + ((g3 - f3) * q3 + (g4 - f4) * q4);
+      if (run & ended) more += fmax(gain, 0.0);
+    }
     // a task that ends keeps this pass's frequencies: the likelihood is theirs
     f1 = run ? g1 : f1;
     f2 = run ? g2 : f2;
@@ -692,7 +710,7 @@ __device__ __noinline__ double em_tasks(const Src Sv, int Kv, double x, double s
   // one lane that saw a read it cannot stand for spoils its task
   const unsigned long long m = __ballot(bad);
   const int base = (threadIdx.x & 63) & ~(kSub - 1);
-  return ((m >> base) & ((1ull << kSub) - 1ull)) ? __longlong_as_double(0x7ff8000000000000LL) : ll;
+  return {((m >> base) & ((1ull << kSub) - 1ull)) ? __longlong_as_double(0x7ff8000000000000LL) : ll, 0.5 * more};
 }
 
 // Where the profile likelihood is predicted to cross the target inside the interval of bound
@@ -1359,8 +1377,8 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
         SS.depth[0] = SS.depth[1] = 0;
         SS.out[0] = 0.0;
         SS.out[1] = 1.0;
-        if (level == 0) SS.guard_rel = fmax(P.guard_rel, SS.fit[5] * nu);
-        SS.guard_log = fmax(P.guard_log, 4.0 * nu * ((double)n + fabs(SS.lp_best)));
+        if (level == 0) SS.guard_rel = fmax(P.guard_rel, (2.0 + 0.125 * SS.fit[5]) * nu);
+        SS.guard_log = fmax(P.guard_log, nu * ((double)n + fabs(SS.lp_best)));
         if (!in_order && n > 0 && SS.unsure == 0 &&
             !fit_is_sure((LdsDouble*)SS.full_f, (uint32_t)n, P.places, SS.guard_rel))
           SS.unsure = 1;
@@ -1487,11 +1505,11 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
                 return both ? em_tasks<4, Src>(src, K, x, st[0], st[1], st[2], st[3], sc, active, tol, nu, passes)
                             : em_tasks<8, Src>(src, K, x, st[0], st[1], st[2], st[3], sc, active, tol, nu, passes);
               };
-              const double val = kind == kRowsLds ? tasks_over(TaskRowsLds{pr})
-                                                  : tasks_over(TaskRowsGlobal<kLG>{list, P.tab_r, variant});
+              const TaskValue val = kind == kRowsLds ? tasks_over(TaskRowsLds{pr})
+                                                     : tasks_over(TaskRowsGlobal<kLG>{list, P.tab_r, variant});
               if (first && active) {
-                if (null_task) SS.null_ll = val;
-                else SS.val[slot_i] = val;
+                (null_task ? SS.null_ll : SS.val[slot_i]) = val.ll;
+                (null_task ? SS.null_more : SS.more[slot_i]) = val.more;
               }
             }
           }
@@ -1523,6 +1541,8 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
             B.active = SS.active[side];
           }
           const double target = (round == 0) ? SS.val[0] - kDrop : SS.target;
+          const double target_more = (round == 0) ? SS.more[0] : SS.target_more;
+          const double end_more = (round == 0) ? SS.more[side ? 2 : 1] : SS.end_more[side];
           const int n_tree = SS.n_tree, slot0 = SS.slot0[side];
           if (exact == 1 + side) {
             // the exact comparison decides this side's end of the range, or its midpoint.  (The values
@@ -1533,7 +1553,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
             const int depth = exact ? 0 : SS.depth[side];
             if (B.active == 2) {
               const double v = side ? B.vhi : B.vlo;
-              close = !(fabs(v - target) > guard);
+              close = !(fabs(v - target) > guard + end_more + target_more);
               if (!close) B.step(side, v >= target, 0.0, v, tol, fh);
             }
             // down the evaluated levels: every level is one sequential bisection step (the interval
@@ -1546,7 +1566,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
               if (k >= depth) break;
               const double m = 0.5 * (B.lo + B.hi), at = SS.pts[side][k], v = SS.val[slot0 + k];
               if (m != at) break;
-              close = !(fabs(v - target) > guard);
+              close = !(fabs(v - target) > guard + SS.more[slot0 + k] + target_more);
               if (close) break;
               const bool ge = v >= target;
               B.step(side, ge, m, v, tol, fh);
@@ -1566,12 +1586,14 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
             SS.out[side] = B.out;
             SS.iter[side] = B.iter;
             SS.active[side] = B.active;
+            SS.end_more[side] = end_more;
             SS.exact_x[side] = (B.active == 2) ? (side ? 1.0 : 0.0) : 0.5 * (B.lo + B.hi);
           }
           const unsigned long long u = __ballot(walker && close), open = __ballot(walker && B.active != 0);
           const double out0 = readlane_d(B.out, 0), out1 = readlane_d(B.out, 32);
           if (lane == 0) {
             SS.target = target;
+            SS.target_more = target_more;
             if (exact) SS.exact_have = 1;
             SS.exact = (in_order && u) ? ((u & 1ull) ? 1 : 2) : 0;
             // emitted: a consensus call, or a presence score at the cutoff
@@ -1581,7 +1603,7 @@ __global__ void __launch_bounds__(kSW * 64) __attribute__((amdgpu_waves_per_eu(4
             SS.done = (!emitted || !have_v || !open) ? 1 : 0;
             int unsure = 0;
             if (level < 2 && have_v) {
-              const double err = SS.guard_log + 4.0 * nu * fabs(score);
+              const double err = SS.guard_log + nu * fabs(score) + SS.null_more;
               if (!(fabs(score - P.polymorphism_cutoff) > err) || (emitted && !prints_surely_f1(score, err))) unsure = 2;
             }
             if (level == 0 && have_v && emitted && unsure == 0) {
